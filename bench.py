@@ -633,10 +633,13 @@ def main():
         w, c = (int(x) for x in args.two_step.split(":"))
         ctx.set_tile_width(dtype, w)
         ctx.set_two_step_lds(c)
-    tile_width = ctx.tile_width(dtype)
+    steps_per_launch, tile_width = abi.diagonal_form(mat, blk, M)
     two_step, two_step_wg = ctx.two_step_lds(dtype)
+    chained = steps_per_launch > 2 or (steps_per_launch == 2 and not two_step)
+    two_step = two_step and not chained
     log("autotuned step kernel variant: %d (column tiles of %d vectors)%s"
-        % (variant, tile_width, ", LDS two-step form on %d workgroups per CU" % two_step_wg if two_step else ""))
+        % (variant, tile_width, ", chained form, %d steps per launch" % steps_per_launch if chained else
+           ", LDS two-step form on %d workgroups per CU" % two_step_wg if two_step else ""))
 
     for _ in range(args.warmup):
         abi.moments_diagonal_run(mat, blk, M)
@@ -655,20 +658,21 @@ def main():
     ms_per_step = wall * 1000 / args.steps
     value = nnz * M * R / (wall / args.steps) / 1e9
 
-    # fused step launches per moment computation: one per two moments and column tile (one per
-    # four moments in the two-step form, each reading r_k-1 and r_k and writing r_k+1 and r_k+2)
+    # launches per moment computation and column tile: one per two moments, one per four in the
+    # two-step form, one per 2 K in the chained form of K steps per launch
     widths = launch_widths(R, tile_width)
     steps_per_run = M // 2
-    steps_per_launch = 2 if two_step else 1
-    step_ms = gpu_ms / (args.steps * steps_per_run // steps_per_launch * len(widths))      # one launch
+    step_ms = gpu_ms / (args.steps * -(-steps_per_run // steps_per_launch) * len(widths))      # one launch
     # the variants 45..59 and the two-step form read the matrix's value-table form (8-bit codes of
     # the off-diagonal entries, the diagonal dense) when it has one: its bytes replace
     # nnz (s + 4) + 4 (N + 1) in a launch's count
-    coded = mat.coded_bytes() if (variant >= 45 or two_step) else 0
+    coded = mat.coded_bytes() if (variant >= 45 or two_step or chained) else 0
     matrix_bytes = coded if coded else nnz * (s + 4) + 4 * (n + 1)
     # algorithmic bytes of the steps one launch does (a two-step launch moves fewer: it reads and
     # writes 4 vector blocks instead of 6, which the counted traffic shows)
     bytes_per_launch = sum(steps_per_launch * (matrix_bytes + 3 * n * w * s) for w in widths) / len(widths)
+    if chained:  # K steps on chip: two vector blocks read and two written, the matrix once
+        bytes_per_launch = sum(matrix_bytes + 4 * n * w * s for w in widths) / len(widths)
     achieved = bytes_per_launch / (step_ms / 1000)
     # the same step over all R vectors as one pass (the matrix read once): the algorithmic bytes of
     # the whole step over the time of its launches
@@ -682,20 +686,22 @@ def main():
 
     traffic_key = "%dx%d %s v%d launch%d %s%s %s%s" % (args.cells[0], args.cells[1], dtype.name, R, max(widths),
                                                        args.format, " coded" if coded else "", args.order,
-                                                       " two-step" if two_step else "")
+                                                       " two-step" if two_step else
+                                                       " chain%d" % steps_per_launch if chained else "")
     extra = {"starter_draw_s": t_draw,
              "one_pass_equivalent": {"ms_per_step": pass_ms, "achieved_GBps": pass_gbps,
                                      "frac": pass_gbps * 1e9 / HBM_PEAK, "launch_widths": widths}}
     cg, rg, tg = ctx.stream_probe(1 << 31)
-    step_traffic_gbps = (counted_traffic(traffic_key) or float("nan")) / (step_ms / 1000) / 1e9
+    counted = counted_traffic(traffic_key)
+    step_traffic_gbps = counted / (step_ms / 1000) / 1e9 if counted else None
     extra["stream_probe"] = {"copy_GBps": cg, "read_GBps": rg, "triad_GBps": tg,
-                             "step_traffic_over_copy": step_traffic_gbps / cg,
-                             "step_traffic_over_triad": step_traffic_gbps / tg}
-    log("stream probe: copy %.0f GB/s, read %.0f GB/s, triad (b = a + b) %.0f GB/s; step traffic at %.2f of the triad"
-        % (cg, rg, tg, step_traffic_gbps / tg))
-    if two_step:
+                             "step_traffic_over_copy": step_traffic_gbps / cg if counted else None,
+                             "step_traffic_over_triad": step_traffic_gbps / tg if counted else None}
+    log("stream probe: copy %.0f GB/s, read %.0f GB/s, triad (b = a + b) %.0f GB/s%s"
+        % (cg, rg, tg, "; step traffic at %.2f of the triad" % (step_traffic_gbps / tg) if counted else ""))
+    if two_step or chained:
         # the same computation with single steps (the default column tiles, the autotuned single-step
-        # variant), timed in the same run for comparison
+        # variant; setting the width turns the chained form off), timed in the same run for comparison
         ctx.set_two_step(dtype, 0)
         ctx.set_tile_width(dtype, 16 if dtype == np.float64 else 64)
         abi.moments_diagonal_run(mat, blk, M)
@@ -704,27 +710,27 @@ def main():
         abi.moments_diagonal_run(mat, blk, M)
         ms_single = ctx.timer_stop()
         extra["single_steps"] = {"ms_per_step": ms_single / steps_per_run, "value": nnz * M * R / (ms_single / 1000) / 1e9,
-                                 "two_step_speedup": ms_single / (gpu_ms / args.steps)}
-        log("single steps on the same box: %.4f ms per step (the two-step form %.2fx faster)"
+                                 "speedup_over_single_steps": ms_single / (gpu_ms / args.steps)}
+        log("single steps on the same box: %.4f ms per step (this form %.2fx faster)"
             % (ms_single / steps_per_run, ms_single / (gpu_ms / args.steps)))
     if not args.no_plain:
-        # the plain single-vector path (one vector, SELL-64 kernel) on the same matrix, timed over
+        # the plain single-vector path (one vector, its default form) on the same matrix, timed over
         # 512 moments and reported in the same metric
-        mat1 = ctx.mat(h2, fmt=1)
-        blk1 = ctx.block(r0[:1])
+        ctx1 = abi.Ctx(0)
+        mat1 = ctx1.mat(h2, fmt=1)
+        blk1 = ctx1.block(r0[:1])
         abi.moments_diagonal_run(mat1, blk1, 512)
-        ctx.synchronize()
-        ctx.timer_start()
+        ctx1.synchronize()
+        ctx1.timer_start()
         abi.moments_diagonal_run(mat1, blk1, 512)
-        ms1 = ctx.timer_stop()
+        ms1 = ctx1.timer_stop()
         v1 = nnz * 512 * 1 / (ms1 / 1000) / 1e9
         b1 = step_bytes(n, nnz, 1, s)
         extra["plain_single_vector"] = {"value": v1, "unit": "GNNZ*moments/s",
                                         "step_ms": ms1 / 256, "achieved_GBps": b1 / (ms1 / 256 / 1000) / 1e9,
                                         "block_over_plain": value / v1}
         log("plain: %.1f GNNZ*moments/s; block/plain = %.2f" % (v1, value / v1))
-        blk1.close()
-        mat1.close()
+        ctx1.close()
 
     if not args.no_fp32 and dtype == np.float64:
         extra["fp32_variant"] = fp32_variant(args.cells, M, R, args.format, args.order)

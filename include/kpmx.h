@@ -117,8 +117,22 @@ int kpmx_block_destroy(kpmx_block* b);
 /* DiagonalMoments / BatchDiagonalMoments: mu_n = <r|T_n(H~)|r> for every vector of the block,
  * two moments per Chebyshev step (cppcore/include/kpm/calc_moments.hpp:35-89,
  * cppcore/src/kpm/default/collectors.cpp:5-34).  num_moments must be even.
- * mu: host, num_vectors x num_moments, scalar type of h2. */
+ * mu: host, num_vectors x num_moments, scalar type of h2.
+ * On SELL matrices the recurrence runs in its chained form where that is expected to be faster:
+ * several steps per launch on tiles of consecutive rows, each with the rows within that many hops
+ * (its halo), the vectors held in LDS and registers; tile height and steps per launch come from the
+ * halos of sampled tiles.  The plan of a (matrix, block width) is built on the device by the first
+ * call and freed with the matrix.  Row orders with large halos, light-cone limits and blocks whose
+ * step variant, tile width or two-step form is pinned keep the forms below; all forms agree to
+ * rounding. */
 int kpmx_moments_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, void* mu);
+
+/* The form kpmx_moments_diagonal takes for these arguments (no counterpart in the reference; its
+ * plans are built if they are not there): steps_per_launch 1 (single steps), 2 (a two-step form) or
+ * more (the chained form's launches; the last of a run may do fewer), and columns, the vectors of
+ * one launch of the block's widest starter tile. */
+int kpmx_diagonal_form(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, int* steps_per_launch,
+                       int* columns);
 
 /* Autotuner (no counterpart in the reference, whose CPU kernels have one fixed shape): time the
  * variants of the fused diagonal step kernel (three tile shapes, each on the full resident grid,
@@ -134,10 +148,13 @@ int kpmx_moments_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_
  * diagonal as a dense vector, built at upload when the off-diagonal entries take that few
  * distinct values, for other matrices run as 2).  On fp64 SELL matrices it then also times the
  * LDS two-step form (see kpmx_ctx_set_autotune_two_step) and keeps it, with its column-tile
- * width, when it is faster per vector. */
+ * width, when it is faster per vector.  Last it times the chained form: the context keeps it for the
+ * scalar type while it is the fastest of all, otherwise the chosen variant (or two-step form) runs. */
 int kpmx_autotune_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int* variant);
 /* Pin the diagonal step variant (as numbered above) for one scalar type and vector width on the
- * context, e.g. a choice an earlier autotuning run reported (no counterpart in the reference). */
+ * context, e.g. a choice an earlier autotuning run reported (no counterpart in the reference).
+ * Diagonal recurrences of the scalar type then run single (or two-step) launches, not the chained
+ * form. */
 int kpmx_ctx_set_step_variant(kpmx_ctx* ctx, int scalar, int vector_width, int variant);
 
 /* Pin the variant of the adjoint step kernel (numbered as the diagonal step variants; no
@@ -150,7 +167,8 @@ int kpmx_ctx_set_adjoint_variant(kpmx_ctx* ctx, int variant);
  * sub-tiles of this many columns (each copied out of the tile first); narrower tiles move fewer
  * bytes per gathered row, so one XCD's L2 holds the rows of a wider band, at the price of one
  * matrix read per sub-tile and step.  The moments are the same up to rounding.  Defaults: 16 for
- * fp64, 64 for the others.  get: the current width. */
+ * fp64, 64 for the others; setting a width turns the chained form off for the scalar type.  get: the
+ * current width. */
 int kpmx_ctx_set_tile_width(kpmx_ctx* ctx, int scalar, int width);
 int kpmx_ctx_get_tile_width(kpmx_ctx* ctx, int scalar, int* width);
 
@@ -208,10 +226,10 @@ int kpmx_moments_diagonal_fetch(const kpmx_mat* h2, const kpmx_block* r0, int64_
  * the block is run as column sub-tiles, see kpmx_ctx_set_tile_width), plus (num_moments / 2) x
  * 4 x (vector width) doubles of sums, plus num_vectors x num_moments scalars, plus one step's
  * partial sums, must fit, otherwise KPMX_EINVAL with the sizes in the message.  No device memory
- * is allocated or freed (h2 and r0 are uploaded beforehand).  It always runs single steps (the
- * two-step forms need workspaces of their own), so where kpmx_moments_diagonal runs two steps per
- * launch the two results agree to rounding rather than bit for bit.  Calls that overlap on one
- * GPU share the array and race. */
+ * is allocated or freed (h2 and r0 are uploaded beforehand).  It runs the chained form when an earlier
+ * kpmx_moments_diagonal has left the matrix its plan and the four work vectors of that form fit, else
+ * single steps; where the two calls run different forms their results agree to rounding rather than
+ * bit for bit.  Calls that overlap on one GPU share the array and race. */
 int kpmx_moments_diagonal_noalloc(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, void* mu);
 
 /* GenericMoments: mu_n = <beta| op T_n(H~) |r0> for the first vector of r0

@@ -220,6 +220,14 @@ def moments_diagonal_noalloc(mat, block, num_moments):
     return out
 
 
+def diagonal_form(mat, block, num_moments):
+    """(steps per launch, vectors per launch) of the form the diagonal recurrence takes
+    (kpmx_diagonal_form)."""
+    k, w = ctypes.c_int(), ctypes.c_int()
+    _check(lib().kpmx_diagonal_form(mat.h, block.h, ctypes.c_int64(num_moments), ctypes.byref(k), ctypes.byref(w)))
+    return k.value, w.value
+
+
 def autotune_diagonal(mat, block):
     """Pick the fastest tile shape of the diagonal step kernel for this matrix and block."""
     v = ctypes.c_int()

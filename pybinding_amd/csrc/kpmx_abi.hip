@@ -20,6 +20,7 @@
 
 #include "../../include/kpmx.h"
 #include "kpmx_internal.hpp"
+#include "kpmx_chain.hpp"
 
 using namespace kpmx;
 
@@ -157,6 +158,11 @@ struct kpmx_ctx {
     int two_step_lds[4] = {0, 0, 0, 0};        // the LDS form (k_step2_lds) of the two-step recurrence
     bool autotune_two_step = true;             // kpmx_autotune_diagonal may choose the LDS two-step form
     bool two_step_auto[4] = {false, false, false, false};  // the two-step settings are the autotuner's
+    // the chained form of the diagonal recurrence (kpmx_chain_step.hpp) per scalar type: the default,
+    // off once the caller pins a step variant or a tile width, or while the autotuner has found another
+    // form faster; a two-step form that the caller has asked for goes before it where it applies
+    enum { CHAIN_ON, CHAIN_PINNED_OFF, CHAIN_TUNED_OFF };
+    int chain[4] = {CHAIN_ON, CHAIN_ON, CHAIN_ON, CHAIN_ON};
     Workspace work3, work4;  // the third and fourth vector of the two-step recurrence
     int graph_policy = KPMX_GRAPH_NEVER;
     int adjoint_variant = -1;  // adjoint step variant (kpmx_ctx_set_adjoint_variant); -1: the default
@@ -189,6 +195,15 @@ struct LdsHalo {
             dev_free(p);
         *this = LdsHalo{};
     }
+};
+
+// A chained-recurrence plan of one matrix for one column width, with the device memory it owns
+// (one allocation; null data: the matrix is better off with other forms).
+struct ChainHolder {
+    int cols = 0;
+    ChainPlan plan;
+    char* data = nullptr;
+    ~ChainHolder() { dev_free(data); }
 };
 
 struct kpmx_mat {
@@ -231,6 +246,7 @@ struct kpmx_mat {
     void* cdiag = nullptr;
     void* ctable = nullptr;
     int cmax_width = 0, ctable_size = 0;
+    mutable std::vector<std::unique_ptr<ChainHolder>> chains;  // by column width, built on first use
     ~kpmx_mat() {
         for (void* p : {(void*)cslice_ptr, (void*)cslice_width, (void*)cindices, (void*)ccodes, cdiag, ctable}) dev_free(p);
         dev_free(d_h1_ptr);
@@ -263,6 +279,7 @@ struct kpmx_block {
     std::vector<void*> sums;
     int64_t sums_moments = 0;
     int sums_cap = 0;  // column tile cap the sums were run with
+    bool sums_chain = false;  // the sums were run by the chained form (whole starter tiles)
     // captured diagonal recurrence and the launch state it was captured with
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -912,6 +929,289 @@ void run_recurrence2(const kpmx_mat* h2, const Tile& t, int64_t steps, double* s
     }
 }
 
+// ------------------------------------------------------------------------ chained recurrence
+ChainMatrix chain_matrix(const kpmx_mat* h2) {
+    ChainMatrix m;
+    m.scalar = h2->scalar;
+    m.n = h2->rows;
+    if (h2->ccodes) {
+        m.max_width = h2->cmax_width;
+        m.slice_ptr = h2->cslice_ptr;
+        m.slice_width = h2->cslice_width;
+        m.indices = h2->cindices;
+        m.codes = h2->ccodes;
+        m.diag = h2->cdiag;
+        m.table = h2->ctable;
+        m.table_size = h2->ctable_size;
+    } else {
+        m.max_width = h2->max_width;
+        m.slice_ptr = h2->slice_ptr;
+        m.slice_width = h2->slice_width;
+        m.indices = h2->sell_indices;
+        m.vals = h2->sell_vals;
+    }
+    return m;
+}
+
+// Estimated microseconds per step of launches of `steps` steps on tiles of `rows` rows whose local
+// rows number e[j] up to distance j.  Fitted to measured launches: a CU holds two workgroups; their
+// loads and stores (about 21 KB a microsecond and CU from HBM, 32 KB while the vectors stay in
+// the Infinity Cache) overlap most of their steps, an item (16 bytes of a row) costs 0.4 ns alone and
+// 0.25 ns beside the other workgroup for three entries, a step 0.5 us of barriers and sums, a launch
+// 3 us.
+double chain_cost(const ChainMatrix& m, double rows, const double* e, int steps, double row_bytes, int num_cu) {
+    const double tiles = std::ceil((double)m.n / rows), wgs = tiles > num_cu ? 2 : 1;
+    double rounds = tiles / (wgs * num_cu);
+    rounds = rounds < 8 ? std::ceil(rounds) : rounds + 0.5;
+    const double sb = (double)scalar_bytes(m.scalar), width = m.max_width;
+    const double entry = 2 + (m.form() == CHAIN_STD ? sb : m.form() == CHAIN_TABLE ? 1 : 0);
+    const double bytes = (e[steps] + e[steps - 1] + 2 * rows) * row_bytes + e[steps - 1] * (entry * width + sb);
+    const double rate = 4 * (double)m.n * row_bytes < 192e6 ? 32e3 : 21e3;
+    double row_steps = 0;
+    for (int j = 1; j <= steps; ++j) row_steps += e[steps - j];
+    const double form = m.form() == CHAIN_UNIFORM ? 1.0 : m.form() == CHAIN_TABLE ? 1.3 : 2.0;
+    const double item = (wgs > 1 ? 0.25e-3 : 0.4e-3) * form * (width + 3) / 6;
+    const double compute = wgs * (row_steps * std::max(1.0, row_bytes / 16) * item + 0.5 * steps);
+    const double memory = wgs * bytes / rate;
+    const double round = std::max(compute, memory) + 0.3 * std::min(compute, memory);
+    return (3.0 + rounds * round) / steps;
+}
+
+// The plan of a matrix for `cols` columns: the tile height and steps per launch with the least
+// estimated time per step over a few heights whose halos are measured on sampled tiles.
+const ChainPlan* build_chain(const kpmx_mat* h2, int cols, ChainHolder& H) {
+    kpmx_ctx* ctx = h2->ctx;
+    const int64_t n = h2->rows;
+    const ChainMatrix m = chain_matrix(h2);
+    const int cap = chain_row_capacity(m, cols);
+    if (cap <= 0 || n < 64) return nullptr;
+    const size_t sb = scalar_bytes(h2->scalar);
+    const double row_bytes = (double)cols * sb;
+    // heights: as many tiles as CUs and small multiples of twice that (no CU idles in the last
+    // round), and fractions of what a workgroup holds
+    std::vector<int> heights;
+    auto add = [&](double h) {
+        const int r = (int)std::max<int64_t>(32, (std::min<int64_t>(n, (int64_t)std::ceil(h)) + 7) / 8 * 8);
+        if (r <= 0.85 * cap && (int)heights.size() < CHAIN_CANDIDATES && std::find(heights.begin(), heights.end(), r) == heights.end())
+            heights.push_back(r);
+    };
+    const double per_round = 2.0 * ctx->num_cu;
+    const double fewest = std::ceil((double)n / (0.85 * cap * per_round));  // rounds of the tallest tiles
+    add((double)n / ctx->num_cu);
+    add(2.0 * n / ctx->num_cu);
+    add((double)n / (fewest * per_round));
+    add((double)n / ((fewest + 1) * per_round));
+    add((double)n / ((fewest + 2) * per_round));
+    add(0.6 * cap);
+    add(0.45 * cap);
+    add(0.3 * cap);
+    if (heights.empty()) return nullptr;
+    constexpr int ST = CHAIN_MAX_STEPS + 1;
+    std::vector<int32_t> ring(heights.size() * CHAIN_SAMPLES * ST);
+    int32_t* d = static_cast<int32_t*>(ctx->aux2.get(ring.size() * sizeof(int32_t)));
+    KPMX_REQUIRE(chain_sample(m, heights.data(), (int)heights.size(), cap, d, ctx->stream) == 0, "no LDS for a chain plan");
+    KPMX_HIP(hipGetLastError());
+    KPMX_HIP(hipMemcpyAsync(ring.data(), d, ring.size() * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+    KPMX_HIP(hipStreamSynchronize(ctx->stream));
+    double best = 1e300;
+    int rows = 0, steps = 0;
+    for (size_t c = 0; c < heights.size(); ++c) {
+        double e[ST] = {};
+        for (int k = 0; k < ST; ++k) {
+            int fit = 0;
+            for (int q = 0; q < CHAIN_SAMPLES; ++q) {
+                const int32_t v = ring[(c * CHAIN_SAMPLES + q) * ST + k];
+                if (v < 0 || v > cap) continue;
+                ++fit;
+                e[k] += v;
+            }
+            if (fit < 0.85 * CHAIN_SAMPLES) break;  // the few tiles that do not fit are halved
+            e[k] /= fit;
+            const double t = k < 2 ? best : chain_cost(m, heights[c], e, k, row_bytes, ctx->num_cu);
+            if (t < best) {
+                best = t;
+                rows = heights[c];
+                steps = k;
+            }
+        }
+    }
+    // single steps: about 5.6 TB/s of three passes over the columns and their share of the matrix, no
+    // less than a launch; a third of that on long rows
+    const double sweep = (3.0 * n * row_bytes + (double)h2->nnz * (sb + 4) * cols / std::max(cols, ctx->tile_cap[h2->scalar])) / 5.6e6;
+    if (!rows || best > std::max(5.5, sweep * (m.max_width > 8 ? 3 : 1))) return nullptr;
+    // halos of every tile into scratch; tiles whose local rows exceed the capacity are halved
+    ChainPlan P;
+    P.tile_rows = rows;
+    P.ext_stride = std::min(CHAIN_MAX_HALO, cap - rows);
+    std::vector<int32_t> begin;
+    for (int64_t r = 0; r < n; r += rows) begin.push_back((int32_t)r);
+    begin.push_back((int32_t)n);
+    auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
+    std::vector<int> most(ST, 0);
+    for (int pass = 0;; ++pass) {
+        P.ntiles = (int64_t)begin.size() - 1;
+        const size_t ring_size = (size_t)P.ntiles * ST;
+        char* w = static_cast<char*>(ctx->aux2.get(pad(begin.size() * sizeof(int32_t)) + pad(ring_size * sizeof(int32_t)) +
+                                                   (size_t)P.ntiles * P.ext_stride * sizeof(int32_t)));
+        P.tile_begin = reinterpret_cast<int32_t*>(w);
+        P.ring = reinterpret_cast<int32_t*>(w + pad(begin.size() * sizeof(int32_t)));
+        P.ext = reinterpret_cast<int32_t*>(w + pad(begin.size() * sizeof(int32_t)) + pad(ring_size * sizeof(int32_t)));
+        KPMX_HIP(hipMemcpyAsync(P.tile_begin, begin.data(), begin.size() * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+        KPMX_REQUIRE(chain_rings(m, P, steps, ctx->stream) == 0, "no LDS for a chain plan");
+        KPMX_HIP(hipGetLastError());
+        ring.resize(ring_size);
+        KPMX_HIP(hipMemcpyAsync(ring.data(), P.ring, ring_size * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+        KPMX_HIP(hipStreamSynchronize(ctx->stream));
+        std::vector<int32_t> split;
+        std::fill(most.begin(), most.end(), 0);
+        for (int64_t t = 0; t < P.ntiles; ++t) {
+            split.push_back(begin[t]);
+            for (int j = 0; j <= steps; ++j) {
+                const int32_t v = ring[t * ST + j];
+                most[j] = v < 0 || v > cap || most[j] < 0 ? -1 : std::max(most[j], v);
+            }
+            const int32_t last = ring[t * ST + steps], own = begin[t + 1] - begin[t];
+            if ((last < 0 || last > cap) && own >= 32) split.push_back(begin[t] + own / 2);
+        }
+        split.push_back((int32_t)n);
+        if (pass == 4 || split.size() == begin.size() || (double)split.size() > 1.4 * begin.size()) break;
+        begin.swap(split);
+    }
+    while (steps > 1 && most[steps] < 0) --steps;
+    if (steps < 2) return nullptr;
+    int halo = 0;
+    for (int64_t t = 0; t < P.ntiles; ++t) halo = std::max(halo, ring[t * ST + steps] - ring[t * ST]);
+    const size_t ring_bytes = (size_t)P.ntiles * ST * sizeof(int32_t), begin_bytes = (size_t)(P.ntiles + 1) * sizeof(int32_t);
+    P.steps = steps;
+    P.width = m.max_width;
+    P.groups = std::max(1, (m.max_width + 3) / 4);
+    P.rows_x = most[steps];
+    const int row_pad = chain_row_pad(m, cols);
+    P.rows_y = (most[steps - 1] + row_pad - 1) / row_pad * row_pad;
+    P.row_items = chain_row_items(h2->scalar, cols);
+    const int form = m.form();
+    const int64_t src_stride = P.ext_stride;
+    const size_t cells = (size_t)P.ntiles * P.rows_y;
+    const size_t parts[7] = {pad(begin_bytes),
+                             pad(ring_bytes),
+                             pad((size_t)P.ntiles * halo * sizeof(int32_t)),
+                             pad(cells * P.groups * sizeof(ushort4)),
+                             form == CHAIN_TABLE ? pad(cells * P.groups * sizeof(uint32_t)) : 0,
+                             form == CHAIN_STD ? pad(cells * P.groups * 4 * sb) : 0,
+                             form != CHAIN_STD ? pad(cells * sb) : 0};
+    size_t total = 0;
+    for (size_t b : parts) total += b;
+    char* data = static_cast<char*>(dev_alloc(total));
+    H.data = data;
+    char* at[7];
+    for (int i = 0; i < 7; ++i) {
+        at[i] = data;
+        data += parts[i];
+    }
+    const ChainPlan scratch = P;
+    P.tile_begin = reinterpret_cast<int32_t*>(at[0]);
+    P.ring = reinterpret_cast<int32_t*>(at[1]);
+    P.ext = reinterpret_cast<int32_t*>(at[2]);
+    P.ext_stride = halo;
+    P.lidx = reinterpret_cast<ushort4*>(at[3]);
+    P.codes = reinterpret_cast<uint32_t*>(at[4]);
+    P.vals = at[5];
+    P.diag = at[6];
+    KPMX_HIP(hipMemcpyAsync(P.tile_begin, scratch.tile_begin, begin_bytes, hipMemcpyDeviceToDevice, ctx->stream));
+    KPMX_HIP(hipMemcpyAsync(P.ring, scratch.ring, ring_bytes, hipMemcpyDeviceToDevice, ctx->stream));
+    if (halo)
+        KPMX_HIP(hipMemcpy2DAsync(P.ext, halo * sizeof(int32_t), scratch.ext, src_stride * sizeof(int32_t),
+                                  halo * sizeof(int32_t), P.ntiles, hipMemcpyDeviceToDevice, ctx->stream));
+    KPMX_REQUIRE(chain_entries(m, P, ctx->stream) == 0, "no LDS for a chain plan");
+    KPMX_HIP(hipGetLastError());
+    H.plan = P;
+    return &H.plan;
+}
+
+// The plan for `cols` columns, built on first use (unless `existing` asks for one that is there
+// already); null where there is none.
+const ChainPlan* chain_plan(const kpmx_mat* h2, int cols, bool existing = false) {
+    for (auto& c : h2->chains)
+        if (c->cols == cols) return c->data ? &c->plan : nullptr;
+    if (existing) return nullptr;
+    auto H = std::make_unique<ChainHolder>();
+    H->cols = cols;
+    try {
+        build_chain(h2, cols, *H);
+    } catch (const Error& e) {
+        if (e.code != KPMX_ENOMEM) throw;
+        dev_free(H->data);
+        H->data = nullptr;  // no memory for the plan: single steps
+    }
+    h2->chains.push_back(std::move(H));
+    return h2->chains.back()->data ? &h2->chains.back()->plan : nullptr;
+}
+
+int chain_cols(const kpmx_mat* h2, const Tile& t) { return std::min(t.vw, chain_max_cols(h2->scalar)); }
+
+constexpr size_t CHAIN_PARTIALS = (size_t)64 << 20;  // partial sums kept before one reduction
+
+// Two pairs of work vectors and the partial sums of one reduction.
+struct ChainBuffers {
+    void* w[2][2];
+    double* partials;
+    size_t partials_bytes;
+};
+size_t chain_step_bytes(const kpmx_mat* h2, const ChainPlan& P, int cols) {
+    return (size_t)P.ntiles * chain_partial_width(h2->scalar, cols) * sizeof(double);
+}
+
+ChainBuffers size_chain(const kpmx_mat* h2, const Tile& t, int64_t steps) {
+    kpmx_ctx* ctx = h2->ctx;
+    const int cols = chain_cols(h2, t);
+    const ChainPlan& P = *chain_plan(h2, cols);
+    const size_t blk = (size_t)h2->rows * cols * scalar_bytes(h2->scalar);
+    const size_t bytes = std::min(std::max(CHAIN_PARTIALS, P.steps * chain_step_bytes(h2, P, cols)),
+                                  (size_t)(steps + P.steps) * chain_step_bytes(h2, P, cols));
+    return {{{ctx->work0.get(blk), ctx->work1.get(blk)}, {ctx->work3.get(blk), ctx->work4.get(blk)}},
+            static_cast<double*>(ctx->partials.get(bytes)),
+            bytes};
+}
+
+// The diagonal recurrence of a starter tile in the chained form, in column groups of at most
+// chain_max_cols vectors; the first launch of a group reads its columns in place.  Two pairs of work
+// vectors take turns: a launch reads (r_{k-1}, r_k) and writes (r_{k+K-1}, r_{k+K}).
+void run_chain(const kpmx_mat* h2, const Tile& t, int64_t steps, double* sums, const ChainBuffers& B) {
+    kpmx_ctx* ctx = h2->ctx;
+    const int cols = chain_cols(h2, t);
+    const ChainPlan& P = *chain_plan(h2, cols);
+    const size_t sb = scalar_bytes(h2->scalar), step_bytes = chain_step_bytes(h2, P, cols);
+    const int64_t per_step = (int64_t)(step_bytes / sizeof(double));
+    const int64_t chunk = std::max<int64_t>(1, (int64_t)(B.partials_bytes / step_bytes) / P.steps) * P.steps;
+    ChainLaunch L;
+    L.m = chain_matrix(h2);
+    L.plan = &P;
+    L.cols = cols;
+    for (int64_t c0 = 0; c0 < t.cols; c0 += cols) {
+        int64_t chunk_start = 0;
+        int turn = 0;
+        for (int64_t k = 0; k < steps; k += L.steps, turn ^= 1) {
+            L.steps = (int)std::min<int64_t>(P.steps, steps - k);
+            L.first = k == 0;
+            L.x = k == 0 ? static_cast<const char*>(t.data) + c0 * sb : B.w[turn ^ 1][1];
+            L.ldx = k == 0 ? t.vw : cols;
+            L.xprev = k == 0 ? nullptr : B.w[turn ^ 1][0];
+            L.out1 = B.w[turn][0];
+            L.out2 = B.w[turn][1];
+            L.partials = B.partials + (k - chunk_start) * per_step;
+            if (launch_chain(L, ctx->stream) != 0) throw Error{KPMX_EINVAL, "unsupported chained recurrence"};
+            KPMX_HIP(hipGetLastError());
+            const int64_t done = k + L.steps;
+            if (done - chunk_start == chunk || done == steps) {
+                launch_chain_reduce(h2->scalar, B.partials, P.ntiles, cols, done - chunk_start, nullptr, 1, t.vw, (int)c0,
+                                    sums + chunk_start * 4 * t.vw, ctx->stream);
+                KPMX_HIP(hipGetLastError());
+                chunk_start = done;
+            }
+        }
+    }
+}
+
 void check_pair(const kpmx_mat* h2, const kpmx_block* r0) {
     KPMX_REQUIRE(h2 && r0, "null matrix or starter block");
     KPMX_REQUIRE(h2->ctx == r0->ctx, "matrix and starter block belong to different contexts");
@@ -951,6 +1251,27 @@ std::vector<RunTile> run_tiles(const kpmx_block* r0, int cap) {
 }
 int diag_cap(const kpmx_mat* h2) { return h2->ctx->tile_cap[h2->scalar]; }
 
+// Whether the diagonal recurrence of this block runs in the chained form: by default on SELL matrices
+// without light-cone limits whose plans promise it to be faster than single steps.  A two-step form
+// that the caller has turned on goes first where it applies.  A plan costs 0.15 to 0.3 ms on its first
+// use and halves the recurrence at least on launch-bound systems, so runs whose single steps are
+// expected to take less than 0.4 ms in all keep those (whatever was run before: the same call always
+// takes the same form).  existing: only with plans that are there already (nothing is allocated).
+bool use_chain(const kpmx_mat* h2, const kpmx_block* r0, int64_t steps, bool existing = false) {
+    const kpmx_ctx* ctx = h2->ctx;
+    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return false;
+    double single_us = 0;
+    for (const RunTile& rt : run_tiles(r0, diag_cap(h2)))
+        single_us += std::max(5.5, 3.0 * h2->rows * rt.sub.vw * scalar_bytes(h2->scalar) / 5.6e6);
+    if (single_us * steps < 400) return false;
+    if (ctx->two_step[h2->scalar] > 0 && !existing)
+        for (const RunTile& rt : run_tiles(r0, diag_cap(h2)))
+            if (use_two_step(h2, rt.sub)) return false;
+    for (const Tile& t : r0->tiles)
+        if (!chain_plan(h2, chain_cols(h2, t), existing)) return false;
+    return true;
+}
+
 // copies a sub-tile's columns into `dst` (default: work2, sized beforehand) and returns the tile
 // to run
 Tile stage_run_tile(const kpmx_mat* h2, const kpmx_block* r0, const RunTile& rt, void* dst = nullptr) {
@@ -967,6 +1288,10 @@ Tile stage_run_tile(const kpmx_mat* h2, const kpmx_block* r0, const RunTile& rt,
 void diag_enqueue(const kpmx_mat* h2, const kpmx_block* r0, int64_t steps) {
     const auto rts = run_tiles(r0, r0->sums_cap);
     for (size_t i = 0; i < rts.size(); ++i) {
+        if (r0->sums_chain) {
+            run_chain(h2, rts[i].sub, steps, static_cast<double*>(r0->sums[i]), size_chain(h2, rts[i].sub, steps));
+            continue;
+        }
         const Tile sub = stage_run_tile(h2, r0, rts[i]);
         if (use_two_step(h2, sub))
             run_recurrence2(h2, sub, steps, static_cast<double*>(r0->sums[i]));
@@ -992,7 +1317,17 @@ void diag_run(const kpmx_mat* h2, const kpmx_block* r0c, int64_t M) {
     KPMX_REQUIRE(M >= 2 && M % 2 == 0, "num_moments must be even and >= 2");
     kpmx_ctx* ctx = h2->ctx;
     const int64_t steps = M / 2;
-    const int cap = diag_cap(h2);
+    bool chain = use_chain(h2, r0, steps);
+    if (chain) {
+        try {
+            for (const Tile& t : r0->tiles) size_chain(h2, t, steps);
+        } catch (const Error& e) {
+            if (e.code != KPMX_ENOMEM) throw;
+            chain = false;  // no memory for its work vectors: single steps
+        }
+    }
+    const int cap = chain ? 64 : diag_cap(h2);
+    r0->sums_chain = chain;
     const auto rts = run_tiles(r0, cap);
     if (r0->sums_moments != M || r0->sums_cap != cap) {
         if (!r0->sums.empty()) KPMX_HIP(hipStreamSynchronize(ctx->stream));
@@ -1012,7 +1347,14 @@ void diag_run(const kpmx_mat* h2, const kpmx_block* r0c, int64_t M) {
     const size_t sb = scalar_bytes(h2->scalar);
     size_t work = 0, part = 0, copy = 0;
     std::vector<uint64_t> key = {h2->serial, (uint64_t)M, (uint64_t)cap};
+    key.push_back((uint64_t)chain);
+    if (chain) {
+        for (const RunTile& rt : rts) size_chain(h2, rt.sub, steps);
+        for (Workspace* w : {&ctx->work0, &ctx->work1, &ctx->work3, &ctx->work4, &ctx->partials})
+            key.push_back((uint64_t)(uintptr_t)w->ptr);
+    }
     for (const RunTile& rt : rts) {
+        if (chain) break;
         const Tile& t = rt.sub;
         work = std::max(work, (size_t)h2->rows * t.vw * sb);
         if (rt.copy) copy = std::max(copy, (size_t)h2->rows * t.vw * sb);
@@ -1033,9 +1375,11 @@ void diag_run(const kpmx_mat* h2, const kpmx_block* r0c, int64_t M) {
             part = std::max(part, ctx->partials.bytes);
         }
     }
-    key.push_back((uint64_t)(uintptr_t)ctx->work0.get(work));
-    key.push_back((uint64_t)(uintptr_t)ctx->work1.get(work));
-    key.push_back((uint64_t)(uintptr_t)ctx->partials.get(part));
+    if (!chain) {
+        key.push_back((uint64_t)(uintptr_t)ctx->work0.get(work));
+        key.push_back((uint64_t)(uintptr_t)ctx->work1.get(work));
+        key.push_back((uint64_t)(uintptr_t)ctx->partials.get(part));
+    }
     if (copy) key.push_back((uint64_t)(uintptr_t)ctx->work2.get(copy));
     if (ctx->graph_policy == KPMX_GRAPH_AUTO && r0->graph_key != key && r0->last_key != key) {
         // automatic mode captures on the second run of the same recurrence: a one-off run
@@ -1571,6 +1915,7 @@ int kpmx_ctx_set_tile_width(kpmx_ctx* ctx, int scalar, int width) {
         KPMX_REQUIRE(width >= 1 && width <= 64 && (width & (width - 1)) == 0, "tile width must be 1, 2, 4, ..., 64");
         ctx->tile_cap[scalar] = width;
         ctx->two_step_auto[scalar] = false;
+        ctx->chain[scalar] = kpmx_ctx::CHAIN_PINNED_OFF;
     });
 }
 
@@ -1641,6 +1986,25 @@ int kpmx_ctx_set_graph_policy(kpmx_ctx* ctx, int policy) {
     });
 }
 
+int kpmx_diagonal_form(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, int* steps_per_launch,
+                       int* columns) {
+    return guarded([&] {
+        check_pair(h2, r0);
+        KPMX_REQUIRE(steps_per_launch && columns, "null argument");
+        KPMX_REQUIRE(num_moments >= 2 && num_moments % 2 == 0, "num_moments must be even and >= 2");
+        KPMX_HIP(hipSetDevice(h2->ctx->device));
+        const Tile& t = r0->tiles.front();
+        if (use_chain(h2, r0, num_moments / 2)) {
+            *columns = chain_cols(h2, t);
+            *steps_per_launch = chain_plan(h2, *columns)->steps;
+            return;
+        }
+        const Tile sub = run_tiles(r0, diag_cap(h2)).front().sub;
+        *columns = sub.vw;
+        *steps_per_launch = use_two_step(h2, sub) ? 2 : 1;
+    });
+}
+
 int kpmx_moments_diagonal_run(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments) {
     return guarded([&] {
         KPMX_REQUIRE(h2 && r0, "null matrix or starter block");
@@ -1670,6 +2034,44 @@ int kpmx_moments_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_
 // collected moments of the recurrence live in this device's `scratch` array (layout below, each
 // piece 256-byte aligned); nothing in it needs clearing (every launch overwrites what it reads
 // later).  Concurrent calls on one device share the array and race.
+namespace {
+// The chained form in the scratch array, with the plans an earlier kpmx_moments_diagonal left with
+// the matrix; false when it does not fit.
+bool chain_noalloc(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, void* mu) {
+    kpmx_ctx* ctx = h2->ctx;
+    if (ctx->two_step[h2->scalar] > 0) return false;
+    const int64_t steps = M / 2;
+    const size_t sb = scalar_bytes(h2->scalar);
+    auto align = [](size_t b) { return (b + 255) / 256 * 256; };
+    size_t work = 0, launch = 0;
+    int vw = 1;
+    for (const Tile& t : r0->tiles) {
+        const int cols = chain_cols(h2, t);
+        const ChainPlan& P = *chain_plan(h2, cols, true);
+        work = std::max(work, align((size_t)h2->rows * cols * sb));
+        launch = std::max(launch, P.steps * chain_step_bytes(h2, P, cols));
+        vw = std::max(vw, t.vw);
+    }
+    // [four work vectors | raw sums | moments | partial sums (rest)]
+    const size_t sums = align((size_t)steps * 4 * vw * sizeof(double)), out = align((size_t)r0->nvec * M * sb);
+    const size_t fixed = 4 * work + sums + out;
+    if (fixed + launch > KPMX_SCRATCH_BYTES) return false;
+    char* s = ctx->scratch;
+    const ChainBuffers B{{{s, s + work}, {s + 2 * work, s + 3 * work}}, reinterpret_cast<double*>(s + fixed),
+                         KPMX_SCRATCH_BYTES - fixed};
+    double* d_sums = reinterpret_cast<double*>(s + 4 * work);
+    char* d_mu = s + 4 * work + sums;
+    for (const Tile& t : r0->tiles) {
+        run_chain(h2, t, steps, d_sums, B);
+        launch_diag_collect(h2->scalar, d_sums, t.vw, t.cols, M, t.c0, d_mu, ctx->stream);
+        KPMX_HIP(hipGetLastError());
+    }
+    KPMX_HIP(hipMemcpyAsync(mu, d_mu, (size_t)r0->nvec * M * sb, hipMemcpyDeviceToHost, ctx->stream));
+    KPMX_HIP(hipStreamSynchronize(ctx->stream));
+    return true;
+}
+}  // namespace
+
 int kpmx_moments_diagonal_noalloc(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, void* mu) {
     return guarded([&] {
         KPMX_REQUIRE(h2 && r0 && mu, "null argument");
@@ -1682,6 +2084,7 @@ int kpmx_moments_diagonal_noalloc(const kpmx_mat* h2, const kpmx_block* r0, int6
         const int64_t steps = M / 2;
         const size_t sb = scalar_bytes(h2->scalar);
         auto align = [](size_t b) { return (b + 255) / 256 * 256; };
+        if (use_chain(h2, r0, steps, true) && chain_noalloc(h2, r0, M, mu)) return;
         // the same column tiles as kpmx_moments_diagonal (sub-tiles of wide starter tiles)
         const auto rts = run_tiles(r0, diag_cap(h2));
         int vw_max = 1;
@@ -2190,6 +2593,7 @@ int kpmx_ctx_set_step_variant(kpmx_ctx* ctx, int scalar, int vector_width, int v
         KPMX_REQUIRE(variant >= 0 && variant < NUM_TUNE_VARIANTS, "variant out of range");
         ctx->tune[scalar][log2i(vector_width)] = variant;
         ctx->tune_coded[scalar][log2i(vector_width)] = -1;
+        ctx->chain[scalar] = kpmx_ctx::CHAIN_PINNED_OFF;
     });
 }
 
@@ -2200,12 +2604,12 @@ namespace {
 // the fastest per vector is kept in the context (tile width and two-step settings) when it beats
 // the single steps' `single_per_vector` milliseconds per vector and step by 2 %, else the
 // settings are left as they were.
-void autotune_two_step(const kpmx_mat* h2, const kpmx_block* r0, double single_per_vector) {
+double autotune_two_step(const kpmx_mat* h2, const kpmx_block* r0, double single_per_vector) {
     kpmx_ctx* ctx = h2->ctx;
     const int sc = h2->scalar;
     if ((sc != KPMX_F64 && sc != KPMX_C128) || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty() ||
         h2->rows < 2 * 64)
-        return;
+        return single_per_vector;
     const int saved[4] = {ctx->two_step[sc], ctx->two_step_wg_per_cu[sc], ctx->two_step_lds[sc], ctx->tile_cap[sc]};
     auto set = [&](int rows, int wg, int lds, int cap) {
         ctx->two_step[sc] = rows;
@@ -2259,6 +2663,45 @@ void autotune_two_step(const kpmx_mat* h2, const kpmx_block* r0, double single_p
     } else {
         set(saved[0], saved[1], saved[2], saved[3]);
     }
+    return best_cap ? best : single_per_vector;
+}
+
+// Takes back the autotuner's choice of the LDS two-step form.
+void reset_two_step_choice(kpmx_ctx* ctx, int scalar) {
+    ctx->two_step[scalar] = ctx->two_step_wg_per_cu[scalar] = ctx->two_step_lds[scalar] = 0;
+    ctx->tile_cap[scalar] = default_tile_cap(scalar);
+    ctx->two_step_auto[scalar] = false;
+}
+
+// Switches the chained form off while another form is faster per vector and step.
+void autotune_chain(const kpmx_mat* h2, const kpmx_block* r0, double best_per_vector) {
+    kpmx_ctx* ctx = h2->ctx;
+    if (ctx->two_step[h2->scalar] > 0 && !ctx->two_step_auto[h2->scalar]) return;  // the caller's
+    const int two_step = ctx->two_step[h2->scalar];
+    ctx->two_step[h2->scalar] = 0;
+    const bool chain = use_chain(h2, r0, 1 << 20);
+    ctx->two_step[h2->scalar] = two_step;
+    if (!chain) return;
+    Tile t = r0->tiles.front();
+    t.cols = std::min<int64_t>(t.cols, chain_cols(h2, t));  // one column group
+    const double step_bytes = 3.0 * (double)h2->rows * t.cols * scalar_bytes(h2->scalar);
+    const int64_t steps = std::max<int64_t>(24, std::min<int64_t>(256, (int64_t)(4e9 / step_bytes)));
+    double* sums = static_cast<double*>(ctx->sums.get((size_t)steps * 4 * t.vw * sizeof(double)));
+    float best = 0;
+    for (int rep = 0; rep < 4; ++rep) {  // the first repetition warms caches and code
+        KPMX_HIP(hipEventRecord(ctx->t0, ctx->stream));
+        run_chain(h2, t, steps, sums, size_chain(h2, t, steps));
+        KPMX_HIP(hipEventRecord(ctx->t1, ctx->stream));
+        KPMX_HIP(hipEventSynchronize(ctx->t1));
+        float ms = 0;
+        KPMX_HIP(hipEventElapsedTime(&ms, ctx->t0, ctx->t1));
+        if (rep == 1 || (rep > 1 && ms < best)) best = ms;
+    }
+    if (best / ((double)steps * t.cols) > best_per_vector) {
+        ctx->chain[h2->scalar] = kpmx_ctx::CHAIN_TUNED_OFF;
+    } else if (ctx->two_step_auto[h2->scalar]) {
+        reset_two_step_choice(ctx, h2->scalar);
+    }
 }
 }  // namespace
 
@@ -2267,11 +2710,8 @@ int kpmx_autotune_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int* varian
         check_pair(h2, r0);
         kpmx_ctx* ctx = h2->ctx;
         KPMX_HIP(hipSetDevice(ctx->device));
-        if (ctx->two_step_auto[h2->scalar]) {  // an earlier autotuner choice: start from the defaults
-            ctx->two_step[h2->scalar] = ctx->two_step_wg_per_cu[h2->scalar] = ctx->two_step_lds[h2->scalar] = 0;
-            ctx->tile_cap[h2->scalar] = default_tile_cap(h2->scalar);
-            ctx->two_step_auto[h2->scalar] = false;
-        }
+        if (ctx->two_step_auto[h2->scalar]) reset_two_step_choice(ctx, h2->scalar);  // start from the defaults
+        if (ctx->chain[h2->scalar] == kpmx_ctx::CHAIN_TUNED_OFF) ctx->chain[h2->scalar] = kpmx_ctx::CHAIN_ON;
         // the first column tile the diagonal recurrence runs (a sub-tile of a wider starter tile)
         const Tile t = stage_run_tile(h2, r0, run_tiles(r0, diag_cap(h2)).front());
         // About 2 GB of vector traffic per timed sample (at least 9 steps, at most 255): small
@@ -2308,7 +2748,9 @@ int kpmx_autotune_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int* varian
         ctx->tune[h2->scalar][log2i(t.vw)] = best;
         ctx->tune_coded[h2->scalar][log2i(t.vw)] = -1;
         if (variant) *variant = best;
-        if (ctx->autotune_two_step) autotune_two_step(h2, r0, best_ms / ((double)steps * t.vw));
+        double per_vector = best_ms / ((double)steps * t.vw);
+        if (ctx->autotune_two_step) per_vector = autotune_two_step(h2, r0, per_vector);
+        autotune_chain(h2, r0, per_vector);
     });
 }
 

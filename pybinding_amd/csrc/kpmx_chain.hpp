@@ -1,0 +1,97 @@
+// Launch interface of the chained diagonal recurrence (kpmx_chain.hip): several Chebyshev steps per
+// launch on row tiles whose vectors stay in LDS.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace kpmx {
+
+constexpr int CHAIN_MAX_STEPS = 12;      // steps per launch at most
+constexpr int CHAIN_MAX_HALO = 6144;     // halo rows of a tile at most
+constexpr int CHAIN_CANDIDATES = 8;      // tile heights whose halos one chain_sample measures
+constexpr int CHAIN_SAMPLES = 32;        // tiles it looks at per height
+
+// Matrix entries of a plan: every stored value (standard SELL), 1-byte codes into a value table,
+// or one value for all off-diagonal entries; the last two keep the diagonal as a dense vector.
+enum { CHAIN_STD = 0, CHAIN_TABLE = 1, CHAIN_UNIFORM = 2 };
+
+// The SELL-64 matrix a plan is built from: with codes the off-diagonal entries and the diagonal.
+struct ChainMatrix {
+    int scalar = 1;
+    int64_t n = 0;
+    int max_width = 0;
+    const int64_t* slice_ptr = nullptr;
+    const int32_t* slice_width = nullptr;
+    const int32_t* indices = nullptr;
+    const void* vals = nullptr;      // standard form
+    const uint8_t* codes = nullptr;  // value-table form
+    const void* diag = nullptr;
+    const void* table = nullptr;
+    int table_size = 0;
+    int form() const { return !codes ? CHAIN_STD : table_size <= 2 ? CHAIN_UNIFORM : CHAIN_TABLE; }
+};
+
+// Device arrays of a plan.  Tile t owns rows [tile_begin[t], tile_begin[t + 1]); its local rows are
+// those, then its halo: the rows at distance 1, 2, ..., `steps` from them in the matrix's graph
+// (ext, ascending inside a ring).  ring[t * (CHAIN_MAX_STEPS + 1) + j] counts the local rows up to
+// distance j.  Entries are kept for the local rows up to distance steps - 1.
+struct ChainPlan {
+    int64_t ntiles = 0, tile_rows = 0;
+    int steps = 0;      // steps per launch the entries reach for
+    int width = 0;      // entries per row
+    int groups = 0;     // ceil(width / 4)
+    int rows_x = 0;     // most local rows of a tile (distance <= steps)
+    int rows_y = 0;     // row stride of the entry arrays (rows at distance <= steps - 1, padded)
+    int row_items = 1;  // items of a row
+    int64_t ext_stride = 0;
+    int32_t* tile_begin = nullptr;
+    int32_t* ring = nullptr;
+    int32_t* ext = nullptr;
+    ushort4* lidx = nullptr;    // [tile][group][row], first item of the column's local row (none: the zero row)
+    uint32_t* codes = nullptr;  // [tile][group][row], four 1-byte codes
+    void* vals = nullptr;       // [tile][entry][row]
+    void* diag = nullptr;       // [tile][row]
+};
+
+// (launches return 0, or -1 where the device refuses)
+// local rows (distance <= j) of sampled tiles of each candidate height: out[(c * CHAIN_SAMPLES + s)
+// * (CHAIN_MAX_STEPS + 1) + j], -1 where they exceed `capacity` rows
+int chain_sample(const ChainMatrix& m, const int* heights, int count, int capacity, int32_t* out, hipStream_t s);
+// ring counts and halo rows (at most P.ext_stride) of every tile (P.tile_begin set; P.ring, P.ext
+// allocated)
+int chain_rings(const ChainMatrix& m, const ChainPlan& P, int max_steps, hipStream_t s);
+// entry arrays of every tile (P.steps, rows_x, rows_y set and the arrays allocated)
+int chain_entries(const ChainMatrix& m, const ChainPlan& P, hipStream_t s);
+
+struct ChainLaunch {
+    ChainMatrix m;
+    const ChainPlan* plan = nullptr;
+    int cols = 8;              // vectors per row of the work blocks
+    int steps = 1;             // steps of this launch (<= plan->steps)
+    bool first = false;        // the first step is 0.5 H2 x
+    const void* x = nullptr;   // r_k, rows of ldx scalars
+    int64_t ldx = 0;
+    const void* xprev = nullptr;  // r_{k-1}, rows of `cols` scalars (not read by a first launch)
+    void* out1 = nullptr;         // r_{k+steps-1} (not written by a one-step launch)
+    void* out2 = nullptr;         // r_{k+steps}
+    double* partials = nullptr;   // [steps][ntiles][chain_partial_width]
+};
+// widest supported column tile of a scalar type
+int chain_max_cols(int scalar);
+// local rows one workgroup's LDS holds
+int chain_row_capacity(const ChainMatrix& m, int cols);
+// items of a row (see kpmx_chain_step.hpp); the row stride of the entry arrays is a multiple of pad
+int chain_row_items(int scalar, int cols);
+int chain_row_pad(const ChainMatrix& m, int cols);
+int chain_partial_width(int scalar, int cols);
+int launch_chain(const ChainLaunch& L, hipStream_t s);
+int launch_chain_f32(const ChainLaunch& L, hipStream_t s);
+int launch_chain_f64(const ChainLaunch& L, hipStream_t s);
+int launch_chain_c64(const ChainLaunch& L, hipStream_t s);
+int launch_chain_c128(const ChainLaunch& L, hipStream_t s);
+// sums[step][system][4 vw] of the columns [c0, c0 + cols) of a vw-column block from the partials of
+// nsteps steps; system_tiles (num_systems + 1) null: one system over all tiles
+void launch_chain_reduce(int scalar, const double* partials, int64_t ntiles, int cols, int64_t nsteps,
+                         const int32_t* system_tiles, int64_t num_systems, int vw, int c0, double* sums, hipStream_t s);
+
+}  // namespace kpmx

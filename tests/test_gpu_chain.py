@@ -1,0 +1,144 @@
+"""The chained diagonal recurrence (several steps per launch on row tiles with halos, the default on
+SELL matrices) against the oracle and against single steps (a pinned step variant) on every element
+layout: each scalar type and column width, the three matrix forms (one hopping value, a value table,
+stored values), rows of 0 to 19 entries, ragged tiles, step counts with every remainder of the steps
+per launch, site orders with small and large halos.  Runs are long enough (150 moments) that the
+dispatch takes the chain for its plan's cost; shorter ones check that they do not need it.
+
+Tolerances: the repository's parity bounds, 1e-10 (fp64, complex128) and 1e-4 (fp32, complex64) of
+mu_0 against the oracle; twice that between two device forms."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import abi
+from pybinding_amd import generators
+
+pytestmark = pytest.mark.gpu
+
+TOL = {np.float64: 1e-10, np.complex128: 1e-10, np.float32: 1e-4, np.complex64: 1e-4}
+
+
+def hilbert(h, n1, n2):
+    inv = np.argsort(generators.honeycomb_cell_order(n1, n2))
+    h = h[inv][:, inv].tocsr()
+    h.sort_indices()
+    return h
+
+
+def scaled(h, dtype):
+    h = (h * (2 / 10.0)).astype(dtype)
+    h.sort_indices()
+    return h
+
+
+def lattice(form, n1=40, n2=24, dtype=np.float64):
+    """honeycomb supercell with one hopping value, with three of them, or all different"""
+    h = hilbert(generators.honeycomb_supercell(n1, n2, disorder=0.7, seed=4), n1, n2)
+    rng = np.random.default_rng(8)
+    if form != "uniform":
+        up = sp.triu(h, 1).tocsr()
+        up.data *= rng.choice([0.8, 1.0, 1.1], up.nnz) if form == "table" else rng.uniform(0.7, 1.1, up.nnz)
+        phase = np.exp(1j * up.data) if np.dtype(dtype).kind == "c" and form == "stored" else 1
+        up.data = up.data * phase
+        h = (up + up.conj().T + sp.diags(h.diagonal())).tocsr()
+    return scaled(h, dtype)
+
+
+def starters(n, nvec, dtype, seed=3):
+    rng = np.random.default_rng(seed)
+    if np.dtype(dtype).kind == "c":
+        return np.exp(2j * np.pi * rng.random((nvec, n))).astype(dtype)
+    return (2 * rng.integers(0, 2, (nvec, n)) - 1).astype(dtype)
+
+
+def run(h2, r0, moments, single=False):
+    ctx = abi.Ctx(0)
+    try:
+        mat, blk = ctx.mat(h2, fmt=1), ctx.block(r0)
+        if single:
+            ctx.set_tile_width(h2.dtype, 64)
+        return abi.moments_diagonal(mat, blk, moments)
+    finally:
+        ctx.close()
+
+
+def check(oracle, h2, r0, moments):
+    dtype = h2.dtype.type
+    mu, ref = run(h2, r0, moments), oracle.diag_moments(h2, r0, moments)
+    scale = np.abs(ref[:, :1])
+    assert np.max(np.abs(mu - ref) / scale) <= TOL[dtype]
+    assert np.max(np.abs(mu - run(h2, r0, moments, single=True)) / scale) <= 2 * TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128, np.complex64])
+@pytest.mark.parametrize("form", ["uniform", "table", "stored"])
+@pytest.mark.parametrize("nvec", [1, 2, 3, 7, 16, 24])
+def test_layouts(oracle, dtype, form, nvec):
+    h2 = lattice(form, dtype=dtype)
+    print("chain", np.dtype(dtype).name, form, nvec, flush=True)
+    check(oracle, h2, starters(h2.shape[0], nvec, dtype), 158)
+
+
+@pytest.mark.parametrize("moments", [2, 24, 150, 152, 154, 156, 158, 160, 162, 164, 166, 168, 170, 172])
+def test_step_counts(oracle, moments):
+    h2 = lattice("uniform", 17, 9)
+    print("chain steps", moments, flush=True)
+    check(oracle, h2, starters(h2.shape[0], 4, np.float64), moments)
+
+
+@pytest.mark.parametrize("n1,n2", [(4, 4), (8, 4), (11, 3), (64, 32), (90, 70)])
+def test_sizes(oracle, n1, n2):
+    """one tile that holds the whole system, ragged last tiles, several tiles per CU"""
+    h2 = lattice("uniform", n1, n2)
+    print("chain size", h2.shape[0], flush=True)
+    check(oracle, h2, starters(h2.shape[0], 5, np.float64), 150)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128])
+@pytest.mark.parametrize("width", [5, 8, 19])
+def test_long_rows(oracle, dtype, width):
+    """rows of up to `width` off-diagonal entries near the diagonal, some rows empty"""
+    n = 1500
+    rng = np.random.default_rng(width)
+    up = sp.random(n, n, density=0.0, format="lil")
+    for d in range(1, width // 2 + 1):
+        v = rng.uniform(0.1, 0.3, n - d) * (rng.random(n - d) < 0.9)
+        v[700:720] = 0
+        up += sp.diags(v, d, shape=(n, n))
+    up = sp.csr_matrix(up)
+    up.eliminate_zeros()
+    h = (up + up.T).tocsr()
+    h2 = (h * (2 / abs(h).sum(axis=1).max())).astype(dtype)  # a scaled Hamiltonian: spectrum in [-2, 2]
+    h2.sort_indices()
+    print("chain width", width, np.dtype(dtype).name, flush=True)
+    check(oracle, h2, starters(n, 6, dtype), 154)
+
+
+def test_orders(oracle):
+    """row-major and random site orders (halos too large for a chain: single steps) agree"""
+    n1, n2 = 96, 80
+    h = generators.honeycomb_supercell(n1, n2, disorder=0.7, seed=4)
+    r0 = starters(h.shape[0], 4, np.float64)
+    for q in (np.arange(h.shape[0]), np.random.default_rng(1).permutation(h.shape[0])):
+        h2 = scaled(h[q][:, q].tocsr(), np.float64)
+        print("chain order", q[:3], flush=True)
+        check(oracle, h2, np.ascontiguousarray(r0[:, q]), 150)
+
+
+def test_repeats_and_graph_replays_are_bitwise():
+    h2 = lattice("table")
+    r0 = starters(h2.shape[0], 9, np.float64)
+    ctx = abi.Ctx(0)
+    try:
+        mat, blk = ctx.mat(h2, fmt=1), ctx.block(r0)
+        first = abi.moments_diagonal(mat, blk, 166)
+        assert np.array_equal(abi.moments_diagonal(mat, blk, 166), first)
+        ctx.set_graph_policy(2)
+        for _ in range(3):
+            assert np.array_equal(abi.moments_diagonal(mat, blk, 166), first)
+            other = ctx.block(starters(h2.shape[0], 3, np.float64, seed=9))
+            abi.moments_diagonal(mat, other, 10)
+            other.close()
+    finally:
+        ctx.close()
