@@ -201,9 +201,16 @@ struct LdsHalo {
 // (one allocation; null data: the matrix is better off with other forms).
 struct ChainHolder {
     int cols = 0;
+    bool coded = false;          // batches: the matrix form it was built from
     ChainPlan plan;
+    std::vector<int32_t> begin;  // plan.tile_begin
     char* data = nullptr;
-    ~ChainHolder() { dev_free(data); }
+    // batches: [systems + 1] first tile of every system, then plan.tile_table
+    int32_t* systems = nullptr;
+    ~ChainHolder() {
+        dev_free(data);
+        dev_free(systems);
+    }
 };
 
 struct kpmx_mat {
@@ -326,6 +333,8 @@ struct kpmx_batch {
     int64_t s_entries = 0;  // stored slots of the standard form (padding included)
     int64_t c_entries = 0;  // stored off-diagonal slots (padding included)
     int64_t table_len = 0;
+    int table_most = 0;                // entries of the largest table
+    std::vector<int32_t> tab_off_host;
     int64_t* cslice_ptr = nullptr;
     int32_t* cslice_width = nullptr;
     int32_t* cidx = nullptr;
@@ -352,6 +361,15 @@ struct kpmx_batch {
     double* partials = nullptr;
     double* partials2 = nullptr;     // the persistent run's two partial buffers
     unsigned* barrier = nullptr;     // the persistent run's grid barrier
+    // the chained form of run modes 0 and 1 (see kpmx_chain_step.hpp): off once the caller pins a
+    // partition, or while the autotuner has found the walkers faster
+    bool chain_on = true;
+    bool graph_chain = false;        // the captured graph runs it
+    std::vector<std::unique_ptr<ChainHolder>> chains;
+    void* w2 = nullptr;              // with w0 and w1 its four work vectors
+    void* w3 = nullptr;
+    double* chain_partials = nullptr;
+    size_t chain_partials_bytes = 0;
     double* sums = nullptr;
     int64_t sums_steps = 0;
     hipGraph_t graph = nullptr;
@@ -368,7 +386,7 @@ struct kpmx_batch {
         drop_graph();
         for (void* p : {(void*)slice_ptr, (void*)slice_width, (void*)slice_sys, (void*)sidx, svals, (void*)tile_begin,
                         (void*)slot_begin, (void*)slot_index, (void*)slot_first, r0, w0, w1, (void*)partials, (void*)partials2,
-                        (void*)barrier, (void*)sums, (void*)cslice_ptr, (void*)cslice_width, (void*)cidx, (void*)ccodes,
+                        (void*)barrier, w2, w3, (void*)chain_partials, (void*)sums, (void*)cslice_ptr, (void*)cslice_width, (void*)cidx, (void*)ccodes,
                         cdiag, ctable, (void*)ctab_off})
             dev_free(p);
     }
@@ -942,7 +960,7 @@ ChainMatrix chain_matrix(const kpmx_mat* h2) {
         m.codes = h2->ccodes;
         m.diag = h2->cdiag;
         m.table = h2->ctable;
-        m.table_size = h2->ctable_size;
+        m.table_size = m.table_most = h2->ctable_size;
     } else {
         m.max_width = h2->max_width;
         m.slice_ptr = h2->slice_ptr;
@@ -977,15 +995,16 @@ double chain_cost(const ChainMatrix& m, double rows, const double* e, int steps,
     return (3.0 + rounds * round) / steps;
 }
 
-// The plan of a matrix for `cols` columns: the tile height and steps per launch with the least
-// estimated time per step over a few heights whose halos are measured on sampled tiles.
-const ChainPlan* build_chain(const kpmx_mat* h2, int cols, ChainHolder& H) {
-    kpmx_ctx* ctx = h2->ctx;
-    const int64_t n = h2->rows;
-    const ChainMatrix m = chain_matrix(h2);
+// Builds a plan for `cols` columns into H: the tile height and steps per launch with the least
+// estimated time per step over a few heights whose halos are measured on sampled tiles.  cut(rows)
+// gives the tiles' first rows and, last, the row count.  H.data stays null when no plan promises less
+// than `single_us` per step.
+template <class Cut>
+void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us, Cut cut, ChainHolder& H) {
+    const int64_t n = m.n;
     const int cap = chain_row_capacity(m, cols);
-    if (cap <= 0 || n < 64) return nullptr;
-    const size_t sb = scalar_bytes(h2->scalar);
+    if (cap <= 0 || n < 64) return;
+    const size_t sb = scalar_bytes(m.scalar);
     const double row_bytes = (double)cols * sb;
     // heights: as many tiles as CUs and small multiples of twice that (no CU idles in the last
     // round), and fractions of what a workgroup holds
@@ -1005,7 +1024,7 @@ const ChainPlan* build_chain(const kpmx_mat* h2, int cols, ChainHolder& H) {
     add(0.6 * cap);
     add(0.45 * cap);
     add(0.3 * cap);
-    if (heights.empty()) return nullptr;
+    if (heights.empty()) return;
     constexpr int ST = CHAIN_MAX_STEPS + 1;
     std::vector<int32_t> ring(heights.size() * CHAIN_SAMPLES * ST);
     int32_t* d = static_cast<int32_t*>(ctx->aux2.get(ring.size() * sizeof(int32_t)));
@@ -1035,17 +1054,12 @@ const ChainPlan* build_chain(const kpmx_mat* h2, int cols, ChainHolder& H) {
             }
         }
     }
-    // single steps: about 5.6 TB/s of three passes over the columns and their share of the matrix, no
-    // less than a launch; a third of that on long rows
-    const double sweep = (3.0 * n * row_bytes + (double)h2->nnz * (sb + 4) * cols / std::max(cols, ctx->tile_cap[h2->scalar])) / 5.6e6;
-    if (!rows || best > std::max(5.5, sweep * (m.max_width > 8 ? 3 : 1))) return nullptr;
+    if (!rows || best > single_us) return;
     // halos of every tile into scratch; tiles whose local rows exceed the capacity are halved
     ChainPlan P;
     P.tile_rows = rows;
     P.ext_stride = std::min(CHAIN_MAX_HALO, cap - rows);
-    std::vector<int32_t> begin;
-    for (int64_t r = 0; r < n; r += rows) begin.push_back((int32_t)r);
-    begin.push_back((int32_t)n);
+    std::vector<int32_t> begin = cut(rows);
     auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
     std::vector<int> most(ST, 0);
     for (int pass = 0;; ++pass) {
@@ -1078,7 +1092,7 @@ const ChainPlan* build_chain(const kpmx_mat* h2, int cols, ChainHolder& H) {
         begin.swap(split);
     }
     while (steps > 1 && most[steps] < 0) --steps;
-    if (steps < 2) return nullptr;
+    if (steps < 2) return;
     int halo = 0;
     for (int64_t t = 0; t < P.ntiles; ++t) halo = std::max(halo, ring[t * ST + steps] - ring[t * ST]);
     const size_t ring_bytes = (size_t)P.ntiles * ST * sizeof(int32_t), begin_bytes = (size_t)(P.ntiles + 1) * sizeof(int32_t);
@@ -1088,7 +1102,7 @@ const ChainPlan* build_chain(const kpmx_mat* h2, int cols, ChainHolder& H) {
     P.rows_x = most[steps];
     const int row_pad = chain_row_pad(m, cols);
     P.rows_y = (most[steps - 1] + row_pad - 1) / row_pad * row_pad;
-    P.row_items = chain_row_items(h2->scalar, cols);
+    P.row_items = chain_row_items(m.scalar, cols);
     const int form = m.form();
     const int64_t src_stride = P.ext_stride;
     const size_t cells = (size_t)P.ntiles * P.rows_y;
@@ -1125,7 +1139,7 @@ const ChainPlan* build_chain(const kpmx_mat* h2, int cols, ChainHolder& H) {
     KPMX_REQUIRE(chain_entries(m, P, ctx->stream) == 0, "no LDS for a chain plan");
     KPMX_HIP(hipGetLastError());
     H.plan = P;
-    return &H.plan;
+    H.begin = std::move(begin);
 }
 
 // The plan for `cols` columns, built on first use (unless `existing` asks for one that is there
@@ -1136,8 +1150,20 @@ const ChainPlan* chain_plan(const kpmx_mat* h2, int cols, bool existing = false)
     if (existing) return nullptr;
     auto H = std::make_unique<ChainHolder>();
     H->cols = cols;
+    // single steps: about 5.6 TB/s of three passes over the columns and their share of the matrix, no
+    // less than a launch; a third of that on long rows
+    const ChainMatrix m = chain_matrix(h2);
+    const size_t sb = scalar_bytes(h2->scalar);
+    const double sweep = (3.0 * (double)h2->rows * cols * sb +
+                          (double)h2->nnz * (sb + 4) * cols / std::max(cols, h2->ctx->tile_cap[h2->scalar])) / 5.6e6;
+    auto cut = [&](int rows) {
+        std::vector<int32_t> begin;
+        for (int64_t r = 0; r < h2->rows; r += rows) begin.push_back((int32_t)r);
+        begin.push_back((int32_t)h2->rows);
+        return begin;
+    };
     try {
-        build_chain(h2, cols, *H);
+        build_chain(h2->ctx, m, cols, std::max(5.5, sweep * (m.max_width > 8 ? 3 : 1)), cut, *H);
     } catch (const Error& e) {
         if (e.code != KPMX_ENOMEM) throw;
         dev_free(H->data);
@@ -1176,25 +1202,23 @@ ChainBuffers size_chain(const kpmx_mat* h2, const Tile& t, int64_t steps) {
 // The diagonal recurrence of a starter tile in the chained form, in column groups of at most
 // chain_max_cols vectors; the first launch of a group reads its columns in place.  Two pairs of work
 // vectors take turns: a launch reads (r_{k-1}, r_k) and writes (r_{k+K-1}, r_{k+K}).
-void run_chain(const kpmx_mat* h2, const Tile& t, int64_t steps, double* sums, const ChainBuffers& B) {
-    kpmx_ctx* ctx = h2->ctx;
-    const int cols = chain_cols(h2, t);
-    const ChainPlan& P = *chain_plan(h2, cols);
-    const size_t sb = scalar_bytes(h2->scalar), step_bytes = chain_step_bytes(h2, P, cols);
-    const int64_t per_step = (int64_t)(step_bytes / sizeof(double));
-    const int64_t chunk = std::max<int64_t>(1, (int64_t)(B.partials_bytes / step_bytes) / P.steps) * P.steps;
+void run_chain(kpmx_ctx* ctx, const ChainMatrix& m, const ChainPlan& P, int cols, const void* r0, int vw, int64_t vectors,
+               int64_t steps, const int32_t* system_tiles, int64_t num_systems, double* sums, const ChainBuffers& B) {
+    const size_t sb = scalar_bytes(m.scalar);
+    const int64_t per_step = P.ntiles * chain_partial_width(m.scalar, cols);
+    const int64_t chunk = std::max<int64_t>(1, (int64_t)(B.partials_bytes / sizeof(double)) / per_step / P.steps) * P.steps;
     ChainLaunch L;
-    L.m = chain_matrix(h2);
+    L.m = m;
     L.plan = &P;
     L.cols = cols;
-    for (int64_t c0 = 0; c0 < t.cols; c0 += cols) {
+    for (int64_t c0 = 0; c0 < vectors; c0 += cols) {
         int64_t chunk_start = 0;
         int turn = 0;
         for (int64_t k = 0; k < steps; k += L.steps, turn ^= 1) {
             L.steps = (int)std::min<int64_t>(P.steps, steps - k);
             L.first = k == 0;
-            L.x = k == 0 ? static_cast<const char*>(t.data) + c0 * sb : B.w[turn ^ 1][1];
-            L.ldx = k == 0 ? t.vw : cols;
+            L.x = k == 0 ? static_cast<const char*>(r0) + c0 * sb : B.w[turn ^ 1][1];
+            L.ldx = k == 0 ? vw : cols;
             L.xprev = k == 0 ? nullptr : B.w[turn ^ 1][0];
             L.out1 = B.w[turn][0];
             L.out2 = B.w[turn][1];
@@ -1203,13 +1227,17 @@ void run_chain(const kpmx_mat* h2, const Tile& t, int64_t steps, double* sums, c
             KPMX_HIP(hipGetLastError());
             const int64_t done = k + L.steps;
             if (done - chunk_start == chunk || done == steps) {
-                launch_chain_reduce(h2->scalar, B.partials, P.ntiles, cols, done - chunk_start, nullptr, 1, t.vw, (int)c0,
-                                    sums + chunk_start * 4 * t.vw, ctx->stream);
+                launch_chain_reduce(m.scalar, B.partials, P.ntiles, cols, done - chunk_start, system_tiles, num_systems, vw,
+                                    (int)c0, sums + chunk_start * num_systems * 4 * vw, ctx->stream);
                 KPMX_HIP(hipGetLastError());
                 chunk_start = done;
             }
         }
     }
+}
+void run_chain(const kpmx_mat* h2, const Tile& t, int64_t steps, double* sums, const ChainBuffers& B) {
+    const int cols = chain_cols(h2, t);
+    run_chain(h2->ctx, chain_matrix(h2), *chain_plan(h2, cols), cols, t.data, t.vw, t.cols, steps, nullptr, 1, sums, B);
 }
 
 void check_pair(const kpmx_mat* h2, const kpmx_block* r0) {
@@ -2871,6 +2899,8 @@ void build_batch_coded(kpmx_batch* b, const int64_t* row_offsets, const int32_t*
     b->cmax_width = ns_tot ? *std::max_element(cwidth.begin(), cwidth.end()) : 0;
     b->c_entries = total;
     b->table_len = tab_off[S];
+    for (int64_t sy = 0; sy < S; ++sy) b->table_most = std::max(b->table_most, (int)(tab_off[sy + 1] - tab_off[sy]));
+    b->tab_off_host = tab_off;
     b->has_coded = b->use_coded = true;
 }
 }  // namespace
@@ -2983,8 +3013,10 @@ int kpmx_batch_starters(kpmx_batch* b, int64_t num_vectors, const void* r0) {
             dev_free(b->r0);
             dev_free(b->w0);
             dev_free(b->w1);
+            dev_free(b->w2);
+            dev_free(b->w3);
             dev_free(b->sums);
-            b->r0 = b->w0 = b->w1 = nullptr;
+            b->r0 = b->w0 = b->w1 = b->w2 = b->w3 = nullptr;
             b->sums = nullptr;
             b->sums_steps = 0;
             b->drop_graph();
@@ -3085,6 +3117,114 @@ void batch_enqueue(kpmx_batch* b, int64_t steps, int64_t t = 0) {
 }  // namespace
 
 namespace {
+int batch_chain_cols(const kpmx_batch* b) { return std::min(pick_vw(b->tile_cols), chain_max_cols(b->scalar)); }
+
+ChainMatrix batch_chain_matrix(const kpmx_batch* b) {
+    ChainMatrix m;
+    m.scalar = b->scalar;
+    m.n = b->n_pad;
+    m.max_width = b->use_coded ? b->cmax_width : b->max_width;
+    m.slice_ptr = b->use_coded ? b->cslice_ptr : b->slice_ptr;
+    m.slice_width = b->use_coded ? b->cslice_width : b->slice_width;
+    m.indices = b->use_coded ? b->cidx : b->sidx;
+    m.vals = b->svals;
+    if (b->use_coded) {
+        m.vals = nullptr;
+        m.codes = b->ccodes;
+        m.diag = b->cdiag;
+        m.table = b->ctable;
+        m.table_size = (int)b->table_len;
+        m.table_most = b->table_most;
+    }
+    return m;
+}
+
+// The plan of the batch's chained form with its work vectors and partial sums, or null: short runs
+// (as for one matrix), pinned partitions, halos that do not fit and memory that is not there keep the
+// walkers.  A tile lies in one system, so its sums belong to that system.
+const ChainHolder* batch_chain(kpmx_batch* b, int64_t steps) {
+    kpmx_ctx* ctx = b->ctx;
+    const size_t sb = scalar_bytes(b->scalar);
+    const double sweep = 3.0 * (double)b->n_pad * b->vw * sb / 5.6e6;
+    if (!b->chain_on || std::max(10.0, sweep) * steps * b->ntiles < 400) return nullptr;
+    const int cols = batch_chain_cols(b);
+    ChainHolder* H = nullptr;
+    for (auto& c : b->chains)
+        if (c->cols == cols && c->coded == b->use_coded) H = c.get();
+    try {
+        if (!H) {
+            b->chains.push_back(std::make_unique<ChainHolder>());
+            H = b->chains.back().get();
+            H->cols = cols;
+            H->coded = b->use_coded;
+            auto cut = [&](int rows) {  // even tiles of at most `rows` rows in every system
+                std::vector<int32_t> begin;
+                for (int64_t sy = 0; sy < b->num_sys; ++sy) {
+                    const int64_t size = b->pad_off[sy + 1] - b->pad_off[sy], count = (size + rows - 1) / rows;
+                    for (int64_t q = 0; q < count; ++q) begin.push_back((int32_t)(b->pad_off[sy] + size * q / count));
+                }
+                begin.push_back((int32_t)b->n_pad);
+                return begin;
+            };
+            const double entries = b->use_coded ? 5.0 * b->c_entries : (4.0 + sb) * b->s_entries;
+            const double us = (3.0 * (double)b->n_pad * cols * sb + entries * cols / b->vw) / 5.6e6;
+            build_chain(ctx, batch_chain_matrix(b), cols, std::max(10.0, us * (b->max_width > 8 ? 3 : 1)), cut, *H);
+            if (H->data) {
+                std::vector<int32_t> up;  // first tile of every system, then the table of every tile
+                size_t sy = 0;
+                for (int64_t t = 0; t < H->plan.ntiles; ++t)
+                    if (sy < (size_t)b->num_sys && H->begin[t] == b->pad_off[sy]) {
+                        up.push_back((int32_t)t);
+                        ++sy;
+                    }
+                up.push_back((int32_t)H->plan.ntiles);
+                KPMX_REQUIRE(up.size() == (size_t)b->num_sys + 1, "internal error: a chain tile across systems");
+                if (b->use_coded)
+                    for (size_t s = 0; s < (size_t)b->num_sys; ++s)
+                        for (int32_t t = up[s]; t < up[s + 1]; ++t) up.push_back(b->tab_off_host[s]);
+                H->systems = static_cast<int32_t*>(dev_alloc(up.size() * sizeof(int32_t)));
+                KPMX_HIP(hipMemcpyAsync(H->systems, up.data(), up.size() * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+                KPMX_HIP(hipStreamSynchronize(ctx->stream));
+                if (b->use_coded) H->plan.tile_table = H->systems + b->num_sys + 1;
+            }
+        }
+        if (!H->data) return nullptr;
+        const size_t blk = (size_t)b->n_pad * b->vw * sb;
+        if (!b->w2) b->w2 = dev_alloc(blk);
+        if (!b->w3) b->w3 = dev_alloc(blk);
+        const size_t step_bytes = (size_t)H->plan.ntiles * chain_partial_width(b->scalar, cols) * sizeof(double);
+        const size_t need = std::min(std::max(CHAIN_PARTIALS, H->plan.steps * step_bytes), (steps + H->plan.steps) * step_bytes);
+        if (need > b->chain_partials_bytes) {
+            KPMX_HIP(hipStreamSynchronize(ctx->stream));
+            b->drop_graph();
+            dev_free(b->chain_partials);
+            b->chain_partials = nullptr;
+            b->chain_partials_bytes = 0;
+            b->chain_partials = static_cast<double*>(dev_alloc(need));
+            b->chain_partials_bytes = need;
+        }
+    } catch (const Error& e) {
+        if (e.code != KPMX_ENOMEM) throw;
+        if (H) {
+            dev_free(H->data);
+            H->data = nullptr;
+        }
+        return nullptr;
+    }
+    return H;
+}
+
+// The recurrence of column tile t in the chained form (sums as batch_enqueue's).
+void batch_enqueue_chain(kpmx_batch* b, const ChainHolder& H, int64_t steps, int64_t t = 0) {
+    kpmx_ctx* ctx = b->ctx;
+    const size_t sb = scalar_bytes(b->scalar);
+    const char* r0 = static_cast<const char*>(b->r0) + (size_t)t * b->n_pad * b->vw * sb;
+    double* sums = b->sums + (size_t)t * steps * b->num_sys * 4 * b->vw;
+    const ChainBuffers B{{{b->w0, b->w1}, {b->w2, b->w3}}, b->chain_partials, b->chain_partials_bytes};
+    run_chain(ctx, batch_chain_matrix(b), H.plan, H.cols, r0, b->vw, std::min<int64_t>(b->tile_cols, b->nvec - t * b->tile_cols),
+              steps, H.systems, b->num_sys, sums, B);
+}
+
 // All steps in one persistent launch (launch_batched_persistent), then a check of its barrier.
 void batch_run_persistent(kpmx_batch* b, int64_t steps) {
     kpmx_ctx* ctx = b->ctx;
@@ -3143,16 +3283,23 @@ int kpmx_batch_run(kpmx_batch* b, int64_t M, int use_graph) {
             batch_run_persistent(b, steps);
             return;
         }
+        const ChainHolder* chain = batch_chain(b, steps);
+        auto enqueue = [&] {
+            for (int64_t t = 0; t < b->ntiles; ++t) {
+                if (chain) batch_enqueue_chain(b, *chain, steps, t);
+                else batch_enqueue(b, steps, t);
+            }
+        };
         if (!use_graph) {
-            for (int64_t t = 0; t < b->ntiles; ++t) batch_enqueue(b, steps, t);
+            enqueue();
             KPMX_HIP(hipGetLastError());
             return;
         }
-        if (b->graph_moments != M || !b->graph_exec) {
+        if (b->graph_moments != M || !b->graph_exec || b->graph_chain != (chain != nullptr)) {
             b->drop_graph();
             KPMX_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
             try {
-                for (int64_t t = 0; t < b->ntiles; ++t) batch_enqueue(b, steps, t);
+                enqueue();
             } catch (...) {
                 hipGraph_t g = nullptr;
                 (void)hipStreamEndCapture(ctx->stream, &g);
@@ -3162,6 +3309,7 @@ int kpmx_batch_run(kpmx_batch* b, int64_t M, int use_graph) {
             KPMX_HIP(hipStreamEndCapture(ctx->stream, &b->graph));
             KPMX_HIP(hipGraphInstantiate(&b->graph_exec, b->graph, nullptr, nullptr, 0));
             b->graph_moments = M;
+            b->graph_chain = chain != nullptr;
         }
         KPMX_HIP(hipGraphLaunch(b->graph_exec, ctx->stream));
     });
@@ -3175,6 +3323,7 @@ int kpmx_batch_set_partition(kpmx_batch* b, int num_workgroups, int walk_chunk) 
                      "the XCD-aware walk needs a multiple of 8 workgroups");
         KPMX_HIP(hipSetDevice(b->ctx->device));
         batch_partition(b, num_workgroups, walk_chunk);
+        b->chain_on = false;
     });
 }
 
@@ -3287,6 +3436,21 @@ int kpmx_batch_autotune(kpmx_batch* b, int* num_workgroups, int* walk_chunk) {
             batch_partition(b, cand[best].first, cand[best].second);
         if (walk_chunk) *walk_chunk = b->walk_chunk;
         if (num_workgroups) *num_workgroups = b->num_wg;
+        // the chained form against the best partition
+        b->chain_on = true;
+        if (const ChainHolder* chain = batch_chain(b, 1 << 16)) {
+            float ms_c = 0;
+            for (int rep = 0; rep < 3; ++rep) {
+                KPMX_HIP(hipEventRecord(ctx->t0, ctx->stream));
+                batch_enqueue_chain(b, *chain, steps);
+                KPMX_HIP(hipEventRecord(ctx->t1, ctx->stream));
+                KPMX_HIP(hipEventSynchronize(ctx->t1));
+                float ms = 0;
+                KPMX_HIP(hipEventElapsedTime(&ms, ctx->t0, ctx->t1));
+                if (rep == 1 || (rep > 1 && ms < ms_c)) ms_c = ms;
+            }
+            b->chain_on = ms_c <= best_ms;
+        }
     });
 }
 

@@ -26,9 +26,10 @@ struct ChainMatrix {
     const void* vals = nullptr;      // standard form
     const uint8_t* codes = nullptr;  // value-table form
     const void* diag = nullptr;
-    const void* table = nullptr;
+    const void* table = nullptr;     // zero first; several systems' tables one after another
     int table_size = 0;
-    int form() const { return !codes ? CHAIN_STD : table_size <= 2 ? CHAIN_UNIFORM : CHAIN_TABLE; }
+    int table_most = 0;              // entries of the largest of them
+    int form() const { return !codes ? CHAIN_STD : table_most <= 2 ? CHAIN_UNIFORM : CHAIN_TABLE; }
 };
 
 // Device arrays of a plan.  Tile t owns rows [tile_begin[t], tile_begin[t + 1]); its local rows are
@@ -45,6 +46,7 @@ struct ChainPlan {
     int row_items = 1;  // items of a row
     int64_t ext_stride = 0;
     int32_t* tile_begin = nullptr;
+    int32_t* tile_table = nullptr;  // first entry of the tile's value table (null: 0)
     int32_t* ring = nullptr;
     int32_t* ext = nullptr;
     ushort4* lidx = nullptr;    // [tile][group][row], first item of the column's local row (none: the zero row)

@@ -190,6 +190,7 @@ struct ChainArgs {
     const value* vals;
     const value* diag;
     const value* table;
+    const int32_t* tile_table;  // first table entry of every tile (null: 0)
     int table_size;
     int groups, rows_x, rows_y;
     int64_t ntiles;
@@ -316,8 +317,9 @@ void k_chain(ChainArgs<E> a) {
             if (tid < nx - (I0 + u) * THREADS) X[tid + (I0 + u) * THREADS] = xv[u];
         });
     });
+    const int first_value = FORM != CHAIN_STD && a.tile_table ? a.tile_table[t] : 0;
     if constexpr (FORM == CHAIN_TABLE)
-        if (tid < a.table_size) tab[tid] = a.table[tid];
+        if (tid < 256 && first_value + tid < a.table_size) tab[tid] = a.table[first_value + tid];
     if (tid < EW) X[a.rows_x * EW + tid] = make_zero<E>();
     if (tid <= a.steps) rings[tid] = rg[tid];
     const ushort4* lidx = a.lidx + t * a.groups * a.rows_y;
@@ -343,7 +345,7 @@ void k_chain(ChainArgs<E> a) {
         }
     V uniform = zero(V{});
     if constexpr (FORM == CHAIN_UNIFORM)
-        if (a.table_size > 1) uniform = a.table[1];
+        if (first_value + 1 < a.table_size) uniform = a.table[first_value + 1];
     __syncthreads();
 
     // the tile's sums of step j, added up in wave order by one wave while the others go on
@@ -509,6 +511,7 @@ int launch_form(const ChainLaunch& L, hipStream_t s) {
     a.vals = static_cast<const V*>(P.vals);
     a.diag = static_cast<const V*>(P.diag);
     a.table = static_cast<const V*>(L.m.table);
+    a.tile_table = P.tile_table;
     a.table_size = L.m.table_size;
     a.groups = P.groups;
     a.rows_x = P.rows_x;

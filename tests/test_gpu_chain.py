@@ -142,3 +142,35 @@ def test_repeats_and_graph_replays_are_bitwise():
             other.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128])
+@pytest.mark.parametrize("form", ["uniform", "table", "stored"])
+@pytest.mark.parametrize("nvec", [1, 2, 3, 4, 10])
+def test_batches(oracle, dtype, form, nvec):
+    """systems of 2 to 4140 sites in one batch, each with its own hopping values: the chained form
+    (graph and stream launches) against the oracle and the walkers (a pinned partition)"""
+    h2s = [lattice(form, n1, n2, dtype=dtype) * dtype(f) for n1, n2, f in
+           ((1, 1, 1), (4, 2, 0.9), (8, 4, 0.8), (11, 3, 0.7), (19, 17, 1), (46, 45, 0.6))]
+    r0 = [starters(h.shape[0], nvec, dtype, seed=i) for i, h in enumerate(h2s)]
+    M = 130
+    print("chain batch", np.dtype(dtype).name, form, nvec, flush=True)
+    ctx = abi.Ctx(0)
+    try:
+        b = abi.Batch(ctx, h2s)
+        b.starters(np.concatenate(r0, axis=1))
+        out = {}
+        for mode in (False, True, True):
+            b.run(M, mode)
+            out.setdefault("chain", b.fetch(M))
+            assert np.array_equal(b.fetch(M), out["chain"])
+        b.set_partition(64)
+        b.run(M, False)
+        out["walkers"] = b.fetch(M)
+    finally:
+        ctx.close()
+    for s, (h, r) in enumerate(zip(h2s, r0)):
+        ref = oracle.diag_moments(h, r, M)
+        scale = np.abs(ref[:, :1])
+        assert np.max(np.abs(out["chain"][s] - ref) / scale) <= TOL[dtype], s
+        assert np.max(np.abs(out["chain"][s] - out["walkers"][s]) / scale) <= 2 * TOL[dtype], s
