@@ -633,7 +633,7 @@ def main():
         w, c = (int(x) for x in args.two_step.split(":"))
         ctx.set_tile_width(dtype, w)
         ctx.set_two_step_lds(c)
-    steps_per_launch, tile_width = abi.diagonal_form(mat, blk, M)
+    steps_per_launch, tile_width = abi.diagonal_form(mat, R, M)
     two_step, two_step_wg = ctx.two_step_lds(dtype)
     chained = steps_per_launch > 2 or (steps_per_launch == 2 and not two_step)
     two_step = two_step and not chained

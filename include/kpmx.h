@@ -127,11 +127,11 @@ int kpmx_block_destroy(kpmx_block* b);
  * rounding. */
 int kpmx_moments_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, void* mu);
 
-/* The form kpmx_moments_diagonal takes for these arguments (no counterpart in the reference; its
- * plans are built if they are not there): steps_per_launch 1 (single steps), 2 (a two-step form) or
+/* The form kpmx_moments_diagonal takes for a block of num_vectors vectors (no counterpart in the
+ * reference; its plans are built if they are not there): steps_per_launch 1 (single steps), 2 (a two-step form) or
  * more (the chained form's launches; the last of a run may do fewer), and columns, the vectors of
  * one launch of the block's widest starter tile. */
-int kpmx_diagonal_form(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, int* steps_per_launch,
+int kpmx_diagonal_form(const kpmx_mat* h2, int64_t num_vectors, int64_t num_moments, int* steps_per_launch,
                        int* columns);
 
 /* Autotuner (no counterpart in the reference, whose CPU kernels have one fixed shape): time the

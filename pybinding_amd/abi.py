@@ -220,11 +220,12 @@ def moments_diagonal_noalloc(mat, block, num_moments):
     return out
 
 
-def diagonal_form(mat, block, num_moments):
+def diagonal_form(mat, num_vectors, num_moments):
     """(steps per launch, vectors per launch) of the form the diagonal recurrence takes
     (kpmx_diagonal_form)."""
     k, w = ctypes.c_int(), ctypes.c_int()
-    _check(lib().kpmx_diagonal_form(mat.h, block.h, ctypes.c_int64(num_moments), ctypes.byref(k), ctypes.byref(w)))
+    _check(lib().kpmx_diagonal_form(mat.h, ctypes.c_int64(num_vectors), ctypes.c_int64(num_moments), ctypes.byref(k),
+                                    ctypes.byref(w)))
     return k.value, w.value
 
 

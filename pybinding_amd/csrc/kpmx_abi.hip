@@ -429,6 +429,21 @@ int pick_vw(int64_t remaining) {
     return vw;
 }
 
+// The starter tiles of a block of num_vectors vectors (without data): 64 wide, the last one the next
+// power of two.
+std::vector<Tile> starter_tiles(int64_t num_vectors) {
+    std::vector<Tile> tiles;
+    for (int64_t c0 = 0; c0 < num_vectors;) {
+        Tile t;
+        t.c0 = c0;
+        t.vw = pick_vw(num_vectors - c0);
+        t.cols = std::min<int64_t>(t.vw, num_vectors - c0);
+        tiles.push_back(t);
+        c0 += t.cols;
+    }
+    return tiles;
+}
+
 int grid_size(kpmx_ctx* ctx, int64_t num_tiles) {
     int64_t max_wg = (int64_t)ctx->num_cu * 8;
     int64_t g = std::min<int64_t>(num_tiles, max_wg);
@@ -1227,7 +1242,7 @@ void run_chain(kpmx_ctx* ctx, const ChainMatrix& m, const ChainPlan& P, int cols
             KPMX_HIP(hipGetLastError());
             const int64_t done = k + L.steps;
             if (done - chunk_start == chunk || done == steps) {
-                launch_chain_reduce(m.scalar, B.partials, P.ntiles, cols, done - chunk_start, system_tiles, num_systems, vw,
+                launch_chain_reduce(m.scalar, CHAIN_SUMS, B.partials, P.ntiles, cols, done - chunk_start, system_tiles, num_systems, vw,
                                     (int)c0, sums + chunk_start * num_systems * 4 * vw, ctx->stream);
                 KPMX_HIP(hipGetLastError());
                 chunk_start = done;
@@ -1258,10 +1273,10 @@ struct RunTile {
     bool copy = false;  // sub-tile: columns [c, c + sub.vw) copied to work2 first
     Tile sub;
 };
-std::vector<RunTile> run_tiles(const kpmx_block* r0, int cap) {
+std::vector<RunTile> run_tiles(const std::vector<Tile>& tiles, int cap) {
     std::vector<RunTile> out;
-    for (size_t i = 0; i < r0->tiles.size(); ++i) {
-        const Tile& t = r0->tiles[i];
+    for (size_t i = 0; i < tiles.size(); ++i) {
+        const Tile& t = tiles[i];
         if (t.vw <= cap) {
             out.push_back({i, 0, false, t});
             continue;
@@ -1277,6 +1292,7 @@ std::vector<RunTile> run_tiles(const kpmx_block* r0, int cap) {
     }
     return out;
 }
+std::vector<RunTile> run_tiles(const kpmx_block* r0, int cap) { return run_tiles(r0->tiles, cap); }
 int diag_cap(const kpmx_mat* h2) { return h2->ctx->tile_cap[h2->scalar]; }
 
 // Whether the diagonal recurrence of this block runs in the chained form: by default on SELL matrices
@@ -1285,19 +1301,58 @@ int diag_cap(const kpmx_mat* h2) { return h2->ctx->tile_cap[h2->scalar]; }
 // use and halves the recurrence at least on launch-bound systems, so runs whose single steps are
 // expected to take less than 0.4 ms in all keep those (whatever was run before: the same call always
 // takes the same form).  existing: only with plans that are there already (nothing is allocated).
-bool use_chain(const kpmx_mat* h2, const kpmx_block* r0, int64_t steps, bool existing = false) {
+bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps, bool existing = false) {
     const kpmx_ctx* ctx = h2->ctx;
     if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return false;
+    const auto rts = run_tiles(tiles, diag_cap(h2));
     double single_us = 0;
-    for (const RunTile& rt : run_tiles(r0, diag_cap(h2)))
+    for (const RunTile& rt : rts)
         single_us += std::max(5.5, 3.0 * h2->rows * rt.sub.vw * scalar_bytes(h2->scalar) / 5.6e6);
     if (single_us * steps < 400) return false;
     if (ctx->two_step[h2->scalar] > 0 && !existing)
-        for (const RunTile& rt : run_tiles(r0, diag_cap(h2)))
+        for (const RunTile& rt : rts)
             if (use_two_step(h2, rt.sub)) return false;
-    for (const Tile& t : r0->tiles)
+    for (const Tile& t : tiles)
         if (!chain_plan(h2, chain_cols(h2, t), existing)) return false;
     return true;
+}
+
+// The plan of a one-vector recurrence that collects something else than the diagonal sums, under the
+// same conditions (null: single steps).
+const ChainPlan* chain_single(const kpmx_mat* h2, int64_t steps) {
+    const kpmx_ctx* ctx = h2->ctx;
+    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return nullptr;
+    if (std::max(5.5, 3.0 * h2->rows * scalar_bytes(h2->scalar) / 5.6e6) * steps < 400) return nullptr;
+    return chain_plan(h2, 1);
+}
+
+// The chained recurrence of `cols` columns of a block (rows of ldx scalars) over `steps` steps, for
+// collections other than the diagonal sums: per_launch(L, k) sets what the launch of steps
+// r_{k+1} ... r_{k+L.steps} leaves, after_launch(L, k) may use its L.out2 = r_{k+L.steps}.
+template <class PerLaunch, class AfterLaunch>
+void chain_steps(const kpmx_mat* h2, const ChainPlan& P, int cols, const void* x, int64_t ldx, int64_t steps,
+                 PerLaunch per_launch, AfterLaunch after_launch) {
+    kpmx_ctx* ctx = h2->ctx;
+    const size_t blk = (size_t)h2->rows * cols * scalar_bytes(h2->scalar);
+    void* w[2][2] = {{ctx->work0.get(blk), ctx->work1.get(blk)}, {ctx->work3.get(blk), ctx->work4.get(blk)}};
+    ChainLaunch L;
+    L.m = chain_matrix(h2);
+    L.plan = &P;
+    L.cols = cols;
+    int turn = 0;
+    for (int64_t k = 0; k < steps; k += L.steps, turn ^= 1) {
+        L.steps = (int)std::min<int64_t>(P.steps, steps - k);
+        L.first = k == 0;
+        L.x = k == 0 ? x : w[turn ^ 1][1];
+        L.ldx = k == 0 ? ldx : cols;
+        L.xprev = k == 0 ? nullptr : w[turn ^ 1][0];
+        L.out1 = w[turn][0];
+        L.out2 = w[turn][1];
+        per_launch(L, k);
+        if (launch_chain(L, ctx->stream) != 0) throw Error{KPMX_EINVAL, "unsupported chained recurrence"};
+        KPMX_HIP(hipGetLastError());
+        after_launch(L, k);
+    }
 }
 
 // copies a sub-tile's columns into `dst` (default: work2, sized beforehand) and returns the tile
@@ -1345,7 +1400,7 @@ void diag_run(const kpmx_mat* h2, const kpmx_block* r0c, int64_t M) {
     KPMX_REQUIRE(M >= 2 && M % 2 == 0, "num_moments must be even and >= 2");
     kpmx_ctx* ctx = h2->ctx;
     const int64_t steps = M / 2;
-    bool chain = use_chain(h2, r0, steps);
+    bool chain = use_chain(h2, r0->tiles, steps);
     if (chain) {
         try {
             for (const Tile& t : r0->tiles) size_chain(h2, t, steps);
@@ -1911,16 +1966,11 @@ int kpmx_block_upload(kpmx_ctx* ctx, int scalar, int64_t n, int64_t num_vectors,
         b->nvec = num_vectors;
         void* staging = ctx->aux0.get((size_t)n * num_vectors * sb);
         KPMX_HIP(hipMemcpyAsync(staging, r0, (size_t)n * num_vectors * sb, hipMemcpyHostToDevice, ctx->stream));
-        for (int64_t c0 = 0; c0 < num_vectors;) {
-            Tile t;
-            t.c0 = c0;
-            t.vw = pick_vw(num_vectors - c0);
-            t.cols = std::min<int64_t>(t.vw, num_vectors - c0);
+        for (Tile t : starter_tiles(num_vectors)) {
             t.data = dev_alloc((size_t)n * t.vw * sb);
             b->tiles.push_back(t);
             launch_gather_block(scalar, staging, n, t.c0, t.cols, t.vw, t.data, ctx->stream);
             KPMX_HIP(hipGetLastError());
-            c0 += t.cols;
         }
         KPMX_HIP(hipStreamSynchronize(ctx->stream));
         *out = b.release();
@@ -2014,20 +2064,19 @@ int kpmx_ctx_set_graph_policy(kpmx_ctx* ctx, int policy) {
     });
 }
 
-int kpmx_diagonal_form(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, int* steps_per_launch,
-                       int* columns) {
+int kpmx_diagonal_form(const kpmx_mat* h2, int64_t num_vectors, int64_t num_moments, int* steps_per_launch, int* columns) {
     return guarded([&] {
-        check_pair(h2, r0);
-        KPMX_REQUIRE(steps_per_launch && columns, "null argument");
+        KPMX_REQUIRE(h2 && steps_per_launch && columns, "null argument");
+        KPMX_REQUIRE(num_vectors >= 1, "num_vectors must be positive");
         KPMX_REQUIRE(num_moments >= 2 && num_moments % 2 == 0, "num_moments must be even and >= 2");
         KPMX_HIP(hipSetDevice(h2->ctx->device));
-        const Tile& t = r0->tiles.front();
-        if (use_chain(h2, r0, num_moments / 2)) {
-            *columns = chain_cols(h2, t);
+        const auto tiles = starter_tiles(num_vectors);
+        if (use_chain(h2, tiles, num_moments / 2)) {
+            *columns = chain_cols(h2, tiles.front());
             *steps_per_launch = chain_plan(h2, *columns)->steps;
             return;
         }
-        const Tile sub = run_tiles(r0, diag_cap(h2)).front().sub;
+        const Tile sub = run_tiles(tiles, diag_cap(h2)).front().sub;
         *columns = sub.vw;
         *steps_per_launch = use_two_step(h2, sub) ? 2 : 1;
     });
@@ -2112,7 +2161,7 @@ int kpmx_moments_diagonal_noalloc(const kpmx_mat* h2, const kpmx_block* r0, int6
         const int64_t steps = M / 2;
         const size_t sb = scalar_bytes(h2->scalar);
         auto align = [](size_t b) { return (b + 255) / 256 * 256; };
-        if (use_chain(h2, r0, steps, true) && chain_noalloc(h2, r0, M, mu)) return;
+        if (use_chain(h2, r0->tiles, steps, true) && chain_noalloc(h2, r0, M, mu)) return;
         // the same column tiles as kpmx_moments_diagonal (sub-tiles of wide starter tiles)
         const auto rts = run_tiles(r0, diag_cap(h2));
         int vw_max = 1;
@@ -2171,6 +2220,8 @@ int kpmx_moments_generic(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, co
         const int64_t n = h2->rows;
         const bool cplx = is_complex(h2->scalar);
         const size_t sb = scalar_bytes(h2->scalar);
+        const int64_t steps = M - 1;
+        const ChainPlan* P = chain_single(h2, steps);  // before the workspaces: a new plan uses them
         // w = op^H beta (host), uploaded once
         std::vector<char> wbuf((size_t)n * sb);
         if (h2->scalar == 0 || h2->scalar == 2) {
@@ -2199,9 +2250,31 @@ int kpmx_moments_generic(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, co
             KPMX_HIP(hipGetLastError());
             t.data = tmp;
         }
-        const int64_t steps = M - 1;
         double* sums = static_cast<double*>(ctx->sums.get((size_t)steps * 4 * sizeof(double)));
-        run_recurrence(h2, t, MODE_DOT, steps, dw, sums, [](StepLaunch&, int64_t) {}, [](StepLaunch const&, int64_t) {});
+        if (P) {
+            const int64_t per_step = P->ntiles * chain_partial_width(h2->scalar, 1, CHAIN_DOTS);
+            // whole launches whose partial sums one reduction takes
+            const int64_t chunk = std::max<int64_t>(1, (int64_t)(CHAIN_PARTIALS / sizeof(double)) / per_step / P->steps) * P->steps;
+            double* partials = static_cast<double*>(
+                ctx->partials.get((size_t)std::min(chunk, steps + P->steps) * per_step * sizeof(double)));
+            int64_t start = 0;
+            chain_steps(h2, *P, 1, t.data, 1, steps,
+                        [&](ChainLaunch& L, int64_t k) {
+                            L.mode = CHAIN_DOTS;
+                            L.w = dw;
+                            L.partials = partials + (k - start) * per_step;
+                        },
+                        [&](const ChainLaunch& L, int64_t k) {
+                            const int64_t done = k + L.steps;
+                            if (done - start != chunk && done != steps) return;
+                            launch_chain_reduce(h2->scalar, CHAIN_DOTS, partials, P->ntiles, 1, done - start, nullptr, 1, 1, 0,
+                                                sums + start * 4, ctx->stream);
+                            KPMX_HIP(hipGetLastError());
+                            start = done;
+                        });
+        } else {
+            run_recurrence(h2, t, MODE_DOT, steps, dw, sums, [](StepLaunch&, int64_t) {}, [](StepLaunch const&, int64_t) {});
+        }
         std::vector<double> s((size_t)steps * 4);
         KPMX_HIP(hipMemcpyAsync(s.data(), sums, s.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         KPMX_HIP(hipStreamSynchronize(ctx->stream));
@@ -2226,6 +2299,7 @@ int kpmx_moments_multi_unit(const kpmx_mat* h2, const kpmx_block* r0, int64_t M,
         KPMX_HIP(hipSetDevice(ctx->device));
         const int64_t n = h2->rows;
         const size_t sb = scalar_bytes(h2->scalar);
+        const ChainPlan* P = chain_single(h2, M - 1);  // before the workspaces: a new plan uses them
         // unique destinations -> slots
         std::vector<int32_t> mark((size_t)n, -1);
         std::vector<int32_t> slot_of((size_t)ndest);
@@ -2259,11 +2333,22 @@ int kpmx_moments_multi_unit(const kpmx_mat* h2, const kpmx_block* r0, int64_t M,
             KPMX_HIP(hipGetLastError());
         }
         t.data = vec;
-        run_recurrence(h2, t, MODE_NONE, M - 1, nullptr, nullptr, [&](StepLaunch& L, int64_t k) {
-            L.mark = dmark;
-            L.mark_out = dmu + (size_t)(k + 1) * sb;
-            L.mark_stride = M;
-        }, [](StepLaunch const&, int64_t) {});
+        if (P) {
+            chain_steps(h2, *P, 1, t.data, 1, M - 1,
+                        [&](ChainLaunch& L, int64_t k) {
+                            L.mode = CHAIN_MARKS;
+                            L.mark = dmark;
+                            L.mark_out = dmu + (size_t)k * sb;
+                            L.mark_stride = M;
+                        },
+                        [](const ChainLaunch&, int64_t) {});
+        } else {
+            run_recurrence(h2, t, MODE_NONE, M - 1, nullptr, nullptr, [&](StepLaunch& L, int64_t k) {
+                L.mark = dmark;
+                L.mark_out = dmu + (size_t)(k + 1) * sb;
+                L.mark_stride = M;
+            }, [](StepLaunch const&, int64_t) {});
+        }
         std::vector<char> host((size_t)nu * M * sb);
         if (nu) KPMX_HIP(hipMemcpyAsync(host.data(), dmu, host.size(), hipMemcpyDeviceToHost, ctx->stream));
         std::vector<char> r0host((size_t)nu * sb);
@@ -2348,6 +2433,74 @@ int kpmx_moments_dense(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, cons
     });
 }
 
+namespace {
+// An operator's entries on the tiles of a plan, for one call.
+struct ChainOpHolder {
+    const ChainPlan* plan = nullptr;
+    ChainOp op;
+    char* data = nullptr;
+    ~ChainOpHolder() { dev_free(data); }
+};
+
+// The plan of panel sweeps with an operator applied in them (H.op), under the conditions of the
+// diagonal recurrence; null where the operator couples a tile to rows beyond its neighbours or memory
+// is short.
+const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, int64_t steps, ChainOpHolder& H) {
+    kpmx_ctx* ctx = h2->ctx;
+    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || op->format != KPMX_FMT_SELL ||
+        !h2->step_rows.empty())
+        return nullptr;
+    const size_t sb = scalar_bytes(h2->scalar);
+    if (2 * std::max(5.5, 3.0 * h2->rows * cols * sb / 5.6e6) * steps < 400) return nullptr;
+    const ChainPlan* P = chain_plan(h2, cols);
+    if (!P) return nullptr;
+    if (H.plan == P) return H.data ? P : nullptr;
+    KPMX_HIP(hipStreamSynchronize(ctx->stream));  // the last plan's launches read its entries
+    dev_free(H.data);
+    H.data = nullptr;
+    H.plan = P;
+    ChainMatrix m;
+    m.scalar = op->scalar;
+    m.n = op->rows;
+    m.max_width = op->max_width;
+    m.slice_ptr = op->slice_ptr;
+    m.slice_width = op->slice_width;
+    m.indices = op->sell_indices;
+    m.vals = op->sell_vals;
+    ChainOp o;
+    o.groups = std::max(1, (op->max_width + 3) / 4);
+    o.rows = (int)P->tile_rows;
+    const size_t cells = (size_t)P->ntiles * o.groups * o.rows;
+    const size_t lidx = (cells * sizeof(ushort4) + 255) / 256 * 256, vals = (cells * 4 * sb + 255) / 256 * 256;
+    try {
+        H.data = static_cast<char*>(dev_alloc(lidx + vals + sizeof(int32_t)));
+        for (Workspace* w : {&ctx->work0, &ctx->work1, &ctx->work3, &ctx->work4}) w->get((size_t)h2->rows * cols * sb);
+    } catch (const Error& e) {
+        if (e.code != KPMX_ENOMEM) throw;
+        dev_free(H.data);
+        H.data = nullptr;
+        return nullptr;
+    }
+    o.lidx = reinterpret_cast<ushort4*>(H.data);
+    o.vals = H.data + lidx;
+    int32_t* missing = reinterpret_cast<int32_t*>(H.data + lidx + vals);
+    launch_zero(KPMX_F32, missing, 1, ctx->stream);
+    KPMX_HIP(hipGetLastError());
+    KPMX_REQUIRE(chain_op_entries(m, *P, o, missing, ctx->stream) == 0, "no LDS for a chain plan");
+    KPMX_HIP(hipGetLastError());
+    int32_t bad = 0;
+    KPMX_HIP(hipMemcpyAsync(&bad, missing, sizeof(bad), hipMemcpyDeviceToHost, ctx->stream));
+    KPMX_HIP(hipStreamSynchronize(ctx->stream));
+    if (bad) {
+        dev_free(H.data);
+        H.data = nullptr;
+        return nullptr;
+    }
+    H.op = o;
+    return P;
+}
+}  // namespace
+
 int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr, const kpmx_block* r0, int64_t M,
                       int mode, void* mu_nm) {
     return guarded([&] {
@@ -2386,6 +2539,7 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
         launch_zero_f64(C, M * M * cw, ctx->stream);
         KPMX_HIP(hipGetLastError());
 
+        ChainOpHolder vop;
         for (const Tile& full : r0->tiles) {
             int g = full.vw;
             while (g > 1 && 2.0 * g * panel1 > budget) g >>= 1;
@@ -2395,6 +2549,9 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
             if (split) g = std::min(g, 4);
             for (int64_t c0 = 0; c0 < full.cols; c0 += g) {
                 const int64_t cols = std::min<int64_t>(g, full.cols - c0);
+                // panels from the chained sweeps, in groups of its widest rows or single columns
+                const int pcols = g >= chain_max_cols(sc) ? chain_max_cols(sc) : 1;
+                const ChainPlan* chain = split ? nullptr : chain_panels(h2, vr, pcols, M - 1, vop);
                 // this group's starters r (n x g), and vl r (n x g)
                 void* Pr = ctx->aux0.get((size_t)n * g * sb);
                 if (g == full.vw) {
@@ -2438,7 +2595,17 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
                 else
                     launch_scatter_scaled(sc, L0, n, g, g, 0.5, Lpan, M * n, ctx->stream);
                 KPMX_HIP(hipGetLastError());
-                run_recurrence(
+                if (chain) {
+                    for (int q = 0; q < g; q += pcols)
+                        chain_steps(h2, *chain, pcols, static_cast<char*>(L0) + (size_t)q * sb, g, M - 1,
+                                    [&](ChainLaunch& L, int64_t k) {
+                                        L.mode = CHAIN_PANEL;
+                                        L.panel = Lpan + ((size_t)q * M + k) * n * sb;
+                                        L.panel_col = M * n;
+                                        L.panel_step = n;
+                                    },
+                                    [](const ChainLaunch&, int64_t) {});
+                } else run_recurrence(
                     h2, tl, MODE_NONE, M - 1, nullptr, nullptr,
                     [&](StepLaunch& L, int64_t k) {
                         if (split) {
@@ -2462,12 +2629,36 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
                     O.copy_split = Rsp;
                 else
                     O.copy_out = Rpan;
-                launch(O, ctx->stream);
+                if (!chain) launch(O, ctx->stream);
                 Tile tr;
                 tr.vw = g;
                 tr.cols = cols;
                 tr.data = Pr;
-                run_recurrence(
+                if (chain) {
+                    for (int q = 0; q < g; q += pcols) {
+                        // the chain leaves rows 0 ... M - 2, one launch on its last vector row M - 1
+                        StepLaunch F = base_launch(vr, pcols, true);
+                        F.mode = MODE_NONE;
+                        F.sub_y = 0;
+                        F.yout = nullptr;
+                        F.hscale = 1.0;
+                        F.copy_col_stride = M * n;
+                        F.copy_out = Rpan + ((size_t)q * M + M - 1) * n * sb;
+                        chain_steps(h2, *chain, pcols, static_cast<char*>(Pr) + (size_t)q * sb, g, M - 1,
+                                    [&](ChainLaunch& L, int64_t k) {
+                                        L.mode = CHAIN_PANEL_OP;
+                                        L.op = &vop.op;
+                                        L.panel = Rpan + ((size_t)q * M + k) * n * sb;
+                                        L.panel_col = M * n;
+                                        L.panel_step = n;
+                                    },
+                                    [&](const ChainLaunch& L, int64_t k) {
+                                        if (k + L.steps < M - 1) return;
+                                        F.x = L.out2;
+                                        launch(F, ctx->stream);
+                                    });
+                    }
+                } else run_recurrence(
                     h2, tr, MODE_NONE, M - 1, nullptr, nullptr, [](StepLaunch&, int64_t) {},
                     [&](StepLaunch const& L, int64_t k) {
                         O.x = L.yout;
@@ -2707,7 +2898,7 @@ void autotune_chain(const kpmx_mat* h2, const kpmx_block* r0, double best_per_ve
     if (ctx->two_step[h2->scalar] > 0 && !ctx->two_step_auto[h2->scalar]) return;  // the caller's
     const int two_step = ctx->two_step[h2->scalar];
     ctx->two_step[h2->scalar] = 0;
-    const bool chain = use_chain(h2, r0, 1 << 20);
+    const bool chain = use_chain(h2, r0->tiles, 1 << 20);
     ctx->two_step[h2->scalar] = two_step;
     if (!chain) return;
     Tile t = r0->tiles.front();

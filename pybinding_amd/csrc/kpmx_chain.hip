@@ -194,7 +194,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void k_chain_entries(ChainMatrix m, c
 // Sums over the tiles of each system, tiles in order inside 32 interleaved groups.
 __global__ __launch_bounds__(1024) void k_chain_reduce(const double* partials, int64_t ntiles, int width, int cols,
                                                        const int32_t* system_tiles, int64_t num_systems, int ncol,
-                                                       int vw, int c0, double* sums) {
+                                                       int kinds, int vw, int c0, double* sums) {
     __shared__ double red[1024];
     const int64_t step = blockIdx.x / num_systems, sys = blockIdx.x % num_systems;
     const int64_t t0 = system_tiles ? system_tiles[sys] : 0, t1 = system_tiles ? system_tiles[sys + 1] : ntiles;
@@ -208,11 +208,60 @@ __global__ __launch_bounds__(1024) void k_chain_reduce(const double* partials, i
         for (int q = 1; q < ng; ++q) v += red[q * width + w];
         // item layout [kind][column of the element][element] -> [kind][column]
         const int ew = cols / ncol, e = w % ew, kc = w / ew, kind = kc / ncol, col = e * ncol + kc % ncol;
-        const int slot = kind == 0 ? 0 : kind + 1;
+        const int slot = kind == 0 || kinds == 4 ? kind : kind + 1;
         double* o = sums + (step * num_systems + sys) * 4 * vw + c0;
         o[slot * vw + col] = v;
-        if (kind == 0) o[vw + col] = 0.0;
-        if (kind == 1 && width == 2 * cols) o[3 * vw + col] = 0.0;
+        if (kind == 0 && kinds < 4) o[vw + col] = 0.0;
+        if (kind == 1 && kinds == 2) o[3 * vw + col] = 0.0;
+    }
+}
+
+// Operator entries on the own rows of every tile (see k_chain_entries): local columns and values.
+template <class V>
+__global__ __launch_bounds__(PLAN_THREADS) void k_chain_op(ChainMatrix m, const int32_t* tile_begin, const int32_t* ring,
+                                                           const int32_t* ext, int64_t ext_stride, int bits, int zero_item,
+                                                           int ew, ChainOp o, int32_t* missing) {
+    extern __shared__ __align__(16) char smem[];
+    RowSet set{reinterpret_cast<int32_t*>(smem), bits};
+    uint16_t* place = reinterpret_cast<uint16_t*>(set.keys + (1 << bits));
+    const int64_t t = blockIdx.x, r0 = tile_begin[t];
+    const int own = (int)(tile_begin[t + 1] - r0);
+    const int32_t* halo = ext + t * ext_stride;
+    const int near = ring[t * (CHAIN_MAX_STEPS + 1) + 1];  // rows that hold r_k at every step
+    set.clear();
+    __syncthreads();
+    for (int i = threadIdx.x; i < near - own; i += PLAN_THREADS) {
+        unsigned h = set.slot(halo[i]);
+        while (atomicCAS(&set.keys[h], -1, halo[i]) != -1) h = set.next(h);  // fewer rows than slots
+        place[h] = (uint16_t)((own + i) * ew);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < o.rows; i += PLAN_THREADS) {
+        const int64_t row = i < own ? r0 + i : r0;
+        const int64_t sl = row >> 6, base = m.slice_ptr[sl] + (row & 63);
+        const int w = i < own ? m.slice_width[sl] : 0;
+        for (int g = 0; g < o.groups; ++g) {
+            uint16_t id[4];
+            for (int q = 0; q < 4; ++q) {
+                const int k = 4 * g + q;
+                id[q] = (uint16_t)zero_item;
+                V v = zero(V{});
+                if (k < w) {
+                    const int32_t c = m.indices[base + (int64_t)k * 64];
+                    v = static_cast<const V*>(m.vals)[base + (int64_t)k * 64];
+                    if (c >= r0 && c < r0 + own) {
+                        id[q] = (uint16_t)((c - r0) * ew);
+                    } else {
+                        unsigned h = set.slot(c);
+                        while (set.keys[h] != c && set.keys[h] != -1) h = set.next(h);
+                        if (set.keys[h] == c) id[q] = place[h];
+                        else *missing = 1;
+                    }
+                }
+                static_cast<V*>(o.vals)[(t * (4 * o.groups) + k) * o.rows + i] = v;
+            }
+            o.lidx[(t * o.groups + g) * o.rows + i] = make_ushort4(id[0], id[1], id[2], id[3]);
+        }
     }
 }
 
@@ -250,7 +299,8 @@ int chain_row_pad(const ChainMatrix& m, int cols) {
                       [](auto s, auto ew) { return decltype(s)::threads / decltype(ew)::value; });
 }
 
-int chain_partial_width(int scalar, int cols) {
+int chain_partial_width(int scalar, int cols, int mode) {
+    if (mode == CHAIN_DOTS) return scalar >= 2 ? 4 : 2;
     return with_shape(scalar, cols, CHAIN_STD, 1, [](auto s, auto ew) { return decltype(s)::NS * decltype(ew)::value; });
 }
 
@@ -265,12 +315,12 @@ int launch_chain(const ChainLaunch& L, hipStream_t s) {
     }
 }
 
-void launch_chain_reduce(int scalar, const double* partials, int64_t ntiles, int cols, int64_t nsteps,
+void launch_chain_reduce(int scalar, int mode, const double* partials, int64_t ntiles, int cols, int64_t nsteps,
                          const int32_t* system_tiles, int64_t num_systems, int vw, int c0, double* sums, hipStream_t s) {
-    const int width = chain_partial_width(scalar, cols);
+    const int width = chain_partial_width(scalar, cols, mode);
     const int ncol = with_layout(scalar, cols, [](auto e, auto) { return elem<decltype(e)>::cols; });
     hipLaunchKernelGGL(k_chain_reduce, dim3((unsigned)(nsteps * num_systems)), dim3(1024), 0, s, partials, ntiles, width,
-                       cols, system_tiles, num_systems, ncol, vw, c0, sums);
+                       cols, system_tiles, num_systems, ncol, width / cols, vw, c0, sums);
 }
 
 int chain_sample(const ChainMatrix& m, const int* heights, int count, int capacity, int32_t* out, hipStream_t s) {
@@ -325,6 +375,27 @@ int chain_entries(const ChainMatrix& m, const ChainPlan& P, hipStream_t s) {
         case 1: return by_form(double{});
         case 2: return by_form(cf32{});
         default: return by_form(cf64{});
+    }
+}
+
+template <class V>
+static int op_entries_of(const ChainMatrix& op, const ChainPlan& P, const ChainOp& o, int32_t* missing, hipStream_t s) {
+    auto kernel = k_chain_op<V>;
+    const int bits = set_bits(std::max<int>(1, (int)P.ext_stride));
+    const size_t bytes = ((size_t)1 << bits) * (sizeof(int32_t) + sizeof(uint16_t));
+    static std::atomic<uint64_t> allowed{0};
+    if (!allow_lds(reinterpret_cast<const void*>(kernel), PLAN_LDS, allowed)) return -1;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)P.ntiles), dim3(PLAN_THREADS), bytes, s, op, P.tile_begin, P.ring, P.ext,
+                       P.ext_stride, bits, P.rows_x * P.row_items, P.row_items, o, missing);
+    return 0;
+}
+
+int chain_op_entries(const ChainMatrix& op, const ChainPlan& P, const ChainOp& o, int32_t* missing, hipStream_t s) {
+    switch (op.scalar) {
+        case 0: return op_entries_of<float>(op, P, o, missing, s);
+        case 1: return op_entries_of<double>(op, P, o, missing, s);
+        case 2: return op_entries_of<cf32>(op, P, o, missing, s);
+        default: return op_entries_of<cf64>(op, P, o, missing, s);
     }
 }
 

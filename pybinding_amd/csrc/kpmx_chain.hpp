@@ -65,7 +65,23 @@ int chain_rings(const ChainMatrix& m, const ChainPlan& P, int max_steps, hipStre
 // entry arrays of every tile (P.steps, rows_x, rows_y set and the arrays allocated)
 int chain_entries(const ChainMatrix& m, const ChainPlan& P, hipStream_t s);
 
+// What a step leaves beside the vectors: the diagonal sums, the dots with a weight vector, panel rows
+// of the new vector, panel rows of an operator applied to the vector before, or the new vector at
+// marked rows.
+enum { CHAIN_SUMS = 0, CHAIN_DOTS = 1, CHAIN_PANEL = 2, CHAIN_PANEL_OP = 3, CHAIN_MARKS = 4 };
+
+// An operator's entries on a plan's tiles (their own rows only).
+struct ChainOp {
+    int groups = 0, rows = 0;  // groups of four entries per row; row stride
+    ushort4* lidx = nullptr;
+    void* vals = nullptr;
+};
+// fills op (allocated for groups and rows) from the operator's SELL arrays (standard form); *missing
+// is set to 1 where an entry's column is no local row of its tile
+int chain_op_entries(const ChainMatrix& op, const ChainPlan& P, const ChainOp& o, int32_t* missing, hipStream_t s);
+
 struct ChainLaunch {
+    int mode = CHAIN_SUMS;
     ChainMatrix m;
     const ChainPlan* plan = nullptr;
     int cols = 8;              // vectors per row of the work blocks
@@ -76,7 +92,18 @@ struct ChainLaunch {
     const void* xprev = nullptr;  // r_{k-1}, rows of `cols` scalars (not read by a first launch)
     void* out1 = nullptr;         // r_{k+steps-1} (not written by a one-step launch)
     void* out2 = nullptr;         // r_{k+steps}
-    double* partials = nullptr;   // [steps][ntiles][chain_partial_width]
+    double* partials = nullptr;   // [steps][ntiles][chain_partial_width] (sums and dots)
+    const void* w = nullptr;      // dots (one column): n weights
+    // panels: column q of r_{k+j} (of the operator on r_{k+j-1}) goes to panel + q panel_col + p panel_step
+    // + row (scalars) with p = j (p = j - 1), step j = 1 ... steps; the operator's first row is halved
+    // in a first launch
+    void* panel = nullptr;
+    int64_t panel_col = 0, panel_step = 0;
+    const ChainOp* op = nullptr;
+    // marks (one column): r_{k+j} of row i goes to mark_out[mark[i] mark_stride + j] where mark[i] >= 0
+    const int32_t* mark = nullptr;
+    void* mark_out = nullptr;
+    int64_t mark_stride = 0;
 };
 // widest supported column tile of a scalar type
 int chain_max_cols(int scalar);
@@ -85,7 +112,7 @@ int chain_row_capacity(const ChainMatrix& m, int cols);
 // items of a row (see kpmx_chain_step.hpp); the row stride of the entry arrays is a multiple of pad
 int chain_row_items(int scalar, int cols);
 int chain_row_pad(const ChainMatrix& m, int cols);
-int chain_partial_width(int scalar, int cols);
+int chain_partial_width(int scalar, int cols, int mode = CHAIN_SUMS);
 int launch_chain(const ChainLaunch& L, hipStream_t s);
 int launch_chain_f32(const ChainLaunch& L, hipStream_t s);
 int launch_chain_f64(const ChainLaunch& L, hipStream_t s);
@@ -93,7 +120,7 @@ int launch_chain_c64(const ChainLaunch& L, hipStream_t s);
 int launch_chain_c128(const ChainLaunch& L, hipStream_t s);
 // sums[step][system][4 vw] of the columns [c0, c0 + cols) of a vw-column block from the partials of
 // nsteps steps; system_tiles (num_systems + 1) null: one system over all tiles
-void launch_chain_reduce(int scalar, const double* partials, int64_t ntiles, int cols, int64_t nsteps,
+void launch_chain_reduce(int scalar, int mode, const double* partials, int64_t ntiles, int cols, int64_t nsteps,
                          const int32_t* system_tiles, int64_t num_systems, int vw, int c0, double* sums, hipStream_t s);
 
 }  // namespace kpmx

@@ -145,6 +145,7 @@ template <class E, int EW, int FORM, bool FEW>
 struct shape {
     using V = typename elem<E>::value;
     static constexpr int NS = elem<E>::kinds * elem<E>::cols;  // sums of an element
+    static constexpr int sums = 2 * (elem<E>::kinds - 1) * elem<E>::cols;  // most of any collection
     // of few entries, rows of one small element keep them in registers, wider rows in LDS; longer
     // rows read them from L1 and L2 in every step
     static constexpr bool narrow = EW * sizeof(E) < 16;
@@ -159,7 +160,7 @@ struct shape {
     // LDS bytes of a local row's entries: local columns, codes, diagonal
     static constexpr size_t row_entries = narrow || !FEW ? 0 : 8 + (FORM == CHAIN_TABLE ? 4 : 0) + (FORM != CHAIN_STD ? sizeof(V) : 0);
     // LDS beside the rows: two buffers of per-wave sums, the zero row, the ring counts, the value table
-    static constexpr size_t fixed = 2 * waves * NS * EW * sizeof(double) + (EW * sizeof(E) + 31) / 16 * 16 + 64 +
+    static constexpr size_t fixed = 2 * waves * sums * EW * sizeof(double) + (EW * sizeof(E) + 31) / 16 * 16 + 64 +
                                     (FORM == CHAIN_TABLE ? 256 * sizeof(V) : 0);
     static constexpr int max_items = !FEW ? 8 : narrow ? 10 : 20;  // registers
     static constexpr int fit(int items) {  // rows that `items` items per thread leave LDS for
@@ -201,6 +202,16 @@ struct ChainArgs {
     E* out2;
     double* partials;
     int steps, first;
+    // the other collections (see ChainLaunch)
+    const E* w;
+    E* panel;
+    int64_t panel_col, panel_step;
+    const ushort4* op_lidx;
+    const value* op_vals;
+    int op_groups, op_rows;
+    const int32_t* mark;
+    E* mark_out;
+    int64_t mark_stride;
 };
 
 // p[i] with a uniform p: a scalar base and a 32-bit lane offset
@@ -211,6 +222,26 @@ __device__ __forceinline__ P& at(P* p, unsigned i) {
 }
 
 // v plus v of another lane of the same row of 16 (DPP)
+// the sums of <w| on one element: conj(w) x (real, imaginary part), then conj(w) y
+template <class T>
+__device__ __forceinline__ void add_dots(T w, T y, T x, double* s) {
+    constexpr int P = elem<T>::kinds == 3 ? 2 : 1;
+    const d2 a = cdot(w, x), b = cdot(w, y);
+    s[0] += a.re;
+    s[P] += b.re;
+    if constexpr (P == 2) {
+        s[1] += a.im;
+        s[3] += b.im;
+    }
+}
+
+// element of one column stored by the column (E of several columns: column i of the element)
+template <class E>
+__device__ __forceinline__ auto column_of(const E& e, int) { return e; }
+__device__ __forceinline__ double column_of(const dpair& e, int i) { return i ? e.b : e.a; }
+__device__ __forceinline__ float column_of(const fquad& e, int i) { return e.v[i]; }
+__device__ __forceinline__ cf32 column_of(const cpair& e, int i) { return e.v[i]; }
+
 template <int CTRL>
 __device__ __forceinline__ double dpp_add(double v) {
     union { double d; int i[2]; } a, b;
@@ -256,14 +287,17 @@ __device__ __forceinline__ void wave_sums(const double* s, double* red) {
     });
 }
 
-// W: entries per row (3 or 4 unrolled; 0: groups of four in a loop)
-template <class E, int EW, int FORM, int W>
+// W: entries per row (3 or 4 unrolled; 0: groups of four in a loop).  MODE: what a step leaves beside
+// the vectors (CHAIN_SUMS ... CHAIN_MARKS, see ChainLaunch).
+template <class E, int EW, int FORM, int W, int MODE>
 __global__ __launch_bounds__((shape<E, EW, FORM, (W > 0)>::threads), (shape<E, EW, FORM, (W > 0)>::waves_per_simd))
 void k_chain(ChainArgs<E> a) {
     using V = typename elem<E>::value;
     using real = typename elem<E>::real;
     using S = shape<E, EW, FORM, (W > 0)>;
-    constexpr int IT = S::items, NS = S::NS, THREADS = S::threads, WAVES = S::waves;
+    constexpr int IT = S::items, THREADS = S::threads, WAVES = S::waves;
+    constexpr bool SUMS = MODE == CHAIN_SUMS || MODE == CHAIN_DOTS;
+    constexpr int NS = MODE == CHAIN_DOTS ? 2 * (elem<E>::kinds - 1) : SUMS ? S::NS : 1;
     constexpr int LD = 2;  // items loaded together
     constexpr bool KEEP = W > 0 && S::narrow;  // entries in registers
     constexpr bool LDS_ENTRIES = W > 0 && !S::narrow;
@@ -272,7 +306,7 @@ void k_chain(ChainArgs<E> a) {
     char* lds = smem + (size_t)S::rows * EW * sizeof(E) + (EW * sizeof(E) + 15) / 16 * 16;
     lds = smem + ((lds - smem) + 15) / 16 * 16;
     double* red = reinterpret_cast<double*>(lds);
-    lds += 2 * WAVES * NS * EW * sizeof(double);
+    lds += 2 * WAVES * S::sums * EW * sizeof(double);
     int* rings = reinterpret_cast<int*>(lds);
     lds += 64;
     V* tab = reinterpret_cast<V*>(lds);
@@ -358,12 +392,21 @@ void k_chain(ChainArgs<E> a) {
         for (int w = 1; w < WAVES; ++w) v += rw[w * NS * EW];
         a.partials[((int64_t)(j - 1) * a.ntiles + t) * (NS * EW) + i] = v;
     };
+    // row `row` (of thread 0) of the panel's step p, every column of the element to its own panel
+    auto to_panel = [&](const E& e, int p, int row) {
+        using T = decltype(column_of(e, 0));
+        T* o = reinterpret_cast<T*>(a.panel) + p * a.panel_step + r0 + row + trow;
+        static_for<elem<E>::cols>([&](auto i) { o[(int64_t)(c * elem<E>::cols + i) * a.panel_col] = column_of(e, i); });
+    };
+    const ushort4* op_lidx = a.op_lidx + t * a.op_groups * a.op_rows;
+    const V* op_vals = a.op_vals + t * 4 * a.op_groups * a.op_rows;
     for (int j = 1; j <= a.steps; ++j) {
         unsigned again = 0;
         asm volatile("" : "+s"(again));
         const int act = __builtin_amdgcn_readfirstlane(rings[a.steps - j]) * EW;
         const real hs = (a.first && j == 1) ? real(0.5) : real(1);
-        if (j > 1) store_sums(j - 1);
+        if constexpr (SUMS)
+            if (j > 1) store_sums(j - 1);
         double s[NS] = {};
         static_for<IT>([&](auto item) {
             constexpr int it = decltype(item)::value;
@@ -428,9 +471,32 @@ void k_chain(ChainArgs<E> a) {
             if constexpr (FORM == CHAIN_UNIFORM) h = product(uniform, h);
             if constexpr (FORM != CHAIN_STD) h = fmac(d, xi, h);
             y[it] = sub(scal(h, hs), y[it]);
-            if (tid < nown - it * THREADS) add_sums(y[it], xi, s);
+            if constexpr (MODE == CHAIN_SUMS)
+                if (tid < nown - it * THREADS) add_sums(y[it], xi, s);
+            if constexpr (MODE == CHAIN_DOTS)
+                if (tid < nown - it * THREADS) add_dots(at(a.w + r0 + row + again, trow), y[it], xi, s);
+            if constexpr (MODE == CHAIN_PANEL)
+                if (tid < nown - it * THREADS) to_panel(y[it], j, row);
+            if constexpr (MODE == CHAIN_PANEL_OP)
+                if (tid < nown - it * THREADS) {
+                    E o = make_zero<E>();
+                    for (int g = 0; g < a.op_groups; ++g) {
+                        const unsigned q = (unsigned)(g * a.op_rows) + r;
+                        const ushort4 l = at(op_lidx + q, trow);
+                        const uint16_t id[4] = {l.x, l.y, l.z, l.w};
+                        static_for<4>([&](auto k) {
+                            o = fmac(at(op_vals + ((unsigned)((4 * g + k) * a.op_rows) + r), trow), Xc[id[k]], o);
+                        });
+                    }
+                    to_panel(scal(o, hs), j - 1, row);
+                }
+            if constexpr (MODE == CHAIN_MARKS)
+                if (tid < nown - it * THREADS) {
+                    const int m = at(a.mark + r0 + row + again, trow);
+                    if (m >= 0) a.mark_out[m * a.mark_stride + j] = y[it];
+                }
         });
-        wave_sums<NS, EW>(s, red + ((j & 1) * WAVES + tid / 64) * NS * EW);
+        if constexpr (SUMS) wave_sums<NS, EW>(s, red + ((j & 1) * WAVES + tid / 64) * NS * EW);
         __syncthreads();
         if (j == a.steps) break;
         static_for<IT>([&](auto it) {
@@ -442,7 +508,7 @@ void k_chain(ChainArgs<E> a) {
         });
         __syncthreads();
     }
-    store_sums(a.steps);
+    if constexpr (SUMS) store_sums(a.steps);
     static_for<IT>([&](auto it) {
         if (tid < nown - it * THREADS) {
             at(a.out2 + r0 * EW + it * THREADS, tid) = y[it];
@@ -497,7 +563,7 @@ inline bool allow_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& a
     return true;
 }
 
-template <class E, int EW, int FORM, int W>
+template <class E, int EW, int FORM, int W, int MODE>
 int launch_form(const ChainLaunch& L, hipStream_t s) {
     using V = typename elem<E>::value;
     const ChainPlan& P = *L.plan;
@@ -525,7 +591,20 @@ int launch_form(const ChainLaunch& L, hipStream_t s) {
     a.partials = L.partials;
     a.steps = L.steps;
     a.first = L.first;
-    auto kernel = k_chain<E, EW, FORM, W>;
+    a.w = static_cast<const E*>(L.w);
+    a.panel = static_cast<E*>(L.panel);
+    a.panel_col = L.panel_col;
+    a.panel_step = L.panel_step;
+    if (L.op) {
+        a.op_lidx = L.op->lidx;
+        a.op_vals = static_cast<const V*>(L.op->vals);
+        a.op_groups = L.op->groups;
+        a.op_rows = L.op->rows;
+    }
+    a.mark = L.mark;
+    a.mark_out = static_cast<E*>(L.mark_out);
+    a.mark_stride = L.mark_stride;
+    auto kernel = k_chain<E, EW, FORM, W, MODE>;
     static std::atomic<uint64_t> allowed{0};  // devices
     if (!allow_lds(reinterpret_cast<const void*>(kernel), LDS_BYTES, allowed)) return -1;
     const int64_t grid = (P.ntiles + 7) / 8 * 8;
@@ -533,20 +612,36 @@ int launch_form(const ChainLaunch& L, hipStream_t s) {
     return 0;
 }
 
-template <class E, int EW>
-int launch_elem(const ChainLaunch& L, hipStream_t s) {
+template <class E, int EW, int MODE>
+int launch_mode(const ChainLaunch& L, hipStream_t s) {
     const int w = L.plan->groups > 1 ? 0 : L.plan->width <= 3 ? 3 : 4;
     auto by_width = [&](auto form) {
         constexpr int F = decltype(form)::value;
-        if (w == 3) return launch_form<E, EW, F, 3>(L, s);
-        if (w == 4) return launch_form<E, EW, F, 4>(L, s);
-        return launch_form<E, EW, F, 0>(L, s);
+        if (w == 3) return launch_form<E, EW, F, 3, MODE>(L, s);
+        if (w == 4) return launch_form<E, EW, F, 4, MODE>(L, s);
+        return launch_form<E, EW, F, 0, MODE>(L, s);
     };
     switch (L.m.form()) {
         case CHAIN_STD: return by_width(std::integral_constant<int, CHAIN_STD>{});
         case CHAIN_TABLE: return by_width(std::integral_constant<int, CHAIN_TABLE>{});
         default: return by_width(std::integral_constant<int, CHAIN_UNIFORM>{});
     }
+}
+
+// the collections beside the diagonal sums exist for one column and, panels, for the widest rows
+template <class E, int EW>
+int launch_elem(const ChainLaunch& L, hipStream_t s) {
+    constexpr bool one = EW * elem<E>::cols == 1, widest = EW == 4;
+    if (L.mode == CHAIN_SUMS) return launch_mode<E, EW, CHAIN_SUMS>(L, s);
+    if constexpr (one) {
+        if (L.mode == CHAIN_DOTS) return launch_mode<E, EW, CHAIN_DOTS>(L, s);
+        if (L.mode == CHAIN_MARKS) return launch_mode<E, EW, CHAIN_MARKS>(L, s);
+    }
+    if constexpr (one || widest) {
+        if (L.mode == CHAIN_PANEL) return launch_mode<E, EW, CHAIN_PANEL>(L, s);
+        if (L.mode == CHAIN_PANEL_OP) return launch_mode<E, EW, CHAIN_PANEL_OP>(L, s);
+    }
+    return -1;
 }
 
 }  // namespace

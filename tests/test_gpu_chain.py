@@ -174,3 +174,66 @@ def test_batches(oracle, dtype, form, nvec):
         scale = np.abs(ref[:, :1])
         assert np.max(np.abs(out["chain"][s] - ref) / scale) <= TOL[dtype], s
         assert np.max(np.abs(out["chain"][s] - out["walkers"][s]) / scale) <= 2 * TOL[dtype], s
+
+
+def pinned(ctx, dtype):
+    ctx.set_tile_width(dtype, 64)  # turns the chained form off
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128, np.complex64])
+@pytest.mark.parametrize("form", ["uniform", "table", "stored"])
+def test_dots_and_marks(oracle, dtype, form):
+    """<beta|op T_n|alpha> and (T_n alpha)[dest] on one vector: against the oracle and single steps"""
+    h2 = lattice(form, dtype=dtype)
+    n, M = h2.shape[0], 163
+    rng = np.random.default_rng(2)
+    alpha = starters(n, 3, dtype)[1:2]
+    beta = rng.standard_normal(n).astype(dtype) * dtype(1 if np.dtype(dtype).kind != "c" else 1 + 0.5j)
+    op = sp.diags([rng.uniform(0.5, 1.5, n), rng.uniform(0.5, 1.5, n - 7)], [0, 7]).tocsr().astype(dtype)
+    dest = [0, 5, n - 1, n // 2, 5]
+    print("chain dots", np.dtype(dtype).name, form, flush=True)
+    ctx = abi.Ctx(0)
+    try:
+        mat, blk = ctx.mat(h2, fmt=1), ctx.block(alpha)
+        out = [(abi.moments_generic(mat, blk, M, beta, o), abi.moments_multi_unit(mat, blk, M, dest)) for o in (None, op)]
+        pinned(ctx, dtype)
+        single = [(abi.moments_generic(mat, blk, M, beta, o), abi.moments_multi_unit(mat, blk, M, dest)) for o in (None, op)]
+    finally:
+        ctx.close()
+    norm = np.linalg.norm(alpha) * np.linalg.norm(beta) * 2
+    for (mu, units), (mu1, units1), o in zip(out, single, (None, op)):
+        ref = oracle.offdiag_moments(h2, alpha[0], M, "generic", beta=beta, op=o)
+        assert np.max(np.abs(mu - ref)) <= TOL[dtype] * norm
+        assert np.max(np.abs(mu - mu1)) <= 2 * TOL[dtype] * norm
+        ref = oracle.offdiag_moments(h2, alpha[0], M, "multi_unit", dest=dest)
+        assert np.max(np.abs(units - ref)) <= TOL[dtype] * np.linalg.norm(alpha)
+        assert np.max(np.abs(units - units1)) <= 2 * TOL[dtype] * np.linalg.norm(alpha)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128, np.complex64])
+@pytest.mark.parametrize("nvec", [1, 2, 4, 9])
+def test_kubo_panels(dtype, nvec):
+    """the panels of the Kubo moments from chained sweeps (the right operator applied inside them) against
+    single steps, with operators of the Hamiltonian's pattern, of more neighbours than it has (outside the
+    first ring: single steps) and with longer rows"""
+    h2 = lattice("stored", 24, 20, dtype=dtype)
+    n, M = h2.shape[0], 90
+    x = np.random.default_rng(5).uniform(-1, 1, n)
+    v = h2.copy()
+    v.data = (h2.data * (np.repeat(x, np.diff(h2.indptr)) - x[h2.indices])).astype(dtype)
+    far = sp.csr_matrix((v @ v).astype(dtype))
+    local = (v + sp.diags(x).astype(dtype)).tocsr().astype(dtype)
+    for left, right in ((v, v), (v, far), (far, local)):
+        left.sort_indices()
+        right.sort_indices()
+        print("chain kubo", np.dtype(dtype).name, nvec, right.nnz, flush=True)
+        ctx = abi.Ctx(0)
+        try:
+            mat, vl, vr = ctx.mat(h2, fmt=1), ctx.mat(left, fmt=1), ctx.mat(right, fmt=1)
+            blk = ctx.block(starters(n, nvec, dtype))
+            mu = abi.kubo_moments(mat, vl, vr, blk, M)
+            pinned(ctx, dtype)
+            ref = abi.kubo_moments(mat, vl, vr, blk, M)
+        finally:
+            ctx.close()
+        assert np.max(np.abs(mu - ref)) <= 2 * TOL[dtype] * np.max(np.abs(ref))
