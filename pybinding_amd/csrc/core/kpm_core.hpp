@@ -234,8 +234,8 @@ public:
 
     idx_t size() const { return original->rows; }
 
-    // `whole_system`: the calculation never uses the slice map (DOS, moments, conductivity); the
-    // GPU then prefers `locality_order` (e.g. sites along a space-filling curve) when one is set,
+    // `whole_system`: the calculation does without the slice map (DOS, moments, conductivity, LDOS
+    // and Green's functions whose recurrence is faster without a light cone); the GPU then prefers `locality_order` (e.g. sites along a space-filling curve) when one is set,
     // because the moments do not depend on the site order and a compact order keeps the gathered
     // vector rows of a sweep in L2.  Otherwise the reference's BFS reorder is used.
     void optimize_for(Indices const& idx, Scale<> scale, bool whole_system = false) {
@@ -246,6 +246,11 @@ public:
                                              std::to_string(size()) + " sites");
         const bool loc = whole_system && is_reordered && !locality_order.empty();
         if (has_idx && original_idx == idx && loc == used_locality) return;
+        if (has_idx && loc && used_locality) {  // the same matrix, other sites
+            map_indices(idx);
+            original_idx = idx;
+            return;
+        }
         timer.tic();
         if (loc) create_ordered(idx, scale, locality_order);
         else if (is_reordered) create_reordered(idx, scale);
@@ -324,10 +329,14 @@ private:
         create_scaled(idx, s);
         reorder_map = order;
         h2 = reorder(h2);
+        map_indices(idx);
+        slice_map = SliceMap(h2.rows);
+    }
+
+    void map_indices(Indices const& idx) {
         optimized_idx = Indices();
         for (auto v : idx.src) optimized_idx.src.push_back(reorder_map[(size_t)v]);
         for (auto v : idx.dest) optimized_idx.dest.push_back(reorder_map[(size_t)v]);
-        slice_map = SliceMap(h2.rows);
     }
 
     void create_scaled(Indices const& idx, Scale<> s) {

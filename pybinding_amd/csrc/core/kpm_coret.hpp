@@ -79,12 +79,27 @@ public:
         return out;
     }
 
+    // Site order of an LDOS or Green's function recurrence of `vectors` vectors.  The light cone of the
+    // BFS order saves work, but pays a launch per step (4.7 us) and a reorder and upload per site; on
+    // the locality order the chained recurrence sweeps the whole system several steps per launch.
+    // Up to 2^21 vector elements such a step takes less than that launch (137 k sites: 0.9 us, 2.1 M
+    // sites: 4.8 us); beyond, in runs too short for a chain and where no chain fits, the cone stays.
+    void optimize_for_sites(Indices const& idx, Scale<> scale, idx_t vectors, idx_t M) {
+        if (!no_chain_ && !oh_.locality_order.empty() && cfg_.algorithm.reorder() && format() == KPMX_FMT_SELL &&
+            M >= 160 && oh_.size() * vectors <= idx_t(1) << 21) {
+            oh_.optimize_for(idx, scale, true);
+            if (compute_.several_steps(oh_, format(), std::min<idx_t>(vectors, 64), M)) return;
+            no_chain_ = true;
+        }
+        oh_.optimize_for(idx, scale);
+    }
+
     std::vector<double> ldos(std::vector<idx_t> const& idx, std::vector<double> const& energy, double broadening,
                              idx_t* cols_out) override {
         const auto scale = scaling_factors();
         const idx_t M = cfg_.kernel.required_num_moments(broadening / scale.a);
         const idx_t K = (idx_t)idx.size();
-        oh_.optimize_for(Indices(idx, idx), scale);
+        optimize_for_sites(Indices(idx, idx), scale, K, M);
         stats_.reset(M, oh_, cfg_.algorithm, K, cfg_.matrix_format);
         auto starter = unit_starter(oh_);
         BatchDiagonalMoments<T> m{M, K, false, {}};
@@ -127,7 +142,7 @@ public:
         if (cols.empty()) throw std::invalid_argument("KPM::calc_greens: no column indices given");
         const auto scale = scaling_factors();
         const idx_t M = cfg_.kernel.required_num_moments(broadening / scale.a);
-        oh_.optimize_for(Indices(row, cols), scale);
+        optimize_for_sites(Indices(row, cols), scale, 1, M);
         stats_.reset(M, oh_, cfg_.algorithm, 1, cfg_.matrix_format);
         if (oh_.optimized_idx.is_diagonal()) {
             DiagonalMoments<T> m{M, {}};
@@ -204,6 +219,7 @@ private:
     Config cfg_;
     OptimizedHamiltonian<T> oh_;
     HipCompute<T> compute_;
+    bool no_chain_ = false;  // the locality order has no chained recurrence
     int kubo_mode_ = KPMX_KUBO_FP64;
     Stats stats_;
     double min_ = 0, max_ = 0;

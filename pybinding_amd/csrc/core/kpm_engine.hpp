@@ -260,6 +260,15 @@ public:
         return h2_->m;
     }
 
+    // Whether diagonal recurrences of `num_vectors` vectors run several steps per launch on `oh`.
+    bool several_steps(OptimizedHamiltonian<T> const& oh, int format, idx_t num_vectors, idx_t num_moments) {
+        kpmx_mat* h2 = matrix(oh, format);
+        set_cone(h2, {});
+        int steps = 0, cols = 0;
+        check(kpmx_diagonal_form(h2, num_vectors, num_moments, &steps, &cols));
+        return steps > 1;
+    }
+
     // The light cone of the reference's optimal_size algorithm: rows computed by every step of
     // a recurrence of `num_moments` moments (calc_moments.hpp:35-51,102-114); step k of the device
     // recurrence is the reference's iteration k + 1.  Empty: whole matrix.
