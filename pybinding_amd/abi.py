@@ -186,6 +186,14 @@ class Mat(_Handle):
         self._ctx = ctx
         self._own(ctx)
 
+    def set_row_order(self, order):
+        """Locality order of the rows for the chained recurrences' tiles: order[i] = position of row i, or
+        None (kpmx_mat_set_row_order)."""
+        q = None if order is None else np.ascontiguousarray(order, dtype=np.int32)
+        if q is not None and q.shape != (self.n,):
+            raise ValueError("the row order has the wrong size")
+        _check(lib().kpmx_mat_set_row_order(self.h, _p(q)))
+
     def coded_bytes(self):
         """Bytes of the value-table form of the SELL matrix (0: none; kpmx_mat_coded_bytes)."""
         b = ctypes.c_int64()

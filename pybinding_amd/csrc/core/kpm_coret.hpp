@@ -79,19 +79,24 @@ public:
         return out;
     }
 
-    // Site order of an LDOS or Green's function recurrence of `vectors` vectors.  The light cone of the
-    // BFS order saves work, but pays a launch per step (4.7 us) and a reorder and upload per site; on
-    // the locality order the chained recurrence sweeps the whole system several steps per launch.
-    // Up to 2^21 vector elements such a step takes less than that launch (137 k sites: 0.9 us, 2.1 M
-    // sites: 4.8 us); beyond, in runs too short for a chain and where no chain fits, the cone stays.
-    void optimize_for_sites(Indices const& idx, Scale<> scale, idx_t vectors, idx_t M) {
-        if (!no_chain_ && !oh_.locality_order.empty() && cfg_.algorithm.reorder() && format() == KPMX_FMT_SELL &&
-            M >= 160 && oh_.size() * vectors <= idx_t(1) << 21) {
-            oh_.optimize_for(idx, scale, true);
-            if (compute_.several_steps(oh_, format(), std::min<idx_t>(vectors, 64), M)) return;
+    // Site order of an LDOS or Green's function recurrence of `vectors` vectors, and its algorithm.  The
+    // light cone of the BFS order saves work, but pays a launch per step (4.7 us); the chained recurrence
+    // sweeps the whole system several steps per launch.  Up to 2^21 vector elements such a step takes
+    // less than that launch (137 k sites: 0.9 us, 2.1 M sites: 4.8 us); beyond, in runs too short for a
+    // chain and where no chain fits, the cone stays.  In double precision the matrix keeps the locality
+    // order from site to site (no BFS and upload for each); in 32 bits it stays BFS-ordered, so that every
+    // row's sum rounds as under the cone, and only the chain's tiles follow the locality order.
+    AlgorithmConfig optimize_for_sites(Indices const& idx, Scale<> scale, idx_t vectors, idx_t M) {
+        auto alg = cfg_.algorithm;
+        if (!no_chain_ && !oh_.locality_order.empty() && alg.reorder() && format() == KPMX_FMT_SELL && M >= 160 &&
+            oh_.size() * vectors <= idx_t(1) << 21) {
+            oh_.optimize_for(idx, scale, sizeof(real_t<T>) == 8);
+            alg.optimal_size = false;
+            if (compute_.several_steps(oh_, format(), std::min<idx_t>(vectors, 64), M)) return alg;
             no_chain_ = true;
         }
         oh_.optimize_for(idx, scale);
+        return cfg_.algorithm;
     }
 
     std::vector<double> ldos(std::vector<idx_t> const& idx, std::vector<double> const& energy, double broadening,
@@ -99,11 +104,11 @@ public:
         const auto scale = scaling_factors();
         const idx_t M = cfg_.kernel.required_num_moments(broadening / scale.a);
         const idx_t K = (idx_t)idx.size();
-        optimize_for_sites(Indices(idx, idx), scale, K, M);
-        stats_.reset(M, oh_, cfg_.algorithm, K, cfg_.matrix_format);
+        const auto alg = optimize_for_sites(Indices(idx, idx), scale, K, M);
+        stats_.reset(M, oh_, alg, K, cfg_.matrix_format);
         auto starter = unit_starter(oh_);
         BatchDiagonalMoments<T> m{M, K, false, {}};
-        timed_compute(&m, starter, cfg_.algorithm);
+        timed_compute(&m, starter, alg);
         apply_damping(m.data, cfg_.kernel, M, K);
         *cols_out = K;
         return spectral_density(compute_.ctx(), m.data, M, K, energy, scale);
@@ -142,16 +147,16 @@ public:
         if (cols.empty()) throw std::invalid_argument("KPM::calc_greens: no column indices given");
         const auto scale = scaling_factors();
         const idx_t M = cfg_.kernel.required_num_moments(broadening / scale.a);
-        optimize_for_sites(Indices(row, cols), scale, 1, M);
-        stats_.reset(M, oh_, cfg_.algorithm, 1, cfg_.matrix_format);
+        const auto alg = optimize_for_sites(Indices(row, cols), scale, 1, M);
+        stats_.reset(M, oh_, alg, 1, cfg_.matrix_format);
         if (oh_.optimized_idx.is_diagonal()) {
             DiagonalMoments<T> m{M, {}};
-            timed_compute(&m, unit_starter(oh_), cfg_.algorithm);
+            timed_compute(&m, unit_starter(oh_), alg);
             apply_damping(m.data, cfg_.kernel, M);
             return {greens_function(compute_.ctx(), m.data, energy, scale)};
         }
         MultiUnitMoments<T> m{M, &oh_.optimized_idx, {}};
-        timed_compute(&m, unit_starter(oh_), cfg_.algorithm);
+        timed_compute(&m, unit_starter(oh_), alg);
         std::vector<std::vector<cd>> out;
         for (auto& d : m.data) {
             apply_damping(d, cfg_.kernel, M);

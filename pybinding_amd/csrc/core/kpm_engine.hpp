@@ -254,16 +254,24 @@ public:
             h2_.reset();
             h2_ = upload(ctx(), oh.h2, format);
             version_ = oh.version;
+            ordered_ = 0;
             format_ = format;
             oh_ = &oh;
         }
         return h2_->m;
     }
 
-    // Whether diagonal recurrences of `num_vectors` vectors run several steps per launch on `oh`.
+    // Whether diagonal recurrences of `num_vectors` vectors without a light cone run several steps per
+    // launch on `oh`; a BFS-ordered matrix gets the locality order for its tiles.
     bool several_steps(OptimizedHamiltonian<T> const& oh, int format, idx_t num_vectors, idx_t num_moments) {
         kpmx_mat* h2 = matrix(oh, format);
         set_cone(h2, {});
+        if (!oh.used_locality && ordered_ != oh.version) {
+            std::vector<int32_t> order((size_t)oh.size());
+            for (size_t s = 0; s < order.size(); ++s) order[(size_t)oh.reorder_map[s]] = oh.locality_order[s];
+            check(kpmx_mat_set_row_order(h2, order.data()));
+            ordered_ = oh.version;
+        }
         int steps = 0, cols = 0;
         check(kpmx_diagonal_form(h2, num_vectors, num_moments, &steps, &cols));
         return steps > 1;
@@ -406,6 +414,7 @@ private:
     bool tuned_[7] = {};  // block widths 1 .. 64 already tuned on this matrix
     std::unique_ptr<MatHandle> h2_;
     uint64_t version_ = 0;
+    uint64_t ordered_ = 0;  // version whose matrix has a row order (kpmx_mat_set_row_order)
     int format_ = -1;
     OptimizedHamiltonian<T> const* oh_ = nullptr;
 };

@@ -254,7 +254,9 @@ struct kpmx_mat {
     void* ctable = nullptr;
     int cmax_width = 0, ctable_size = 0;
     mutable std::vector<std::unique_ptr<ChainHolder>> chains;  // by column width, built on first use
+    int32_t* row_order = nullptr;  // kpmx_mat_set_row_order: ChainMatrix::perm, then ::place
     ~kpmx_mat() {
+        dev_free(row_order);
         for (void* p : {(void*)cslice_ptr, (void*)cslice_width, (void*)cindices, (void*)ccodes, cdiag, ctable}) dev_free(p);
         dev_free(d_h1_ptr);
         dev_free(d_h1_rows);
@@ -967,6 +969,10 @@ ChainMatrix chain_matrix(const kpmx_mat* h2) {
     ChainMatrix m;
     m.scalar = h2->scalar;
     m.n = h2->rows;
+    if (h2->row_order) {
+        m.perm = h2->row_order;
+        m.place = h2->row_order + h2->rows;
+    }
     if (h2->ccodes) {
         m.max_width = h2->cmax_width;
         m.slice_ptr = h2->cslice_ptr;
@@ -976,6 +982,11 @@ ChainMatrix chain_matrix(const kpmx_mat* h2) {
         m.diag = h2->cdiag;
         m.table = h2->ctable;
         m.table_size = m.table_most = h2->ctable_size;
+        m.row_ptr = h2->slice_ptr;
+        m.row_width = h2->slice_width;
+        m.row_indices = h2->sell_indices;
+        m.row_vals = h2->sell_vals;
+        m.row_max_width = h2->max_width;
     } else {
         m.max_width = h2->max_width;
         m.slice_ptr = h2->slice_ptr;
@@ -996,7 +1007,7 @@ double chain_cost(const ChainMatrix& m, double rows, const double* e, int steps,
     const double tiles = std::ceil((double)m.n / rows), wgs = tiles > num_cu ? 2 : 1;
     double rounds = tiles / (wgs * num_cu);
     rounds = rounds < 8 ? std::ceil(rounds) : rounds + 0.5;
-    const double sb = (double)scalar_bytes(m.scalar), width = m.max_width;
+    const double sb = (double)scalar_bytes(m.scalar), width = m.width();
     const double entry = 2 + (m.form() == CHAIN_STD ? sb : m.form() == CHAIN_TABLE ? 1 : 0);
     const double bytes = (e[steps] + e[steps - 1] + 2 * rows) * row_bytes + e[steps - 1] * (entry * width + sb);
     const double rate = 4 * (double)m.n * row_bytes < 192e6 ? 32e3 : 21e3;
@@ -1112,8 +1123,8 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     for (int64_t t = 0; t < P.ntiles; ++t) halo = std::max(halo, ring[t * ST + steps] - ring[t * ST]);
     const size_t ring_bytes = (size_t)P.ntiles * ST * sizeof(int32_t), begin_bytes = (size_t)(P.ntiles + 1) * sizeof(int32_t);
     P.steps = steps;
-    P.width = m.max_width;
-    P.groups = std::max(1, (m.max_width + 3) / 4);
+    P.width = m.width();
+    P.groups = std::max(1, (P.width + 3) / 4);
     P.rows_x = most[steps];
     const int row_pad = chain_row_pad(m, cols);
     P.rows_y = (most[steps - 1] + row_pad - 1) / row_pad * row_pad;
@@ -1952,6 +1963,32 @@ int kpmx_mat_set_step_rows(kpmx_mat* h2, int64_t num_steps, const int64_t* rows)
     });
 }
 
+int kpmx_mat_set_row_order(kpmx_mat* h2, const int32_t* order) {
+    return guarded([&] {
+        KPMX_REQUIRE(h2, "null matrix");
+        kpmx_ctx* ctx = h2->ctx;
+        KPMX_HIP(hipSetDevice(ctx->device));
+        const int64_t n = h2->rows;
+        std::vector<int32_t> both;
+        if (order) {
+            both.assign((size_t)(2 * n), -1);
+            for (int64_t i = 0; i < n; ++i) {
+                KPMX_REQUIRE(order[i] >= 0 && order[i] < n && both[(size_t)order[i]] < 0, "the row order is not a permutation");
+                both[(size_t)order[i]] = (int32_t)i;
+                both[(size_t)(n + i)] = order[i];
+            }
+        }
+        KPMX_HIP(hipStreamSynchronize(ctx->stream));  // queued launches read the plans
+        h2->chains.clear();
+        dev_free(h2->row_order);
+        h2->row_order = nullptr;
+        if (!order || n == 0) return;
+        h2->row_order = static_cast<int32_t*>(dev_alloc(both.size() * sizeof(int32_t)));
+        KPMX_HIP(hipMemcpyAsync(h2->row_order, both.data(), both.size() * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+        KPMX_HIP(hipStreamSynchronize(ctx->stream));
+    });
+}
+
 int kpmx_block_upload(kpmx_ctx* ctx, int scalar, int64_t n, int64_t num_vectors, const void* r0, kpmx_block** out) {
     return guarded([&] {
         KPMX_REQUIRE(ctx && out, "null context or output");
@@ -2448,7 +2485,7 @@ struct ChainOpHolder {
 const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, int64_t steps, ChainOpHolder& H) {
     kpmx_ctx* ctx = h2->ctx;
     if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || op->format != KPMX_FMT_SELL ||
-        !h2->step_rows.empty())
+        !h2->step_rows.empty() || h2->row_order)
         return nullptr;
     const size_t sb = scalar_bytes(h2->scalar);
     if (2 * std::max(5.5, 3.0 * h2->rows * cols * sb / 5.6e6) * steps < 400) return nullptr;
@@ -3326,6 +3363,11 @@ ChainMatrix batch_chain_matrix(const kpmx_batch* b) {
         m.table = b->ctable;
         m.table_size = (int)b->table_len;
         m.table_most = b->table_most;
+        m.row_ptr = b->slice_ptr;
+        m.row_width = b->slice_width;
+        m.row_indices = b->sidx;
+        m.row_vals = b->svals;
+        m.row_max_width = b->max_width;
     }
     return m;
 }

@@ -58,10 +58,12 @@ __device__ void collect_rings(const ChainMatrix& m, int64_t r0, int64_t r1, int 
         if (t == 0) shared_count = 0;
         __syncthreads();
         for (int i = t; i < front; i += PLAN_THREADS) {
-            const int64_t row = own ? r0 + i : last[i];
+            int64_t row = own ? r0 + i : last[i];
+            if (m.perm) row = m.perm[row];
             const int64_t sl = row >> 6, base = m.slice_ptr[sl] + (row & 63);
             for (int k = 0; k < m.slice_width[sl]; ++k) {
-                const int32_t c = m.indices[base + (int64_t)k * 64];
+                int32_t c = m.indices[base + (int64_t)k * 64];
+                if (m.place) c = m.place[c];
                 if (c >= r0 && c < r1) continue;
                 // too many already: the ring is dropped
                 if (__hip_atomic_load(&shared_count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + total > limit) break;
@@ -121,6 +123,10 @@ __global__ __launch_bounds__(PLAN_THREADS) void k_chain_rings(ChainMatrix m, con
                   ring + t * (CHAIN_MAX_STEPS + 1), ext + t * ext_stride);
 }
 
+__device__ __forceinline__ bool is_zero(float v) { return v == 0.f; }
+__device__ __forceinline__ bool is_zero(double v) { return v == 0.0; }
+template <class R> __device__ __forceinline__ bool is_zero(cplx<R> v) { return v.re == R(0) && v.im == R(0); }
+
 // Entries of every local row up to distance steps - 1: 2-byte local columns (a missing entry is the
 // zero row), codes or values, and the diagonal.
 template <class V, int FORM>
@@ -151,9 +157,20 @@ __global__ __launch_bounds__(PLAN_THREADS) void k_chain_entries(ChainMatrix m, c
     __syncthreads();
     for (int i = threadIdx.x; i < rows_y; i += PLAN_THREADS) {
         // rows past the tile's last are padding: no entries
-        const int64_t row = i < own ? r0 + i : i < ny ? halo[i - own] : r0;
+        int64_t row = i < own ? r0 + i : i < ny ? halo[i - own] : r0;
+        if (m.perm) row = m.perm[row];
         const int64_t sl = row >> 6, base = m.slice_ptr[sl] + (row & 63);
-        const int w = i < ny ? m.slice_width[sl] : 0;
+        // local column of a neighbour (every one lies within `steps` of the tile)
+        auto local = [&](int32_t col) -> uint16_t {
+            if (m.place) col = m.place[col];
+            if (col >= r0 && col < r0 + own) return (uint16_t)((col - r0) * ew);
+            unsigned h = set.slot(col);
+            while (keys[h] != col && keys[h] != -1) h = set.next(h);
+            return keys[h] == col ? place[h] : (uint16_t)zero_item;
+        };
+        const bool ordered = FORM != CHAIN_STD && m.ordered();
+        const int w = i >= ny ? 0 : ordered ? m.row_width[sl] : m.slice_width[sl];
+        int next = 0;  // ordered: the next off-diagonal entry
         for (int g = 0; g < groups; ++g) {
             uint16_t id[4];
             uint32_t code = 0;
@@ -162,23 +179,28 @@ __global__ __launch_bounds__(PLAN_THREADS) void k_chain_entries(ChainMatrix m, c
                 id[q] = (uint16_t)zero_item;
                 V v = zero(V{});
                 if (k < w) {
-                    const int64_t e = base + (int64_t)k * 64;
-                    const int32_t c = m.indices[e];
-                    bool stored = true;
                     if constexpr (FORM == CHAIN_STD) {
+                        const int64_t e = base + (int64_t)k * 64;
                         v = static_cast<const V*>(m.vals)[e];
+                        id[q] = local(m.indices[e]);
+                    } else if (ordered) {
+                        const int64_t e = m.row_ptr[sl] + (row & 63) + (int64_t)k * 64;
+                        const int32_t col = m.row_indices[e];
+                        if (col != row) {
+                            const uint32_t cd = m.codes[base + (int64_t)next * 64];
+                            ++next;
+                            code |= cd << (8 * q);
+                            if (!(FORM == CHAIN_UNIFORM && cd == 0)) id[q] = local(col);
+                        } else if (!is_zero(static_cast<const V*>(m.row_vals)[e])) {
+                            id[q] = (uint16_t)(i * ew);  // the diagonal (a padded slot is zero)
+                        }
                     } else {
+                        const int64_t e = base + (int64_t)k * 64;
+                        const int32_t col = m.indices[e];
                         const uint32_t cd = m.codes[e];
-                        stored = c != row && !(FORM == CHAIN_UNIFORM && cd == 0);
-                        if (stored) code |= cd << (8 * q);
-                    }
-                    if (stored) {
-                        if (c >= r0 && c < r0 + own) {
-                            id[q] = (uint16_t)((c - r0) * ew);
-                        } else {
-                            unsigned h = set.slot(c);
-                            while (keys[h] != c && keys[h] != -1) h = set.next(h);
-                            id[q] = keys[h] == c ? place[h] : (uint16_t)zero_item;
+                        if (col != row && !(FORM == CHAIN_UNIFORM && cd == 0)) {
+                            code |= cd << (8 * q);
+                            id[q] = local(col);
                         }
                     }
                 }
@@ -287,7 +309,7 @@ static int with_shape(int scalar, int cols, int form, int width, F&& f) {
 int chain_max_cols(int scalar) { return scalar == 0 ? 16 : scalar == 3 ? 4 : 8; }
 
 int chain_row_capacity(const ChainMatrix& m, int cols) {
-    return with_shape(m.scalar, cols, m.form(), m.max_width, [](auto s, auto) { return decltype(s)::rows; });
+    return with_shape(m.scalar, cols, m.form(), m.width(), [](auto s, auto) { return decltype(s)::rows; });
 }
 
 int chain_row_items(int scalar, int cols) {
@@ -295,7 +317,7 @@ int chain_row_items(int scalar, int cols) {
 }
 
 int chain_row_pad(const ChainMatrix& m, int cols) {
-    return with_shape(m.scalar, cols, m.form(), m.max_width,
+    return with_shape(m.scalar, cols, m.form(), m.width(),
                       [](auto s, auto ew) { return decltype(s)::threads / decltype(ew)::value; });
 }
 

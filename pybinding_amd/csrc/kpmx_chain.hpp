@@ -19,6 +19,11 @@ enum { CHAIN_STD = 0, CHAIN_TABLE = 1, CHAIN_UNIFORM = 2 };
 struct ChainMatrix {
     int scalar = 1;
     int64_t n = 0;
+    // row order of the plan's tiles: perm[plan row] = matrix row, place[matrix row] = plan row (null:
+    // the matrix's own).  The work vectors are in plan order, the first launch's x, weights and marks in
+    // matrix order; panels need the matrix's own.
+    const int32_t* perm = nullptr;
+    const int32_t* place = nullptr;
     int max_width = 0;
     const int64_t* slice_ptr = nullptr;
     const int32_t* slice_width = nullptr;
@@ -29,7 +34,16 @@ struct ChainMatrix {
     const void* table = nullptr;     // zero first; several systems' tables one after another
     int table_size = 0;
     int table_most = 0;              // entries of the largest of them
-    int form() const { return !codes ? CHAIN_STD : table_most <= 2 ? CHAIN_UNIFORM : CHAIN_TABLE; }
+    // value-table form of 32-bit types: the standard SELL of the same rows, whose entry order (diagonal
+    // in its place) the plan keeps
+    const int64_t* row_ptr = nullptr;
+    const int32_t* row_width = nullptr;
+    const int32_t* row_indices = nullptr;
+    const void* row_vals = nullptr;
+    int row_max_width = 0;
+    __host__ __device__ bool ordered() const { return codes && (scalar == 0 || scalar == 2); }
+    __host__ __device__ int width() const { return ordered() ? row_max_width : max_width; }  // entries of a plan's rows
+    __host__ __device__ int form() const { return !codes ? CHAIN_STD : table_most <= 2 ? CHAIN_UNIFORM : CHAIN_TABLE; }
 };
 
 // Device arrays of a plan.  Tile t owns rows [tile_begin[t], tile_begin[t + 1]); its local rows are

@@ -182,6 +182,7 @@ struct shape {
 template <class E>
 struct ChainArgs {
     using value = typename elem<E>::value;
+    const int32_t* perm;  // matrix row of every plan row (null: the same)
     const int32_t* tile_begin;
     const int32_t* ring;
     const int32_t* ext;
@@ -297,6 +298,9 @@ void k_chain(ChainArgs<E> a) {
     using S = shape<E, EW, FORM, (W > 0)>;
     constexpr int IT = S::items, THREADS = S::threads, WAVES = S::waves;
     constexpr bool SUMS = MODE == CHAIN_SUMS || MODE == CHAIN_DOTS;
+    // 32-bit sums run in the order of the stored row, diagonal in its place, as the single steps do: the
+    // vectors are theirs bit for bit (in 64 bits the order is free)
+    constexpr bool ORDERED = sizeof(real) == 4;
     constexpr int NS = MODE == CHAIN_DOTS ? 2 * (elem<E>::kinds - 1) : SUMS ? S::NS : 1;
     constexpr int LD = 2;  // items loaded together
     constexpr bool KEEP = W > 0 && S::narrow;  // entries in registers
@@ -338,6 +342,8 @@ void k_chain(ChainArgs<E> a) {
             const int first = (I0 + u) * THREADS;  // item of thread 0
             g[u] = (int32_t)r0 + (int32_t)trow + first / EW;
             if (tid >= nown - first && tid < nx - first) g[u] = at(halo + (first / EW - own), trow);
+            // the first launch reads the caller's vectors, in the matrix's row order
+            if (a.first && a.perm && tid < nx - first) g[u] = a.perm[g[u]];
         });
         static_for<N>([&](auto u) {
             xv[u] = make_zero<E>();
@@ -392,6 +398,10 @@ void k_chain(ChainArgs<E> a) {
         for (int w = 1; w < WAVES; ++w) v += rw[w * NS * EW];
         a.partials[((int64_t)(j - 1) * a.ntiles + t) * (NS * EW) + i] = v;
     };
+    auto matrix_row = [&](unsigned row) -> int64_t {
+        const int64_t g = r0 + row + trow;
+        return a.perm ? a.perm[g] : g;
+    };
     // row `row` (of thread 0) of the panel's step p, every column of the element to its own panel
     auto to_panel = [&](const E& e, int p, int row) {
         using T = decltype(column_of(e, 0));
@@ -417,12 +427,17 @@ void k_chain(ChainArgs<E> a) {
             constexpr int row = it * (THREADS / EW);  // of thread 0
             const unsigned r = row + again;
             E h = make_zero<E>();
+            V d = zero(V{});
+            const uint16_t self = (uint16_t)((row + trow) * EW);
             auto entry = [&](uint16_t l, V v, bool first) {
                 const E xg = Xc[l];
-                if constexpr (FORM == CHAIN_UNIFORM) h = first ? xg : plus(h, xg);
-                else h = first ? product(v, xg) : fmac(v, xg, h);
+                if constexpr (FORM == CHAIN_UNIFORM && !ORDERED) {
+                    h = first ? xg : plus(h, xg);
+                } else {
+                    if constexpr (ORDERED && FORM != CHAIN_STD) v = l == self ? d : v;
+                    h = first && !ORDERED ? product(v, xg) : fmac(v, xg, h);
+                }
             };
-            V d = zero(V{});
             if constexpr (W > 0) {
                 ushort4 l;
                 uint32_t cd = 0;
@@ -439,6 +454,7 @@ void k_chain(ChainArgs<E> a) {
                 static_for<W>([&](auto k) {
                     if constexpr (FORM == CHAIN_STD) v[k] = at(vals + ((unsigned)(k * a.rows_y) + r), trow);
                     if constexpr (FORM == CHAIN_TABLE) v[k] = tab[(cd >> (8 * k)) & 255];
+                    if constexpr (FORM == CHAIN_UNIFORM) v[k] = uniform;
                 });
                 entry(l.x, v[0], true);
                 entry(l.y, v[1], false);
@@ -460,6 +476,7 @@ void k_chain(ChainArgs<E> a) {
                     static_for<4>([&](auto k) {
                         if constexpr (FORM == CHAIN_STD) v[k] = at(vals + ((unsigned)((4 * g + k) * a.rows_y) + r), trow);
                         if constexpr (FORM == CHAIN_TABLE) v[k] = tab[(cd >> (8 * k)) & 255];
+                        if constexpr (FORM == CHAIN_UNIFORM) v[k] = uniform;
                     });
                     entry(l.x, v[0], false);
                     entry(l.y, v[1], false);
@@ -468,13 +485,13 @@ void k_chain(ChainArgs<E> a) {
                 }
             }
             const E xi = X[tid + it * THREADS];
-            if constexpr (FORM == CHAIN_UNIFORM) h = product(uniform, h);
-            if constexpr (FORM != CHAIN_STD) h = fmac(d, xi, h);
+            if constexpr (FORM == CHAIN_UNIFORM && !ORDERED) h = product(uniform, h);
+            if constexpr (FORM != CHAIN_STD && !ORDERED) h = fmac(d, xi, h);
             y[it] = sub(scal(h, hs), y[it]);
             if constexpr (MODE == CHAIN_SUMS)
                 if (tid < nown - it * THREADS) add_sums(y[it], xi, s);
             if constexpr (MODE == CHAIN_DOTS)
-                if (tid < nown - it * THREADS) add_dots(at(a.w + r0 + row + again, trow), y[it], xi, s);
+                if (tid < nown - it * THREADS) add_dots(a.w[matrix_row(row + again)], y[it], xi, s);
             if constexpr (MODE == CHAIN_PANEL)
                 if (tid < nown - it * THREADS) to_panel(y[it], j, row);
             if constexpr (MODE == CHAIN_PANEL_OP)
@@ -492,7 +509,7 @@ void k_chain(ChainArgs<E> a) {
                 }
             if constexpr (MODE == CHAIN_MARKS)
                 if (tid < nown - it * THREADS) {
-                    const int m = at(a.mark + r0 + row + again, trow);
+                    const int m = a.mark[matrix_row(row + again)];
                     if (m >= 0) a.mark_out[m * a.mark_stride + j] = y[it];
                 }
         });
@@ -568,6 +585,7 @@ int launch_form(const ChainLaunch& L, hipStream_t s) {
     using V = typename elem<E>::value;
     const ChainPlan& P = *L.plan;
     ChainArgs<E> a{};
+    a.perm = L.m.perm;
     a.tile_begin = P.tile_begin;
     a.ring = P.ring;
     a.ext = P.ext;
