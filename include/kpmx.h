@@ -166,7 +166,8 @@ int kpmx_ctx_set_step_variant(kpmx_ctx* ctx, int scalar, int vector_width, int v
 
 /* Pin the variant of the adjoint step kernel (numbered as the diagonal step variants; no
  * counterpart in the reference) on the context; -1 restores the default (wave-staged entries on
- * twice the resident grid, fp64 blocks of 8 or more vectors as column pairs). */
+ * twice the resident grid, fp64 blocks of 8 or more vectors as column pairs).  A pinned variant also
+ * turns the backward launches of several steps off (kpmx_adjoint_diagonal). */
 int kpmx_ctx_set_adjoint_variant(kpmx_ctx* ctx, int variant);
 
 /* Widest column tile of the diagonal recurrence for one scalar type (1, 2, 4, ..., 64; no
@@ -271,7 +272,9 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
  * fused with the gradient accumulation over the sparsity pattern.  checkpoint: steps between stored
  * vector pairs, the vectors in between recomputed by running the recurrence backwards
  * (v_{j-1} = H2 v_j - v_{j+1}) inside the adjoint steps, restarting from every stored pair; <= 0
- * keeps every vector (no recomputation).
+ * keeps every vector (no recomputation).  Runs long enough for a plan use the chained form: launches of
+ * several steps forward (checkpointed) and backward (rows of at most four entries; fp32 only with
+ * checkpoints), under the conditions of kpmx_moments_diagonal.
  * Real H2 (KPMX_F32 / KPMX_F64) uploaded with KPMX_FMT_SELL; at most 64 vectors.
  * mu (optional): host, num_vectors x num_moments, the forward moments. */
 int kpmx_adjoint_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, const double* w,

@@ -202,6 +202,7 @@ struct LdsHalo {
 struct ChainHolder {
     int cols = 0;
     bool coded = false;          // batches: the matrix form it was built from
+    bool adjoint = false;        // of the backward recurrence
     ChainPlan plan;
     std::vector<int32_t> begin;  // plan.tile_begin
     char* data = nullptr;
@@ -1002,9 +1003,10 @@ ChainMatrix chain_matrix(const kpmx_mat* h2) {
 // loads and stores (about 21 KB a microsecond and CU from HBM, 32 KB while the vectors stay in
 // the Infinity Cache) overlap most of their steps, an item (16 bytes of a row) costs 0.4 ns alone and
 // 0.25 ns beside the other workgroup for three entries, a step 0.5 us of barriers and sums, a launch
-// 3 us.
+// 3 us.  A backward launch moves two such pairs of vectors and gathers two.
 double chain_cost(const ChainMatrix& m, double rows, const double* e, int steps, double row_bytes, int num_cu) {
     const double tiles = std::ceil((double)m.n / rows), wgs = tiles > num_cu ? 2 : 1;
+    if (m.adjoint) row_bytes *= 2;
     double rounds = tiles / (wgs * num_cu);
     rounds = rounds < 8 ? std::ceil(rounds) : rounds + 0.5;
     const double sb = (double)scalar_bytes(m.scalar), width = m.width();
@@ -1030,6 +1032,7 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     const int64_t n = m.n;
     const int cap = chain_row_capacity(m, cols);
     if (cap <= 0 || n < 64) return;
+    const int most_own = m.adjoint ? chain_adjoint_own_rows(m.scalar, cols) : cap;
     const size_t sb = scalar_bytes(m.scalar);
     const double row_bytes = (double)cols * sb;
     // heights: as many tiles as CUs and small multiples of twice that (no CU idles in the last
@@ -1037,7 +1040,7 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     std::vector<int> heights;
     auto add = [&](double h) {
         const int r = (int)std::max<int64_t>(32, (std::min<int64_t>(n, (int64_t)std::ceil(h)) + 7) / 8 * 8);
-        if (r <= 0.85 * cap && (int)heights.size() < CHAIN_CANDIDATES && std::find(heights.begin(), heights.end(), r) == heights.end())
+        if (r <= 0.85 * cap && r <= most_own && (int)heights.size() < CHAIN_CANDIDATES && std::find(heights.begin(), heights.end(), r) == heights.end())
             heights.push_back(r);
     };
     const double per_round = 2.0 * ctx->num_cu;
@@ -1114,6 +1117,14 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
             if ((last < 0 || last > cap) && own >= 32) split.push_back(begin[t] + own / 2);
         }
         split.push_back((int32_t)n);
+        // one step less where that fits every tile and the halves would start another of few rounds of
+        // workgroups (backward pass, 305 k rows: 5 steps on 546 tiles 44 us, 4 on 510 tiles 31 us)
+        const auto rounds = [&](size_t tiles) { return (tiles + 2 * ctx->num_cu - 1) / (2 * ctx->num_cu); };
+        if (steps > 2 && most[steps] < 0 && most[steps - 1] > 0 && rounds(begin.size() - 1) < 3 &&
+            rounds(split.size() - 1) > rounds(begin.size() - 1)) {
+            --steps;
+            break;
+        }
         if (pass == 4 || split.size() == begin.size() || (double)split.size() > 1.4 * begin.size()) break;
         begin.swap(split);
     }
@@ -1168,20 +1179,15 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     H.begin = std::move(begin);
 }
 
-// The plan for `cols` columns, built on first use (unless `existing` asks for one that is there
-// already); null where there is none.
-const ChainPlan* chain_plan(const kpmx_mat* h2, int cols, bool existing = false) {
+// The plan of m for `cols` columns, built on first use (unless `existing` asks for one that is there
+// already); null where there is none.  single_us: a single step of these columns.
+const ChainPlan* chain_plan(const kpmx_mat* h2, const ChainMatrix& m, int cols, double single_us, bool existing) {
     for (auto& c : h2->chains)
-        if (c->cols == cols) return c->data ? &c->plan : nullptr;
+        if (c->cols == cols && c->adjoint == m.adjoint) return c->data ? &c->plan : nullptr;
     if (existing) return nullptr;
     auto H = std::make_unique<ChainHolder>();
     H->cols = cols;
-    // single steps: about 5.6 TB/s of three passes over the columns and their share of the matrix, no
-    // less than a launch; a third of that on long rows
-    const ChainMatrix m = chain_matrix(h2);
-    const size_t sb = scalar_bytes(h2->scalar);
-    const double sweep = (3.0 * (double)h2->rows * cols * sb +
-                          (double)h2->nnz * (sb + 4) * cols / std::max(cols, h2->ctx->tile_cap[h2->scalar])) / 5.6e6;
+    H->adjoint = m.adjoint;
     auto cut = [&](int rows) {
         std::vector<int32_t> begin;
         for (int64_t r = 0; r < h2->rows; r += rows) begin.push_back((int32_t)r);
@@ -1189,7 +1195,7 @@ const ChainPlan* chain_plan(const kpmx_mat* h2, int cols, bool existing = false)
         return begin;
     };
     try {
-        build_chain(h2->ctx, m, cols, std::max(5.5, sweep * (m.max_width > 8 ? 3 : 1)), cut, *H);
+        build_chain(h2->ctx, m, cols, std::max(5.5, single_us), cut, *H);
     } catch (const Error& e) {
         if (e.code != KPMX_ENOMEM) throw;
         dev_free(H->data);
@@ -1197,6 +1203,35 @@ const ChainPlan* chain_plan(const kpmx_mat* h2, int cols, bool existing = false)
     }
     h2->chains.push_back(std::move(H));
     return h2->chains.back()->data ? &h2->chains.back()->plan : nullptr;
+}
+// Single steps take about 5.6 TB/s of three passes over the columns and their share of the matrix, no
+// less than a launch; a third of that on long rows.
+const ChainPlan* chain_plan(const kpmx_mat* h2, int cols, bool existing = false) {
+    const ChainMatrix m = chain_matrix(h2);
+    const size_t sb = scalar_bytes(h2->scalar);
+    const double sweep = (3.0 * (double)h2->rows * cols * sb +
+                          (double)h2->nnz * (sb + 4) * cols / std::max(cols, h2->ctx->tile_cap[h2->scalar])) / 5.6e6;
+    return chain_plan(h2, m, cols, sweep * (m.max_width > 8 ? 3 : 1), existing);
+}
+// The backward recurrence of the adjoint (at most four entries per row): six passes, and 40 bytes per
+// entry for its value, index and gradient.
+ChainMatrix adjoint_chain_matrix(const kpmx_mat* h2) {
+    ChainMatrix m;
+    m.adjoint = true;
+    m.scalar = h2->scalar;
+    m.n = h2->rows;
+    m.max_width = h2->max_width;
+    m.slice_ptr = h2->slice_ptr;
+    m.slice_width = h2->slice_width;
+    m.indices = h2->sell_indices;
+    m.vals = h2->sell_vals;
+    return m;
+}
+const ChainPlan* adjoint_chain_plan(const kpmx_mat* h2, int vw) {
+    if (h2->max_width > 4) return nullptr;
+    const int cols = chain_adjoint_cols(h2->scalar, vw);
+    const double single = (6.0 * (double)h2->rows * cols * scalar_bytes(h2->scalar) + 40.0 * (double)h2->nnz * cols / vw) / 5.6e6;
+    return chain_plan(h2, adjoint_chain_matrix(h2), cols, single, false);
 }
 
 int chain_cols(const kpmx_mat* h2, const Tile& t) { return std::min(t.vw, chain_max_cols(h2->scalar)); }
@@ -1364,6 +1399,155 @@ void chain_steps(const kpmx_mat* h2, const ChainPlan& P, int cols, const void* x
         KPMX_HIP(hipGetLastError());
         after_launch(L, k);
     }
+}
+
+// The forward pass of a checkpointed tape in the chained form: launches end at v_cC+1, so that they
+// write the pairs (v_cC, v_cC+1) and the last one, (v_S-1, v_S), where the tape keeps them.
+bool use_tape_chain(const kpmx_mat* h2, const Tile& t, int64_t steps) {
+    if (h2->row_order || !use_chain(h2, {t}, steps) || chain_plan(h2, chain_cols(h2, t))->steps < 3) return false;
+    try {
+        size_chain(h2, t, steps);
+    } catch (const Error& e) {
+        if (e.code != KPMX_ENOMEM) throw;
+        return false;
+    }
+    return true;
+}
+void run_tape_chain(const kpmx_tape* T, const Tile& t, double* sums) {
+    const kpmx_mat* h2 = T->h2;
+    kpmx_ctx* ctx = h2->ctx;
+    const int64_t S = T->S, C = T->C, last = (T->nck - 1) * C + 1;  // the last kept pair's second vector
+    const size_t sb = scalar_bytes(h2->scalar);
+    const int cols = chain_cols(h2, t), vw = t.vw;
+    const ChainPlan& P = *chain_plan(h2, cols);
+    const ChainBuffers B = size_chain(h2, t, S);
+    const int64_t per_step = P.ntiles * chain_partial_width(h2->scalar, cols);
+    const int64_t chunk = (int64_t)(B.partials_bytes / sizeof(double)) / per_step;
+    auto pair = [&](int64_t c) { return c < T->nck ? T->cks + (size_t)c * 2 * T->blk : T->slot(3); };
+    ChainLaunch L;
+    L.m = chain_matrix(h2);
+    L.plan = &P;
+    L.cols = cols;
+    for (int64_t c0 = 0; c0 < vw; c0 += cols) {
+        const size_t off = c0 * sb;
+        int64_t chunk_start = 0, c = 0;
+        int turn = 0;
+        L.x = T->cks + off;  // v_0
+        L.xprev = nullptr;
+        L.ldx = L.ldprev = vw;
+        for (int64_t k = 0; k < S; k += L.steps) {
+            const int64_t rest = (c < T->nck ? c * C + 1 : S) - k;
+            L.steps = (int)std::min<int64_t>(P.steps, rest);
+            if (rest == L.steps + 1) --L.steps;  // a launch of one step leaves no pair
+            const bool keep = L.steps == rest;
+            L.first = k == 0;
+            L.out1 = keep ? pair(c) + off : B.w[turn][0];
+            L.out2 = keep ? pair(c) + T->blk + off : B.w[turn][1];
+            L.ldout = keep ? vw : cols;
+            L.partials = B.partials + (k - chunk_start) * per_step;
+            if (launch_chain(L, ctx->stream) != 0) throw Error{KPMX_EINVAL, "unsupported chained recurrence"};
+            KPMX_HIP(hipGetLastError());
+            const int64_t done = k + L.steps;
+            if (done - chunk_start + P.steps > chunk || done == S) {
+                launch_chain_reduce(h2->scalar, CHAIN_SUMS, B.partials, P.ntiles, cols, done - chunk_start, nullptr, 1, vw, (int)c0,
+                                    sums + chunk_start * 4 * vw, ctx->stream);
+                KPMX_HIP(hipGetLastError());
+                chunk_start = done;
+            }
+            L.xprev = L.out1;  // v_0 after the first launch, which has one step
+            L.x = L.out2;
+            L.ldx = L.ldprev = L.ldout;
+            if (keep) ++c;
+            else turn ^= 1;
+        }
+    }
+    if (S - last <= 1)  // the last pair is, or overlaps, the last checkpoint
+        KPMX_HIP(hipMemcpyAsync(T->slot(3), T->cks + ((size_t)T->nck * 2 - 1 - (S == last)) * T->blk, T->blk * (1 + (S == last)),
+                                hipMemcpyDeviceToDevice, ctx->stream));
+}
+
+size_t backward_pair(const kpmx_tape* T) {  // bytes of two work vectors of a column group
+    return (size_t)2 * T->h2->rows * chain_adjoint_cols(T->h2->scalar, T->vw) * scalar_bytes(T->h2->scalar);
+}
+// The adjoint steps j = S-1 .. 1 in the chained form.  Null: single steps (variants that the caller
+// chose; long rows; fp32 tapes that keep every vector, where a rebuilt vector would differ in the last
+// bits from the kept one; small runs, as in use_chain).
+const ChainPlan* backward_chain(const kpmx_tape* T) {
+    const kpmx_mat* h2 = T->h2;
+    kpmx_ctx* ctx = h2->ctx;
+    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || ctx->adjoint_variant >= 0 || (T->store_all && h2->scalar == KPMX_F32))
+        return nullptr;
+    if (std::max(5.5, 6.0 * (double)T->blk / 5.6e6) * T->S < 400) return nullptr;
+    const ChainPlan* P = adjoint_chain_plan(h2, T->vw);
+    if (!P) return nullptr;
+    try {
+        ctx->work3.get(2 * backward_pair(T));
+        ctx->work4.get(2 * backward_pair(T));
+        ctx->partials.get((size_t)h2->rows * 4 * sizeof(double));
+    } catch (const Error& e) {
+        if (e.code != KPMX_ENOMEM) throw;
+        return nullptr;
+    }
+    return P;
+}
+// Leaves lambda_1 in lam1 (a block like the starters) and the steps' gradient in grad (SELL order).
+// Column groups run one after the other on packed work vectors.  Between kept pairs, v_j is rebuilt from
+// step to step; v_cC and v_cC+1 are read where the forward pass left them (so fp32 blocks follow the
+// single steps bit by bit).
+void run_backward_chain(const kpmx_tape* T, const ChainPlan& P, const std::vector<double>& alpha,
+                        const std::vector<double>& gamma, char* lam1, double* grad) {
+    const kpmx_mat* h2 = T->h2;
+    kpmx_ctx* ctx = h2->ctx;
+    const size_t blk = T->blk, sb = scalar_bytes(h2->scalar), pair = backward_pair(T);
+    const int64_t S = T->S, C = T->C;
+    char* lam = static_cast<char*>(ctx->work3.get(2 * pair));
+    char* v = static_cast<char*>(ctx->work4.get(2 * pair));
+    AdjointChainLaunch L;
+    L.m = adjoint_chain_matrix(h2);
+    L.plan = &P;
+    L.cols = chain_adjoint_cols(h2->scalar, T->vw);
+    L.grad = static_cast<double*>(ctx->partials.get((size_t)h2->rows * 4 * sizeof(double)));
+    launch_zero_f64(L.grad, h2->rows * 4, ctx->stream);
+    if ((T->nvec + L.cols - 1) / L.cols * L.cols < T->vw)  // columns without a vector stay 0
+        launch_zero(h2->scalar, lam1, h2->rows * T->vw, ctx->stream);
+    for (int64_t c0 = 0; c0 < T->nvec; c0 += L.cols) {
+        char *from = lam, *to = lam + pair, *vfrom = v, *vto = v + pair;
+        for (int64_t j = S - 1; j >= 1; j -= L.steps) {
+            const int64_t r = j % C;
+            int64_t rest = j;
+            const bool kept = T->store_all || j == S - 1 || r <= 1;
+            L.v = vfrom;
+            L.v_next = vfrom + pair / 2;
+            L.ldv = L.cols;
+            if (kept) {  // r = 1: v_j+1 is not used
+                char* p = T->store_all ? T->slot(j) : j == S - 1 ? T->slot(3) : T->cks + ((size_t)(j / C) * 2 + r) * blk;
+                L.v = p + c0 * sb;
+                L.v_next = p + c0 * sb + (T->store_all || j == S - 1 || r == 0 ? blk : 0);
+                L.ldv = T->vw;
+            }
+            if (!T->store_all) rest = r == 1 ? 1 : r == 0 ? C - 1 : r - 1;  // the steps above the next kept pair
+            L.steps = (int)std::min<int64_t>(P.steps, rest);
+            const bool rebuilt = !T->store_all && L.steps < rest, last = L.steps == j;
+            L.v_out = rebuilt ? vto : nullptr;
+            L.v_next_out = rebuilt ? vto + pair / 2 : nullptr;
+            L.lam = j == S - 1 ? nullptr : from;
+            L.lam_next = j == S - 1 ? nullptr : from + pair / 2;
+            L.lam_out = last ? lam1 + c0 * sb : to;
+            L.ldlam = last ? T->vw : L.cols;
+            L.lam_next_out = last ? nullptr : to + pair / 2;
+            for (int i = 0; i < L.steps; ++i) {
+                L.ca[i] = 2.0 * alpha[(size_t)(j - i)];
+                L.chv[i] = 2.0 * gamma[(size_t)(j - i)];
+                L.cg[i] = gamma[(size_t)(j - i)];
+            }
+            if (launch_adjoint_chain(L, ctx->stream) != 0) throw Error{KPMX_EINVAL, "unsupported adjoint configuration"};
+            KPMX_HIP(hipGetLastError());
+            std::swap(from, to);
+            if (rebuilt) std::swap(vfrom, vto);
+        }
+    }
+    launch_adjoint_chain_grad(L.m, L.grad, grad, ctx->stream);
+    KPMX_HIP(hipGetLastError());
 }
 
 // copies a sub-tile's columns into `dst` (default: work2, sized beforehand) and returns the tile
@@ -3796,6 +3980,9 @@ int kpmx_adjoint_forward(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, in
                     L.yout = T->slot(k + 1);
                 },
                 [](StepLaunch const&, int64_t) {});
+        } else if (use_tape_chain(h2, t, S)) {
+            KPMX_HIP(hipMemcpyAsync(T->cks, t.data, blk, hipMemcpyDeviceToDevice, ctx->stream));
+            run_tape_chain(T, t, sums);
         } else {
             KPMX_HIP(hipMemcpyAsync(T->cks, t.data, blk, hipMemcpyDeviceToDevice, ctx->stream));
             run_recurrence(h2, t, MODE_DIAG, S, nullptr, sums, [](StepLaunch&, int64_t) {},
@@ -3851,13 +4038,16 @@ int kpmx_adjoint_backward(kpmx_tape* T, const double* w, double* grad) {
         for (auto& v : alpha) v *= inv_r;
         for (auto& v : beta) v *= inv_r;
 
+        const ChainPlan* chain = backward_chain(T);  // before aux2 is used: plans are built in it
         const int64_t gsize = std::max<int64_t>(h2->sell_total, 1);
         double* dgrad = static_cast<double*>(ctx->aux2.get((size_t)gsize * sizeof(double)));
         launch_zero_f64(dgrad, gsize, ctx->stream);
         void* lamA = ctx->work0.get(blk);  // lambda_{j+2}, overwritten with lambda_j
         void* lamB = ctx->work1.get(blk);  // lambda_{j+1}
-        launch_zero(h2->scalar, lamA, n * vw, ctx->stream);
-        launch_zero(h2->scalar, lamB, n * vw, ctx->stream);
+        if (!chain) {
+            launch_zero(h2->scalar, lamA, n * vw, ctx->stream);
+            launch_zero(h2->scalar, lamB, n * vw, ctx->stream);
+        }
         AdjointLaunch A;
         A.scalar = h2->scalar;
         A.vw = vw;
@@ -3900,7 +4090,8 @@ int kpmx_adjoint_backward(kpmx_tape* T, const double* w, double* grad) {
             return p ? p : T->slot(j % 3);
         };
         // adjoint steps j = S-1 .. 1 (lambda_S = lambda_S+1 = 0)
-        for (int64_t j = S - 1; j >= 1; --j) {
+        if (chain) run_backward_chain(T, *chain, alpha, gamma, static_cast<char*>(lamB), dgrad);
+        for (int64_t j = chain ? 0 : S - 1; j >= 1; --j) {
             A.lam1 = lamB;
             A.lam2 = lamA;
             A.lam_out = lamA;

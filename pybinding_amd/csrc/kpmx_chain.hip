@@ -309,6 +309,7 @@ static int with_shape(int scalar, int cols, int form, int width, F&& f) {
 int chain_max_cols(int scalar) { return scalar == 0 ? 16 : scalar == 3 ? 4 : 8; }
 
 int chain_row_capacity(const ChainMatrix& m, int cols) {
+    if (m.adjoint) return chain_adjoint_capacity(m.scalar, cols);
     return with_shape(m.scalar, cols, m.form(), m.width(), [](auto s, auto) { return decltype(s)::rows; });
 }
 
@@ -317,6 +318,7 @@ int chain_row_items(int scalar, int cols) {
 }
 
 int chain_row_pad(const ChainMatrix& m, int cols) {
+    if (m.adjoint) return chain_adjoint_row_pad(m.scalar, cols);
     return with_shape(m.scalar, cols, m.form(), m.width(),
                       [](auto s, auto ew) { return decltype(s)::threads / decltype(ew)::value; });
 }

@@ -24,6 +24,7 @@ struct ChainMatrix {
     // matrix order; panels need the matrix's own.
     const int32_t* perm = nullptr;
     const int32_t* place = nullptr;
+    bool adjoint = false;  // for the backward recurrence: two vectors in LDS, standard form
     int max_width = 0;
     const int64_t* slice_ptr = nullptr;
     const int32_t* slice_width = nullptr;
@@ -79,6 +80,35 @@ int chain_rings(const ChainMatrix& m, const ChainPlan& P, int max_steps, hipStre
 // entry arrays of every tile (P.steps, rows_x, rows_y set and the arrays allocated)
 int chain_entries(const ChainMatrix& m, const ChainPlan& P, hipStream_t s);
 
+// Reverse steps j, j - 1, ..., j - steps + 1 of the adjoint (kpmx_chain_adjoint.hip) on `cols` columns:
+// reads v_j, v_j+1, lambda_j+1, lambda_j+2 (lam null: both zero) and writes the same four `steps` lower
+// (v_out null: no v, lam_next_out null: lambda_j+1-steps only); grad[4 row + k] of every stored entry is
+// updated.  The outputs are no inputs.
+struct AdjointChainLaunch {
+    ChainMatrix m;  // standard form
+    const ChainPlan* plan = nullptr;
+    int cols = 4, steps = 1;
+    int64_t ldv = 0, ldlam = 0;  // row strides of v and v_next, of lam_out in scalars (the others: cols)
+    const void* v = nullptr;
+    const void* v_next = nullptr;
+    const void* lam = nullptr;
+    const void* lam_next = nullptr;
+    void* v_out = nullptr;
+    void* v_next_out = nullptr;
+    void* lam_out = nullptr;
+    void* lam_next_out = nullptr;
+    double* grad = nullptr;
+    double ca[CHAIN_MAX_STEPS], chv[CHAIN_MAX_STEPS], cg[CHAIN_MAX_STEPS];  // of step j - i
+};
+int chain_adjoint_cols(int scalar, int vw);  // columns of a group of blocks of vw >= 4
+// local rows, own rows and row padding of its tiles (-1: no such layout); at most 4 entries per row
+int chain_adjoint_capacity(int scalar, int cols);
+int chain_adjoint_own_rows(int scalar, int cols);
+int chain_adjoint_row_pad(int scalar, int cols);
+int launch_adjoint_chain(const AdjointChainLaunch& L, hipStream_t s);
+// grad (SELL order, every stored entry) from the row-major sums
+void launch_adjoint_chain_grad(const ChainMatrix& m, const double* rows, double* grad, hipStream_t s);
+
 // What a step leaves beside the vectors: the diagonal sums, the dots with a weight vector, panel rows
 // of the new vector, panel rows of an operator applied to the vector before, or the new vector at
 // marked rows.
@@ -106,6 +136,7 @@ struct ChainLaunch {
     const void* xprev = nullptr;  // r_{k-1}, rows of `cols` scalars (not read by a first launch)
     void* out1 = nullptr;         // r_{k+steps-1} (not written by a one-step launch)
     void* out2 = nullptr;         // r_{k+steps}
+    int64_t ldprev = 0, ldout = 0;  // row strides of xprev and of out1 and out2 in scalars (0: cols)
     double* partials = nullptr;   // [steps][ntiles][chain_partial_width] (sums and dots)
     const void* w = nullptr;      // dots (one column): n weights
     // panels: column q of r_{k+j} (of the operator on r_{k+j-1}) goes to panel + q panel_col + p panel_step

@@ -197,7 +197,7 @@ struct ChainArgs {
     int groups, rows_x, rows_y;
     int64_t ntiles;
     const E* x;
-    int64_t ldx;  // in elements
+    int64_t ldx, ldprev, ldout;  // in elements
     const E* xprev;
     E* out1;
     E* out2;
@@ -351,7 +351,7 @@ void k_chain(ChainArgs<E> a) {
         });
         static_for<N>([&](auto u) {
             y[I0 + u] = make_zero<E>();
-            if (!a.first && tid < ny - (I0 + u) * THREADS) y[I0 + u] = a.xprev[(int64_t)g[u] * EW + c];
+            if (!a.first && tid < ny - (I0 + u) * THREADS) y[I0 + u] = a.xprev[(int64_t)g[u] * a.ldprev + c];
         });
         static_for<N>([&](auto u) {
             if (tid < nx - (I0 + u) * THREADS) X[tid + (I0 + u) * THREADS] = xv[u];
@@ -528,8 +528,9 @@ void k_chain(ChainArgs<E> a) {
     if constexpr (SUMS) store_sums(a.steps);
     static_for<IT>([&](auto it) {
         if (tid < nown - it * THREADS) {
-            at(a.out2 + r0 * EW + it * THREADS, tid) = y[it];
-            if (a.steps > 1) at(a.out1 + r0 * EW + it * THREADS, tid) = X[tid + it * THREADS];
+            const int64_t o = (r0 + it * (THREADS / EW) + trow) * a.ldout + c;
+            a.out2[o] = y[it];
+            if (a.steps > 1) a.out1[o] = X[tid + it * THREADS];
         }
     });
 }
@@ -603,6 +604,8 @@ int launch_form(const ChainLaunch& L, hipStream_t s) {
     a.ntiles = P.ntiles;
     a.x = static_cast<const E*>(L.x);
     a.ldx = L.ldx / elem<E>::cols;
+    a.ldprev = L.ldprev ? L.ldprev / elem<E>::cols : EW;
+    a.ldout = L.ldout ? L.ldout / elem<E>::cols : EW;
     a.xprev = static_cast<const E*>(L.xprev);
     a.out1 = static_cast<E*>(L.out1);
     a.out2 = static_cast<E*>(L.out2);

@@ -273,3 +273,29 @@ def test_row_order(oracle, dtype, form):
     assert np.max(np.abs(out[0] - ref) / np.abs(ref[:, :1])) <= TOL[dtype]
     for a, b, scale in zip(out, single, (n, n, 1)):
         assert np.max(np.abs(a - b)) <= scale * (2 * TOL[dtype] if TOL[dtype] < 1e-6 else 2.0 ** -20)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("form", ["uniform", "stored"])
+@pytest.mark.parametrize("nvec,checkpoint", [(1, 16), (3, 2), (8, 3), (9, 64), (16, 74), (16, 73), (20, 37), (33, 16), (5, 0)])
+def test_adjoint(form, dtype, nvec, checkpoint):
+    """Forward and backward passes in launches of several steps against single steps, with the
+    checkpoints near the ends of the run.  Tolerance: 75 steps forward and back that round
+    differently in fp64, 75 x 4 x 2^-53 < 1e-13 and a hundredfold for what cancels; in fp32 the
+    vectors are equal and only double sums are taken in another order."""
+    h2 = lattice(form, dtype=dtype)
+    moments = 150
+    w = np.random.default_rng(6).standard_normal(moments)
+    out = []
+    for single in (False, True):
+        ctx = abi.Ctx(0)
+        mat, blk = ctx.mat(h2, fmt=1), ctx.block(starters(h2.shape[0], nvec, dtype))
+        if single:
+            ctx.set_tile_width(dtype, 64)
+        print("chain adjoint", np.dtype(dtype).name, form, nvec, checkpoint, single, flush=True)
+        out.append(abi.adjoint_diagonal(mat, blk, moments, w, checkpoint))
+        ctx.close()
+    (grad, mu), (ref, mu_ref) = out
+    assert np.max(np.abs(grad - ref)) <= 1e-11 * np.max(np.abs(ref))
+    scale = np.abs(mu_ref[:, :1])
+    assert np.max(np.abs(mu - mu_ref) / scale) <= (1e-11 if dtype == np.float64 else 2.0 ** -22)
