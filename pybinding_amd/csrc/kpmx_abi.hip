@@ -1238,26 +1238,39 @@ int chain_cols(const kpmx_mat* h2, const Tile& t) { return std::min(t.vw, chain_
 
 constexpr size_t CHAIN_PARTIALS = (size_t)64 << 20;  // partial sums kept before one reduction
 
-// Two pairs of work vectors and the partial sums of one reduction.
+// Two pairs of work vectors and the partial sums of one reduction, for `groups` column groups that run
+// side by side (each with vectors of its own, one after another in w[][]).
 struct ChainBuffers {
     void* w[2][2];
     double* partials;
     size_t partials_bytes;
+    int groups = 1;
 };
 size_t chain_step_bytes(const kpmx_mat* h2, const ChainPlan& P, int cols) {
     return (size_t)P.ntiles * chain_partial_width(h2->scalar, cols) * sizeof(double);
+}
+// As many column groups as leave every workgroup in the first round (two per CU): launches of small
+// systems are latency, not work (fp64, 512 moments: 32 vectors on 3.8 k sites 1.44 ms one after the
+// other and 0.63 ms side by side, on 15 k sites 1.53 and 1.13 ms, 16 on 61 k sites 1.09 and 0.87 ms).
+int chain_groups(const kpmx_ctx* ctx, const ChainPlan& P, int cols, int64_t vectors) {
+    const int64_t all = (vectors + cols - 1) / cols;
+    const int64_t fit = std::min(all, std::max<int64_t>(1, 2 * ctx->num_cu / P.ntiles));
+    const int64_t turns = (all + fit - 1) / fit;
+    return (int)((all + turns - 1) / turns);
 }
 
 ChainBuffers size_chain(const kpmx_mat* h2, const Tile& t, int64_t steps) {
     kpmx_ctx* ctx = h2->ctx;
     const int cols = chain_cols(h2, t);
     const ChainPlan& P = *chain_plan(h2, cols);
-    const size_t blk = (size_t)h2->rows * cols * scalar_bytes(h2->scalar);
-    const size_t bytes = std::min(std::max(CHAIN_PARTIALS, P.steps * chain_step_bytes(h2, P, cols)),
-                                  (size_t)(steps + P.steps) * chain_step_bytes(h2, P, cols));
+    const int groups = chain_groups(ctx, P, cols, t.cols);
+    const size_t blk = (size_t)h2->rows * cols * scalar_bytes(h2->scalar) * groups;
+    const size_t step = chain_step_bytes(h2, P, cols) * groups;
+    const size_t bytes = std::min(std::max(CHAIN_PARTIALS, P.steps * step), (size_t)(steps + P.steps) * step);
     return {{{ctx->work0.get(blk), ctx->work1.get(blk)}, {ctx->work3.get(blk), ctx->work4.get(blk)}},
             static_cast<double*>(ctx->partials.get(bytes)),
-            bytes};
+            bytes,
+            groups};
 }
 
 // The diagonal recurrence of a starter tile in the chained form, in column groups of at most
@@ -1267,12 +1280,15 @@ void run_chain(kpmx_ctx* ctx, const ChainMatrix& m, const ChainPlan& P, int cols
                int64_t steps, const int32_t* system_tiles, int64_t num_systems, double* sums, const ChainBuffers& B) {
     const size_t sb = scalar_bytes(m.scalar);
     const int64_t per_step = P.ntiles * chain_partial_width(m.scalar, cols);
-    const int64_t chunk = std::max<int64_t>(1, (int64_t)(B.partials_bytes / sizeof(double)) / per_step / P.steps) * P.steps;
+    const int64_t chunk = std::max<int64_t>(1, (int64_t)(B.partials_bytes / sizeof(double)) / B.groups / per_step / P.steps) * P.steps;
     ChainLaunch L;
     L.m = m;
     L.plan = &P;
     L.cols = cols;
-    for (int64_t c0 = 0; c0 < vectors; c0 += cols) {
+    L.w_group = m.n * cols;
+    L.partials_group = chunk * per_step;
+    for (int64_t c0 = 0; c0 < vectors; c0 += (int64_t)L.col_groups * cols) {
+        L.col_groups = (int)std::min<int64_t>(B.groups, (vectors - c0 + cols - 1) / cols);
         int64_t chunk_start = 0;
         int turn = 0;
         for (int64_t k = 0; k < steps; k += L.steps, turn ^= 1) {
@@ -1280,6 +1296,7 @@ void run_chain(kpmx_ctx* ctx, const ChainMatrix& m, const ChainPlan& P, int cols
             L.first = k == 0;
             L.x = k == 0 ? static_cast<const char*>(r0) + c0 * sb : B.w[turn ^ 1][1];
             L.ldx = k == 0 ? vw : cols;
+            L.x_group = k == 0 ? cols : L.w_group;
             L.xprev = k == 0 ? nullptr : B.w[turn ^ 1][0];
             L.out1 = B.w[turn][0];
             L.out2 = B.w[turn][1];
@@ -1288,8 +1305,10 @@ void run_chain(kpmx_ctx* ctx, const ChainMatrix& m, const ChainPlan& P, int cols
             KPMX_HIP(hipGetLastError());
             const int64_t done = k + L.steps;
             if (done - chunk_start == chunk || done == steps) {
-                launch_chain_reduce(m.scalar, CHAIN_SUMS, B.partials, P.ntiles, cols, done - chunk_start, system_tiles, num_systems, vw,
-                                    (int)c0, sums + chunk_start * num_systems * 4 * vw, ctx->stream);
+                for (int g = 0; g < L.col_groups; ++g)
+                    launch_chain_reduce(m.scalar, CHAIN_SUMS, B.partials + g * L.partials_group, P.ntiles, cols, done - chunk_start,
+                                        system_tiles, num_systems, vw, (int)c0 + g * cols, sums + chunk_start * num_systems * 4 * vw,
+                                        ctx->stream);
                 KPMX_HIP(hipGetLastError());
                 chunk_start = done;
             }

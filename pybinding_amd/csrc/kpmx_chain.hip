@@ -329,7 +329,8 @@ int chain_partial_width(int scalar, int cols, int mode) {
 }
 
 int launch_chain(const ChainLaunch& L, hipStream_t s) {
-    if (!L.plan || L.steps < 1 || L.steps > L.plan->steps || L.plan->rows_x > chain_row_capacity(L.m, L.cols))
+    if (!L.plan || L.steps < 1 || L.steps > L.plan->steps || L.plan->rows_x > chain_row_capacity(L.m, L.cols) ||
+        L.col_groups < 1 || (L.col_groups > 1 && L.mode != CHAIN_SUMS))
         return -1;
     switch (L.m.scalar) {
         case 0: return launch_chain_f32(L, s);

@@ -138,6 +138,10 @@ struct ChainLaunch {
     void* out2 = nullptr;         // r_{k+steps}
     int64_t ldprev = 0, ldout = 0;  // row strides of xprev and of out1 and out2 in scalars (0: cols)
     double* partials = nullptr;   // [steps][ntiles][chain_partial_width] (sums and dots)
+    // sums: groups of `cols` columns in one launch, and the strides between them of x, of xprev, out1 and
+    // out2 (in scalars) and of the partials
+    int col_groups = 1;
+    int64_t x_group = 0, w_group = 0, partials_group = 0;
     const void* w = nullptr;      // dots (one column): n weights
     // panels: column q of r_{k+j} (of the operator on r_{k+j-1}) goes to panel + q panel_col + p panel_step
     // + row (scalars) with p = j (p = j - 1), step j = 1 ... steps; the operator's first row is halved

@@ -202,6 +202,7 @@ struct ChainArgs {
     E* out1;
     E* out2;
     double* partials;
+    int64_t x_group, w_group, partials_group;  // from one column group to the next
     int steps, first;
     // the other collections (see ChainLaunch)
     const E* w;
@@ -323,7 +324,16 @@ void k_chain(ChainArgs<E> a) {
 
     // tiles of one eighth of the rows on one XCD: neighbours' halo rows stay in its L2
     const int64_t per = (a.ntiles + 7) / 8;
-    const int64_t t = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
+    int64_t turn = blockIdx.x / 8;
+    if constexpr (MODE == CHAIN_SUMS)
+        for (; turn >= per; turn -= per) {  // column groups side by side
+            a.x += a.x_group;
+            a.xprev += a.w_group;
+            a.out1 += a.w_group;
+            a.out2 += a.w_group;
+            a.partials += a.partials_group;
+        }
+    const int64_t t = (int64_t)(blockIdx.x % 8) * per + turn;
     if (t >= a.ntiles) return;
     const int tid = threadIdx.x, c = tid % EW;
     const unsigned trow = (unsigned)tid / EW;
@@ -612,6 +622,9 @@ int launch_form(const ChainLaunch& L, hipStream_t s) {
     a.out1 = static_cast<E*>(L.out1);
     a.out2 = static_cast<E*>(L.out2);
     a.partials = L.partials;
+    a.x_group = L.x_group / elem<E>::cols;
+    a.w_group = L.w_group / elem<E>::cols;
+    a.partials_group = L.partials_group;
     a.steps = L.steps;
     a.first = L.first;
     a.w = static_cast<const E*>(L.w);
@@ -630,7 +643,7 @@ int launch_form(const ChainLaunch& L, hipStream_t s) {
     auto kernel = k_chain<E, EW, FORM, W, MODE>;
     static std::atomic<uint64_t> allowed{0};  // devices
     if (!allow_lds(reinterpret_cast<const void*>(kernel), LDS_BYTES, allowed)) return -1;
-    const int64_t grid = (P.ntiles + 7) / 8 * 8;
+    const int64_t grid = (P.ntiles + 7) / 8 * 8 * L.col_groups;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(shape<E, EW, FORM, (W > 0)>::threads), LDS_BYTES, s, a);
     return 0;
 }

@@ -97,6 +97,15 @@ def test_sizes(oracle, n1, n2):
     check(oracle, h2, starters(h2.shape[0], 5, np.float64), 150)
 
 
+@pytest.mark.parametrize("dtype,n1,n2,nvec", [(np.float64, 64, 32, 33), (np.float64, 90, 70, 20), (np.complex128, 64, 32, 18),
+                                              (np.float32, 90, 70, 64), (np.complex64, 24, 40, 40)])
+def test_column_groups(oracle, dtype, n1, n2, nvec):
+    """column groups side by side in one launch, all at once or in turns of which the last has fewer"""
+    h2 = lattice("uniform", n1, n2, dtype)
+    print("chain groups", np.dtype(dtype).name, h2.shape[0], nvec, flush=True)
+    check(oracle, h2, starters(h2.shape[0], nvec, dtype), 158)
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex128])
 @pytest.mark.parametrize("width", [5, 8, 19])
 def test_long_rows(oracle, dtype, width):
