@@ -273,8 +273,8 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
  * vector pairs, the vectors in between recomputed by running the recurrence backwards
  * (v_{j-1} = H2 v_j - v_{j+1}) inside the adjoint steps, restarting from every stored pair; <= 0
  * keeps every vector (no recomputation).  Runs long enough for a plan use the chained form: launches of
- * several steps forward (checkpointed) and backward (rows of at most four entries; fp32 only with
- * checkpoints), under the conditions of kpmx_moments_diagonal.
+ * several steps forward (checkpointed) and backward (rows of at most four entries; without checkpoints
+ * only fp64 and at most four vectors), under the conditions of kpmx_moments_diagonal.
  * Real H2 (KPMX_F32 / KPMX_F64) uploaded with KPMX_FMT_SELL; at most 64 vectors.
  * mu (optional): host, num_vectors x num_moments, the forward moments. */
 int kpmx_adjoint_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, const double* w,
@@ -298,7 +298,9 @@ int kpmx_tape_destroy(kpmx_tape* tape);
  *             indices; system s owns rows [row_offsets[s], row_offsets[s+1]) and may only couple
  *             to them).
  *   starters: num_vectors (1..64) starters per system, host, vector-major num_vectors x N.
- *   run:      all num_moments / 2 steps.  use_graph (the run mode): 0 one launch per step (and
+ *   run:      all num_moments / 2 steps, in modes 0 and 1 in launches of several steps (the chained
+ *             form of kpmx_moments_diagonal) unless a partition was set or the autotuner found single
+ *             steps faster.  use_graph (the run mode): 0 one launch per step or chain of steps (and
  *             per-system reduction), 1 the whole step sequence captured in one HIP graph on the
  *             first run for this num_moments and replayed afterwards, 2 one persistent kernel
  *             launch for all steps (grid barriers between steps; the partition's workgroups must
@@ -314,7 +316,7 @@ int kpmx_batch_run(kpmx_batch* b, int64_t num_moments, int use_graph);
  * contiguous regions, one per XCD, whose runs of walk_chunk slices are dealt round-robin to that
  * XCD's walkers, so the gathered rows of the band they sweep together stay in the XCD's L2.
  * Results stay within rounding of any other partition (only the grouping of each system's sums
- * changes). */
+ * changes).  A set partition also keeps modes 0 and 1 on single steps. */
 int kpmx_batch_set_partition(kpmx_batch* b, int num_workgroups, int walk_chunk);
 /* Matrix form of the batched step (no counterpart in the reference).  The value-table form --
  * off-diagonal entries as a 4-byte column and a 1-byte code into a table of at most 256 values
@@ -339,7 +341,8 @@ int kpmx_batch_format(const kpmx_batch* b, int* available, int* enabled, int64_t
 /* Autotuner of the batched step (no counterpart in the reference): times the step on this batch
  * and its starters over contiguous ranges for 1 to 256 workgroups per CU (four walkers, one per
  * wave, each) and over the XCD-aware walk (runs of 1, 2 or 4 slices on half, one, two and four
- * times the resident grid), and keeps the fastest partition.  num_workgroups, walk_chunk (optional): the chosen
+ * times the resident grid), and keeps the fastest partition; then the chained form against it, which
+ * modes 0 and 1 run where it is the faster one.  num_workgroups, walk_chunk (optional): the chosen
  * partition. */
 int kpmx_batch_autotune(kpmx_batch* b, int* num_workgroups, int* walk_chunk);
 int kpmx_batch_fetch(kpmx_batch* b, int64_t num_moments, void* mu);

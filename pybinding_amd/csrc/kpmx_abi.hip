@@ -1360,12 +1360,21 @@ std::vector<RunTile> run_tiles(const std::vector<Tile>& tiles, int cap) {
 std::vector<RunTile> run_tiles(const kpmx_block* r0, int cap) { return run_tiles(r0->tiles, cap); }
 int diag_cap(const kpmx_mat* h2) { return h2->ctx->tile_cap[h2->scalar]; }
 
+// Whether a run of `steps` single steps of single_us each pays for a plan in its first pass.  A plan
+// with its buffers costs about 0.13 ms and 2 us per thousand rows up to half a millisecond; chained steps
+// save 60 % of launch-bound steps and 40 % or more of the others.  First passes measured with a plan and
+// with single steps: 15 k sites, 80 steps 0.36 and 0.40 ms; 61 k sites, 80 steps 0.48 and 0.52 ms; but
+// 180 k sites, 10 vectors, 50 steps 1.18 and 0.99 ms.  Below 0.4 ms nothing is tried.  The same call
+// always takes the same form, whatever ran before.
+bool chain_pays(int64_t n, double single_us, int64_t steps) {
+    const double plan_us = 130 + std::min(2e-3 * (double)n, 500.0);
+    return std::max(5.5, single_us) * steps >= std::max(400.0, plan_us / (single_us <= 5.5 ? 0.6 : 0.4));
+}
+
 // Whether the diagonal recurrence of this block runs in the chained form: by default on SELL matrices
-// without light-cone limits whose plans promise it to be faster than single steps.  A two-step form
-// that the caller has turned on goes first where it applies.  A plan costs 0.15 to 0.3 ms on its first
-// use and halves the recurrence at least on launch-bound systems, so runs whose single steps are
-// expected to take less than 0.4 ms in all keep those (whatever was run before: the same call always
-// takes the same form).  existing: only with plans that are there already (nothing is allocated).
+// without light-cone limits whose plans promise it to be faster than single steps, where that pays.  A
+// two-step form that the caller has turned on goes first where it applies.  existing: only with plans
+// that are there already (nothing is allocated).
 bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps, bool existing = false) {
     const kpmx_ctx* ctx = h2->ctx;
     if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return false;
@@ -1373,7 +1382,7 @@ bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps
     double single_us = 0;
     for (const RunTile& rt : rts)
         single_us += std::max(5.5, 3.0 * h2->rows * rt.sub.vw * scalar_bytes(h2->scalar) / 5.6e6);
-    if (single_us * steps < 400) return false;
+    if (!chain_pays(h2->rows, single_us, steps)) return false;
     if (ctx->two_step[h2->scalar] > 0 && !existing)
         for (const RunTile& rt : rts)
             if (use_two_step(h2, rt.sub)) return false;
@@ -1387,7 +1396,7 @@ bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps
 const ChainPlan* chain_single(const kpmx_mat* h2, int64_t steps) {
     const kpmx_ctx* ctx = h2->ctx;
     if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return nullptr;
-    if (std::max(5.5, 3.0 * h2->rows * scalar_bytes(h2->scalar) / 5.6e6) * steps < 400) return nullptr;
+    if (!chain_pays(h2->rows, 3.0 * h2->rows * scalar_bytes(h2->scalar) / 5.6e6, steps)) return nullptr;
     return chain_plan(h2, 1);
 }
 
@@ -1424,7 +1433,11 @@ void chain_steps(const kpmx_mat* h2, const ChainPlan& P, int cols, const void* x
 // write the pairs (v_cC, v_cC+1) and the last one, (v_S-1, v_S), where the tape keeps them.
 bool use_tape_chain(const kpmx_mat* h2, const Tile& t, int64_t steps) {
     if (h2->row_order || !use_chain(h2, {t}, steps) || chain_plan(h2, chain_cols(h2, t))->steps < 3) return false;
-    try {
+    kpmx_ctx* ctx = h2->ctx;
+    const size_t column = (size_t)h2->rows * scalar_bytes(h2->scalar);
+    try {  // as large as the backward pass needs them: growing a buffer frees it first
+        for (Workspace* w : {&ctx->work0, &ctx->work1}) w->get(column * t.vw);
+        for (Workspace* w : {&ctx->work3, &ctx->work4}) w->get(column * 4 * chain_adjoint_cols(h2->scalar, t.vw));
         size_chain(h2, t, steps);
     } catch (const Error& e) {
         if (e.code != KPMX_ENOMEM) throw;
@@ -1489,14 +1502,16 @@ size_t backward_pair(const kpmx_tape* T) {  // bytes of two work vectors of a co
     return (size_t)2 * T->h2->rows * chain_adjoint_cols(T->h2->scalar, T->vw) * scalar_bytes(T->h2->scalar);
 }
 // The adjoint steps j = S-1 .. 1 in the chained form.  Null: single steps (variants that the caller
-// chose; long rows; fp32 tapes that keep every vector, where a rebuilt vector would differ in the last
-// bits from the kept one; small runs, as in use_chain).
+// chose; long rows; small runs, as in use_chain; tapes that keep every vector, in fp32, where a rebuilt
+// vector would differ in the last bits from the kept one, or of several column groups, which would each
+// fetch the whole rows of the kept blocks in every launch: 1 M sites, 16 fp64 vectors, 1024 moments
+// 107 ms against 101 ms with single steps).
 const ChainPlan* backward_chain(const kpmx_tape* T) {
     const kpmx_mat* h2 = T->h2;
     kpmx_ctx* ctx = h2->ctx;
-    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || ctx->adjoint_variant >= 0 || (T->store_all && h2->scalar == KPMX_F32))
-        return nullptr;
-    if (std::max(5.5, 6.0 * (double)T->blk / 5.6e6) * T->S < 400) return nullptr;
+    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || ctx->adjoint_variant >= 0) return nullptr;
+    if (T->store_all && (h2->scalar == KPMX_F32 || T->vw > chain_adjoint_cols(h2->scalar, T->vw))) return nullptr;
+    if (!chain_pays(h2->rows, 6.0 * (double)T->blk / 5.6e6, T->S)) return nullptr;
     const ChainPlan* P = adjoint_chain_plan(h2, T->vw);
     if (!P) return nullptr;
     try {
@@ -2691,7 +2706,7 @@ const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, 
         !h2->step_rows.empty() || h2->row_order)
         return nullptr;
     const size_t sb = scalar_bytes(h2->scalar);
-    if (2 * std::max(5.5, 3.0 * h2->rows * cols * sb / 5.6e6) * steps < 400) return nullptr;
+    if (!chain_pays(h2->rows, 3.0 * h2->rows * cols * sb / 5.6e6, 2 * steps)) return nullptr;  // both sweeps
     const ChainPlan* P = chain_plan(h2, cols);
     if (!P) return nullptr;
     if (H.plan == P) return H.data ? P : nullptr;

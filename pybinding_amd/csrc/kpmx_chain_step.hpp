@@ -8,7 +8,21 @@
 // rows within distance K - j, so after K steps the tile's own rows are exact and nothing is read
 // from another workgroup.  A launch reads two vectors (halo rows twice) and writes two: 4 / K
 // passes per step, and one launch for K steps.  The halo's redundant work is what limits K: the
-// plan (plan_chain in kpmx_abi.hip) weighs both from the tiles' measured halo sizes.
+// plan (build_chain in kpmx_abi.hip) weighs both from the tiles' measured halo sizes.
+//
+// Measured, single steps before and chained steps now, in us per step (K the steps per launch):
+//   fp64, 32 vectors, 1.05 M sites, one hopping   155    65   K = 6, 96 us per launch of 8 columns
+//   fp32, 32 vectors, 1.2 M sites, one hopping     93    50   K = 5, of 16 columns
+//   fp64, 1 vector, 2.1 M sites                    26   5.8   K = 5
+//   fp64, 24 vectors, 123 k rows of 19 entries     88    29   K = 3, of 8 columns
+//   complex128, 16 vectors, 512 k sites            69    51   K = 5, of 4 columns, stored values
+//   fp64, 8 vectors, 61 k sites                   5.8   2.0   K = 8
+//   fp32, 1 vector, 137 k sites                   4.7   1.4   K = 12
+// Large blocks are bound by their passes over memory (load and store phases take about half of a
+// launch) beside LDS gathers and arithmetic, small ones by the latency of a step: two barriers, the
+// gather and the sums.  Narrower column groups hold taller tiles but measured slower (fp64 block of 32:
+// 8.4, 9.6 and 10.9 ms in groups of 8, 4 and 2; complex128 of 16: 6.6 and 8.7 ms in groups of 4 and 2;
+// fp32 of 32: 6.8, 7.8 and 8.1 ms in groups of 16, 8 and 4).
 //
 // Layout: an item is one element of up to 16 bytes (a column pair, four fp32 columns, ...) of one
 // local row; item i sits at X[i] and belongs to thread i % T for the whole launch, so r_{k-1} needs
