@@ -1,0 +1,25 @@
+// When a run takes the chained recurrence (several Chebyshev steps per launch).
+#pragma once
+#include <algorithm>
+#include <cstdint>
+
+namespace kpmx {
+
+// Estimated microseconds of a single step on vw columns of n rows of `scalar` bytes: three passes at
+// 5.6 TB/s, no less than a launch.
+inline double single_step_us(int64_t n, int64_t vw, size_t scalar) {
+    return std::max(5.5, 3.0 * (double)n * (double)vw * (double)scalar / 5.6e6);
+}
+
+// Whether a run of `steps` single steps of single_us each pays for a plan in its first pass.  A plan
+// with its buffers costs about 0.13 ms and 2 us per thousand rows up to half a millisecond; chained steps
+// save 60 % of launch-bound steps and 40 % or more of the others.  First passes measured with a plan and
+// with single steps: 15 k sites, 80 steps 0.36 and 0.40 ms; 61 k sites, 80 steps 0.48 and 0.52 ms; but
+// 180 k sites, 10 vectors, 50 steps 1.18 and 0.99 ms.  Below 0.4 ms nothing is tried.  The same call
+// always takes the same form, whatever ran before.
+inline bool chain_pays(int64_t n, double single_us, int64_t steps) {
+    const double plan_us = 130 + std::min(2e-3 * (double)n, 500.0);
+    return single_us * (double)steps >= std::max(400.0, plan_us / (single_us <= 5.5 ? 0.6 : 0.4));
+}
+
+}  // namespace kpmx

@@ -1,6 +1,7 @@
 // CoreT<T>: the KPM Core for one scalar type (cppcore/src/kpm/Core.cpp:17-156), computing every
 // moment through HipCompute.
 #pragma once
+#include "chain_rule.hpp"
 #include "kpm_engine.hpp"
 
 namespace kpmx_host {
@@ -83,13 +84,16 @@ public:
     // light cone of the BFS order saves work, but pays a launch per step (4.7 us); the chained recurrence
     // sweeps the whole system several steps per launch.  Up to 2^21 vector elements such a step takes
     // less than that launch (137 k sites: 0.9 us, 2.1 M sites: 4.8 us); beyond, in runs too short for a
-    // chain and where no chain fits, the cone stays.  In double precision the matrix keeps the locality
+    // chain to pay (asked before anything is prepared for it) and where no chain fits, the cone stays.  In double precision the matrix keeps the locality
     // order from site to site (no BFS and upload for each); in 32 bits it stays BFS-ordered, so that every
     // row's sum rounds as under the cone, and only the chain's tiles follow the locality order.
     AlgorithmConfig optimize_for_sites(Indices const& idx, Scale<> scale, idx_t vectors, idx_t M) {
         auto alg = cfg_.algorithm;
+        idx_t vw = 1;
+        while (vw < vectors && vw < 64) vw <<= 1;
         if (!no_chain_ && !oh_.locality_order.empty() && alg.reorder() && format() == KPMX_FMT_SELL && M >= 160 &&
-            oh_.size() * vectors <= idx_t(1) << 21) {
+            oh_.size() * vectors <= idx_t(1) << 21 &&
+            kpmx::chain_pays(oh_.size(), kpmx::single_step_us(oh_.size(), vw, sizeof(T)), M / 2)) {
             oh_.optimize_for(idx, scale, sizeof(real_t<T>) == 8);
             alg.optimal_size = false;
             if (compute_.several_steps(oh_, format(), std::min<idx_t>(vectors, 64), M)) return alg;

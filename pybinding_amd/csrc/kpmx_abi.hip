@@ -21,6 +21,7 @@
 #include "../../include/kpmx.h"
 #include "kpmx_internal.hpp"
 #include "kpmx_chain.hpp"
+#include "core/chain_rule.hpp"
 
 using namespace kpmx;
 
@@ -1360,17 +1361,6 @@ std::vector<RunTile> run_tiles(const std::vector<Tile>& tiles, int cap) {
 std::vector<RunTile> run_tiles(const kpmx_block* r0, int cap) { return run_tiles(r0->tiles, cap); }
 int diag_cap(const kpmx_mat* h2) { return h2->ctx->tile_cap[h2->scalar]; }
 
-// Whether a run of `steps` single steps of single_us each pays for a plan in its first pass.  A plan
-// with its buffers costs about 0.13 ms and 2 us per thousand rows up to half a millisecond; chained steps
-// save 60 % of launch-bound steps and 40 % or more of the others.  First passes measured with a plan and
-// with single steps: 15 k sites, 80 steps 0.36 and 0.40 ms; 61 k sites, 80 steps 0.48 and 0.52 ms; but
-// 180 k sites, 10 vectors, 50 steps 1.18 and 0.99 ms.  Below 0.4 ms nothing is tried.  The same call
-// always takes the same form, whatever ran before.
-bool chain_pays(int64_t n, double single_us, int64_t steps) {
-    const double plan_us = 130 + std::min(2e-3 * (double)n, 500.0);
-    return std::max(5.5, single_us) * steps >= std::max(400.0, plan_us / (single_us <= 5.5 ? 0.6 : 0.4));
-}
-
 // Whether the diagonal recurrence of this block runs in the chained form: by default on SELL matrices
 // without light-cone limits whose plans promise it to be faster than single steps, where that pays.  A
 // two-step form that the caller has turned on goes first where it applies.  existing: only with plans
@@ -1381,7 +1371,7 @@ bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps
     const auto rts = run_tiles(tiles, diag_cap(h2));
     double single_us = 0;
     for (const RunTile& rt : rts)
-        single_us += std::max(5.5, 3.0 * h2->rows * rt.sub.vw * scalar_bytes(h2->scalar) / 5.6e6);
+        single_us += single_step_us(h2->rows, rt.sub.vw, scalar_bytes(h2->scalar));
     if (!chain_pays(h2->rows, single_us, steps)) return false;
     if (ctx->two_step[h2->scalar] > 0 && !existing)
         for (const RunTile& rt : rts)
@@ -1396,7 +1386,7 @@ bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps
 const ChainPlan* chain_single(const kpmx_mat* h2, int64_t steps) {
     const kpmx_ctx* ctx = h2->ctx;
     if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return nullptr;
-    if (!chain_pays(h2->rows, 3.0 * h2->rows * scalar_bytes(h2->scalar) / 5.6e6, steps)) return nullptr;
+    if (!chain_pays(h2->rows, single_step_us(h2->rows, 1, scalar_bytes(h2->scalar)), steps)) return nullptr;
     return chain_plan(h2, 1);
 }
 
@@ -1511,7 +1501,7 @@ const ChainPlan* backward_chain(const kpmx_tape* T) {
     kpmx_ctx* ctx = h2->ctx;
     if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || ctx->adjoint_variant >= 0) return nullptr;
     if (T->store_all && (h2->scalar == KPMX_F32 || T->vw > chain_adjoint_cols(h2->scalar, T->vw))) return nullptr;
-    if (!chain_pays(h2->rows, 6.0 * (double)T->blk / 5.6e6, T->S)) return nullptr;
+    if (!chain_pays(h2->rows, single_step_us(h2->rows, 2 * T->vw, scalar_bytes(h2->scalar)), T->S)) return nullptr;
     const ChainPlan* P = adjoint_chain_plan(h2, T->vw);
     if (!P) return nullptr;
     try {
@@ -2706,7 +2696,7 @@ const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, 
         !h2->step_rows.empty() || h2->row_order)
         return nullptr;
     const size_t sb = scalar_bytes(h2->scalar);
-    if (!chain_pays(h2->rows, 3.0 * h2->rows * cols * sb / 5.6e6, 2 * steps)) return nullptr;  // both sweeps
+    if (!chain_pays(h2->rows, single_step_us(h2->rows, cols, sb), 2 * steps)) return nullptr;  // both sweeps
     const ChainPlan* P = chain_plan(h2, cols);
     if (!P) return nullptr;
     if (H.plan == P) return H.data ? P : nullptr;
