@@ -368,7 +368,10 @@ struct kpmx_batch {
     // the chained form of run modes 0 and 1 (see kpmx_chain_step.hpp): off once the caller pins a
     // partition, or while the autotuner has found the walkers faster
     bool chain_on = true;
-    bool graph_chain = false;        // the captured graph runs it
+    // what the captured graph's chained launches depend on beside num_moments (null: it runs the walkers,
+    // which compute every column of the padded block)
+    const ChainHolder* graph_chain = nullptr;
+    int64_t graph_nvec = 0, graph_tile_cols = 0;
     std::vector<std::unique_ptr<ChainHolder>> chains;
     void* w2 = nullptr;              // with w0 and w1 its four work vectors
     void* w3 = nullptr;
@@ -3736,7 +3739,8 @@ int kpmx_batch_run(kpmx_batch* b, int64_t M, int use_graph) {
             KPMX_HIP(hipGetLastError());
             return;
         }
-        if (b->graph_moments != M || !b->graph_exec || b->graph_chain != (chain != nullptr)) {
+        if (b->graph_moments != M || !b->graph_exec || b->graph_chain != chain ||
+            (chain && (b->graph_nvec != b->nvec || b->graph_tile_cols != b->tile_cols))) {
             b->drop_graph();
             KPMX_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
             try {
@@ -3750,7 +3754,9 @@ int kpmx_batch_run(kpmx_batch* b, int64_t M, int use_graph) {
             KPMX_HIP(hipStreamEndCapture(ctx->stream, &b->graph));
             KPMX_HIP(hipGraphInstantiate(&b->graph_exec, b->graph, nullptr, nullptr, 0));
             b->graph_moments = M;
-            b->graph_chain = chain != nullptr;
+            b->graph_chain = chain;
+            b->graph_nvec = b->nvec;
+            b->graph_tile_cols = b->tile_cols;
         }
         KPMX_HIP(hipGraphLaunch(b->graph_exec, ctx->stream));
     });

@@ -1,0 +1,113 @@
+"""Checks of the engine's dispatch on a HIP runtime without a device (host_runtime.cpp), one per function:
+which kernels a call launches, what it keeps in graphs and what it does without memory.  Results are
+not looked at (no kernel runs).  `python host_dispatch.py LIBRARY NAME` runs one of them in a process of
+its own, where that runtime takes the place of the real one; test_host_dispatch.py runs them all."""
+import ctypes
+import os
+import sys
+from collections import Counter
+
+import numpy as np
+import scipy.sparse as sp
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path[:0] = [os.path.dirname(HERE), HERE]
+
+CHECKS = {}
+
+
+def check(f):
+    CHECKS[f.__name__] = f
+    return f
+
+
+class Runtime:
+    def __init__(self, path):
+        self.lib = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
+        self.lib.host_runtime_log.restype = ctypes.c_char_p
+        self.lib.host_runtime_used.restype = ctypes.c_size_t
+
+    def launches(self):
+        """Kernel names and their counts since the last call."""
+        return Counter(self.lib.host_runtime_log().decode().split())
+
+    def of(self, f, *args):
+        self.launches()
+        f(*args)
+        return self.launches()
+
+    def captures(self):
+        return self.lib.host_runtime_captures()
+
+    def spare(self, nbytes):
+        """Leaves `nbytes` of device memory (None: plenty)."""
+        self.lib.host_runtime_limit(ctypes.c_size_t(self.lib.host_runtime_used() + nbytes if nbytes is not None else 8 << 30))
+
+    def growth(self, sampled, of_all):
+        """Local rows that each distance adds to a tile, in the sampled and in all tiles."""
+        self.lib.host_runtime_growth(int(sampled), int(of_all))
+
+    def cost(self, kernel, us):
+        self.lib.host_runtime_cost(kernel.encode(), ctypes.c_double(us))
+
+
+def chain(n, dtype=np.float64, width=2):
+    """a matrix of `width` off-diagonal entries per row (a ring with neighbours at 1, 2, ...), one value"""
+    rows = np.repeat(np.arange(n), width)
+    step = np.tile([s for k in range(1, width // 2 + 1) for s in (k, -k)], n)
+    h = sp.csr_matrix((np.full(n * width, 0.3), (rows, (rows + step) % n)), shape=(n, n)).astype(dtype)
+    h.sort_indices()
+    return h
+
+
+def block(n, nvec, dtype=np.float64):
+    return np.ones((nvec, n), dtype=dtype)
+
+
+def chained(launches):
+    return launches["k_chain"]
+
+
+def stepped(launches):
+    return sum(c for k, c in launches.items() if k.startswith("k_step"))
+
+
+@check
+def batch_graph_is_captured_for_its_vectors(rt):
+    """A batch replays a graph only for the vectors it was captured with: each run launches every column
+    group (of 8 fp64, 4 complex128 vectors)."""
+    import abi
+    for dtype, counts, cols in ((np.float64, (20, 32, 17, 32), 8), (np.complex128, (9, 16), 4), (np.float64, (33, 64), 8)):
+        ctx = abi.Ctx(0)
+        b = abi.Batch(ctx, [chain(3000, dtype), chain(5000, dtype)])
+        M = 258
+        runs = []
+        for nvec in counts:
+            b.starters(block(8000, nvec, dtype))
+            plain = rt.of(b.run, M, False)
+            assert chained(plain) and chained(plain) % -(-nvec // cols) == 0
+            graph = rt.of(b.run, M, True)
+            assert rt.of(b.run, M, True) == graph  # a replay
+            runs.append((nvec, chained(graph), chained(plain)))
+        assert all(g == p for _, g, p in runs), runs
+        ctx.close()
+
+
+@check
+def batch_graph_is_captured_for_its_plan(rt):
+    """1 and 4 vectors share a padded block, but not the plan: also where the partial sums of both reach
+    their limit and the buffer does not grow"""
+    import abi
+    ctx = abi.Ctx(0)
+    b = abi.Batch(ctx, [chain(150000), chain(150000)])
+    M = 1 << 18
+    before = rt.captures()
+    for nvec in (1, 4):
+        b.starters(block(300000, nvec))
+        b.run(M, True)
+    assert rt.captures() - before == 2
+    ctx.close()
+
+
+if __name__ == "__main__":
+    CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
