@@ -111,9 +111,9 @@ int kpmx_mat_set_step_rows(kpmx_mat* h2, int64_t num_steps, const int64_t* rows)
 
 /* A locality order of the rows for the tiles of the chained recurrences (no counterpart in the
  * reference): order[i], a permutation, is row i's position; null returns to the matrix's own order.
- * Vectors, moments and the order of every row's sums stay the matrix's.  Plans are built anew; a run
- * captured before must not be replayed.  A matrix whose own order has compact tiles needs none; panel
- * sweeps (Kubo moments) ignore the chained form on a matrix with one. */
+ * Vectors, moments and the order of every row's sums stay the matrix's.  Plans are built and
+ * graphs captured anew.  A matrix whose own order has compact tiles needs none; panel sweeps (Kubo
+ * moments) ignore the chained form on a matrix with one. */
 int kpmx_mat_set_row_order(kpmx_mat* h2, const int32_t* order);
 
 /* Upload starter vectors (host, vector-major num_vectors x n) and keep them resident.

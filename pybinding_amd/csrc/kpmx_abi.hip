@@ -116,6 +116,11 @@ constexpr size_t KPMX_SCRATCH_BYTES = (size_t)64 << 20;
 static __device__ __align__(256) char scratch[KPMX_SCRATCH_BYTES];
 
 namespace {
+uint64_t next_serial() {
+    static std::atomic<uint64_t> next{1};
+    return next++;
+}
+
 std::mutex g_scratch_mu;
 std::vector<void*> g_scratch_ptr;  // device address of `scratch`, per device
 
@@ -217,7 +222,9 @@ struct ChainHolder {
 
 struct kpmx_mat {
     kpmx_ctx* ctx = nullptr;
-    uint64_t serial = 0;  // unique per upload: keys captured graphs (addresses can be reused)
+    // keys captured graphs (addresses can be reused): unique per upload and per row order, which frees the
+    // plans that a captured chained run reads
+    uint64_t serial = 0;
     int scalar = 1;
     int format = KPMX_FMT_CSR;
     int64_t rows = 0, nnz = 0;
@@ -2071,8 +2078,7 @@ int kpmx_mat_upload(kpmx_ctx* ctx, int scalar, int format, int64_t rows, int64_t
         const size_t sb = scalar_bytes(scalar);
         auto m = std::make_unique<kpmx_mat>();
         m->ctx = ctx;
-        static std::atomic<uint64_t> next_serial{1};
-        m->serial = next_serial++;
+        m->serial = next_serial();
         m->scalar = scalar;
         m->format = format;
         m->rows = rows;
@@ -2190,6 +2196,7 @@ int kpmx_mat_set_row_order(kpmx_mat* h2, const int32_t* order) {
             }
         }
         KPMX_HIP(hipStreamSynchronize(ctx->stream));  // queued launches read the plans
+        h2->serial = next_serial();
         h2->chains.clear();
         dev_free(h2->row_order);
         h2->row_order = nullptr;

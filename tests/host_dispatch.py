@@ -109,5 +109,23 @@ def batch_graph_is_captured_for_its_plan(rt):
     ctx.close()
 
 
+@check
+def row_order_drops_captured_runs(rt):
+    """A row order frees the plans that a captured run's launches read: the run is captured again"""
+    import abi
+    n = 6000
+    ctx = abi.Ctx(0)
+    ctx.set_graph_policy(2)
+    mat, blk = ctx.mat(chain(n), fmt=1), ctx.block(block(n, 4))
+    for i, order in enumerate((None, np.arange(n)[::-1], None)):
+        if i:
+            mat.set_row_order(order)
+        before = rt.captures()
+        for repeat in range(3):
+            assert chained(rt.of(abi.moments_diagonal, mat, blk, 258))
+        assert rt.captures() - before == 1, i
+    ctx.close()
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))

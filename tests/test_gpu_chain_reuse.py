@@ -3,8 +3,10 @@ conditions: the results are those of a fresh object, bit for bit."""
 import numpy as np
 import pytest
 
+import abi
 from pybinding_amd import generators
 from pybinding_amd.batch import kpm_batch
+from test_gpu_chain import lattice, starters
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +38,35 @@ def test_batch_with_other_vector_counts(dtype, counts):
         for repeat in range(2):
             assert np.array_equal(kb.moments(M, nvec), tiled)
     kb.close()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_row_order_between_graph_replays(dtype):
+    """a row order frees the plans that a captured run reads: the next run is captured anew"""
+    h = lattice("uniform", dtype=dtype)
+    q = np.random.default_rng(6).permutation(h.shape[0])
+    h2 = h[q][:, q].tocsr()
+    h2.sort_indices()
+    r0, M = starters(h.shape[0], 5, dtype), 162
+
+    def fresh(order):
+        ctx = abi.Ctx(0)
+        mat = ctx.mat(h2, fmt=1)
+        if order is not None:
+            mat.set_row_order(order)
+        mu = abi.moments_diagonal(mat, ctx.block(r0), M)
+        ctx.close()
+        return mu
+
+    ctx = abi.Ctx(0)
+    ctx.set_graph_policy(2)
+    mat, blk = ctx.mat(h2, fmt=1), ctx.block(r0)
+    other = h.shape[0] - 1 - q
+    for i, order in enumerate((None, q, other, None, q)):
+        print("row order", np.dtype(dtype).name, None if order is None else order[:3], flush=True)
+        if i:
+            mat.set_row_order(order)
+        ref = fresh(order)
+        for repeat in range(3):
+            assert np.array_equal(abi.moments_diagonal(mat, blk, M), ref)
+    ctx.close()
