@@ -155,8 +155,9 @@ int kpmx_diagonal_form(const kpmx_mat* h2, int64_t num_vectors, int64_t num_mome
  * diagonal as a dense vector, built at upload when the off-diagonal entries take that few
  * distinct values, for other matrices run as 2).  On fp64 SELL matrices it then also times the
  * LDS two-step form (see kpmx_ctx_set_autotune_two_step) and keeps it, with its column-tile
- * width, when it is faster per vector.  Last it times the chained form: the context keeps it for the
- * scalar type while it is the fastest of all, otherwise the chosen variant (or two-step form) runs. */
+ * width, when it is faster per vector.  Last it times the chained form: unless that
+ * is the fastest of all, this matrix's blocks of this width (its power of two) run the chosen variant
+ * or two-step form from then on; other matrices and widths keep the chained form. */
 int kpmx_autotune_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int* variant);
 /* Pin the diagonal step variant (as numbered above) for one scalar type and vector width on the
  * context, e.g. a choice an earlier autotuning run reported (no counterpart in the reference).

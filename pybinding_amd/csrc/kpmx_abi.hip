@@ -165,10 +165,11 @@ struct kpmx_ctx {
     bool autotune_two_step = true;             // kpmx_autotune_diagonal may choose the LDS two-step form
     bool two_step_auto[4] = {false, false, false, false};  // the two-step settings are the autotuner's
     // the chained form of the diagonal recurrence (kpmx_chain_step.hpp) per scalar type: the default,
-    // off once the caller pins a step variant or a tile width, or while the autotuner has found another
-    // form faster; a two-step form that the caller has asked for goes before it where it applies
-    enum { CHAIN_ON, CHAIN_PINNED_OFF, CHAIN_TUNED_OFF };
-    int chain[4] = {CHAIN_ON, CHAIN_ON, CHAIN_ON, CHAIN_ON};
+    // off once the caller pins a step variant or a tile width; a two-step form that the caller has asked
+    // for goes before it where it applies, one that the autotuner chose does not (chain_tuned_off of the
+    // matrix it was chosen for says so)
+    bool chain[4] = {true, true, true, true};
+    bool two_step_asked(int scalar) const { return two_step[scalar] > 0 && !two_step_auto[scalar]; }
     Workspace work3, work4;  // the third and fourth vector of the two-step recurrence
     int graph_policy = KPMX_GRAPH_NEVER;
     int adjoint_variant = -1;  // adjoint step variant (kpmx_ctx_set_adjoint_variant); -1: the default
@@ -264,6 +265,8 @@ struct kpmx_mat {
     int cmax_width = 0, ctable_size = 0;
     mutable std::vector<std::unique_ptr<ChainHolder>> chains;  // by column width, built on first use
     int32_t* row_order = nullptr;  // kpmx_mat_set_row_order: ChainMatrix::perm, then ::place
+    // bit log2(vw): the autotuner found another form faster for blocks of vw vectors
+    mutable unsigned chain_tuned_off = 0;
     ~kpmx_mat() {
         dev_free(row_order);
         for (void* p : {(void*)cslice_ptr, (void*)cslice_width, (void*)cindices, (void*)ccodes, cdiag, ctable}) dev_free(p);
@@ -1371,19 +1374,28 @@ std::vector<RunTile> run_tiles(const std::vector<Tile>& tiles, int cap) {
 std::vector<RunTile> run_tiles(const kpmx_block* r0, int cap) { return run_tiles(r0->tiles, cap); }
 int diag_cap(const kpmx_mat* h2) { return h2->ctx->tile_cap[h2->scalar]; }
 
+// Whether blocks of vw vectors may run in the chained form on this matrix: SELL, no light cone, not
+// pinned to other forms nor tuned to be slower.
+bool chain_allowed(const kpmx_mat* h2, int vw) {
+    return h2->ctx->chain[h2->scalar] && h2->format == KPMX_FMT_SELL && h2->step_rows.empty() &&
+           !(h2->chain_tuned_off >> log2i(vw) & 1);
+}
+
 // Whether the diagonal recurrence of this block runs in the chained form: by default on SELL matrices
 // without light-cone limits whose plans promise it to be faster than single steps, where that pays.  A
 // two-step form that the caller has turned on goes first where it applies.  existing: only with plans
 // that are there already (nothing is allocated).
 bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps, bool existing = false) {
     const kpmx_ctx* ctx = h2->ctx;
-    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return false;
-    const auto rts = run_tiles(tiles, diag_cap(h2));
+    for (const Tile& t : tiles)
+        if (!chain_allowed(h2, t.vw)) return false;
+    // (a tile width that the autotuner chose for some matrix does not enter)
+    const auto rts = run_tiles(tiles, ctx->two_step_auto[h2->scalar] ? default_tile_cap(h2->scalar) : diag_cap(h2));
     double single_us = 0;
     for (const RunTile& rt : rts)
         single_us += single_step_us(h2->rows, rt.sub.vw, scalar_bytes(h2->scalar));
     if (!chain_pays(h2->rows, single_us, steps)) return false;
-    if (ctx->two_step[h2->scalar] > 0 && !existing)
+    if (ctx->two_step_asked(h2->scalar) && !existing)
         for (const RunTile& rt : rts)
             if (use_two_step(h2, rt.sub)) return false;
     for (const Tile& t : tiles)
@@ -1394,8 +1406,7 @@ bool use_chain(const kpmx_mat* h2, const std::vector<Tile>& tiles, int64_t steps
 // The plan of a one-vector recurrence that collects something else than the diagonal sums, under the
 // same conditions (null: single steps).
 const ChainPlan* chain_single(const kpmx_mat* h2, int64_t steps) {
-    const kpmx_ctx* ctx = h2->ctx;
-    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || !h2->step_rows.empty()) return nullptr;
+    if (!chain_allowed(h2, 1)) return nullptr;
     if (!chain_pays(h2->rows, single_step_us(h2->rows, 1, scalar_bytes(h2->scalar)), steps)) return nullptr;
     return chain_plan(h2, 1);
 }
@@ -1509,7 +1520,7 @@ size_t backward_pair(const kpmx_tape* T) {  // bytes of two work vectors of a co
 const ChainPlan* backward_chain(const kpmx_tape* T) {
     const kpmx_mat* h2 = T->h2;
     kpmx_ctx* ctx = h2->ctx;
-    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || ctx->adjoint_variant >= 0) return nullptr;
+    if (!ctx->chain[h2->scalar] || (h2->chain_tuned_off >> log2i(T->vw) & 1) || ctx->adjoint_variant >= 0) return nullptr;
     if (T->store_all && (h2->scalar == KPMX_F32 || T->vw > chain_adjoint_cols(h2->scalar, T->vw))) return nullptr;
     if (!chain_pays(h2->rows, single_step_us(h2->rows, 2 * T->vw, scalar_bytes(h2->scalar)), T->S)) return nullptr;
     const ChainPlan* P = adjoint_chain_plan(h2, T->vw);
@@ -2248,7 +2259,7 @@ int kpmx_ctx_set_tile_width(kpmx_ctx* ctx, int scalar, int width) {
         KPMX_REQUIRE(width >= 1 && width <= 64 && (width & (width - 1)) == 0, "tile width must be 1, 2, 4, ..., 64");
         ctx->tile_cap[scalar] = width;
         ctx->two_step_auto[scalar] = false;
-        ctx->chain[scalar] = kpmx_ctx::CHAIN_PINNED_OFF;
+        ctx->chain[scalar] = false;
     });
 }
 
@@ -2371,7 +2382,7 @@ namespace {
 // the matrix; false when it does not fit.
 bool chain_noalloc(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, void* mu) {
     kpmx_ctx* ctx = h2->ctx;
-    if (ctx->two_step[h2->scalar] > 0) return false;
+    if (ctx->two_step_asked(h2->scalar)) return false;
     const int64_t steps = M / 2;
     const size_t sb = scalar_bytes(h2->scalar);
     auto align = [](size_t b) { return (b + 255) / 256 * 256; };
@@ -2702,9 +2713,7 @@ struct ChainOpHolder {
 // is short.
 const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, int64_t steps, ChainOpHolder& H) {
     kpmx_ctx* ctx = h2->ctx;
-    if (ctx->chain[h2->scalar] != kpmx_ctx::CHAIN_ON || h2->format != KPMX_FMT_SELL || op->format != KPMX_FMT_SELL ||
-        !h2->step_rows.empty() || h2->row_order)
-        return nullptr;
+    if (!chain_allowed(h2, cols) || op->format != KPMX_FMT_SELL || h2->row_order) return nullptr;
     const size_t sb = scalar_bytes(h2->scalar);
     if (!chain_pays(h2->rows, single_step_us(h2->rows, cols, sb), 2 * steps)) return nullptr;  // both sweeps
     const ChainPlan* P = chain_plan(h2, cols);
@@ -3067,7 +3076,7 @@ int kpmx_ctx_set_step_variant(kpmx_ctx* ctx, int scalar, int vector_width, int v
         KPMX_REQUIRE(variant >= 0 && variant < NUM_TUNE_VARIANTS, "variant out of range");
         ctx->tune[scalar][log2i(vector_width)] = variant;
         ctx->tune_coded[scalar][log2i(vector_width)] = -1;
-        ctx->chain[scalar] = kpmx_ctx::CHAIN_PINNED_OFF;
+        ctx->chain[scalar] = false;
     });
 }
 
@@ -3147,15 +3156,11 @@ void reset_two_step_choice(kpmx_ctx* ctx, int scalar) {
     ctx->two_step_auto[scalar] = false;
 }
 
-// Switches the chained form off while another form is faster per vector and step.
+// Switches the chained form off for this matrix and block width while another form is faster per
+// vector and step.
 void autotune_chain(const kpmx_mat* h2, const kpmx_block* r0, double best_per_vector) {
     kpmx_ctx* ctx = h2->ctx;
-    if (ctx->two_step[h2->scalar] > 0 && !ctx->two_step_auto[h2->scalar]) return;  // the caller's
-    const int two_step = ctx->two_step[h2->scalar];
-    ctx->two_step[h2->scalar] = 0;
-    const bool chain = use_chain(h2, r0->tiles, 1 << 20);
-    ctx->two_step[h2->scalar] = two_step;
-    if (!chain) return;
+    if (ctx->two_step_asked(h2->scalar) || !use_chain(h2, r0->tiles, 1 << 20)) return;
     Tile t = r0->tiles.front();
     t.cols = std::min<int64_t>(t.cols, chain_cols(h2, t));  // one column group
     const double step_bytes = 3.0 * (double)h2->rows * t.cols * scalar_bytes(h2->scalar);
@@ -3172,7 +3177,7 @@ void autotune_chain(const kpmx_mat* h2, const kpmx_block* r0, double best_per_ve
         if (rep == 1 || (rep > 1 && ms < best)) best = ms;
     }
     if (best / ((double)steps * t.cols) > best_per_vector) {
-        ctx->chain[h2->scalar] = kpmx_ctx::CHAIN_TUNED_OFF;
+        h2->chain_tuned_off |= 1u << log2i(t.vw);
     } else if (ctx->two_step_auto[h2->scalar]) {
         reset_two_step_choice(ctx, h2->scalar);
     }
@@ -3185,7 +3190,7 @@ int kpmx_autotune_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int* varian
         kpmx_ctx* ctx = h2->ctx;
         KPMX_HIP(hipSetDevice(ctx->device));
         if (ctx->two_step_auto[h2->scalar]) reset_two_step_choice(ctx, h2->scalar);  // start from the defaults
-        if (ctx->chain[h2->scalar] == kpmx_ctx::CHAIN_TUNED_OFF) ctx->chain[h2->scalar] = kpmx_ctx::CHAIN_ON;
+        h2->chain_tuned_off &= ~(1u << log2i(r0->tiles.front().vw));
         // the first column tile the diagonal recurrence runs (a sub-tile of a wider starter tile)
         const Tile t = stage_run_tile(h2, r0, run_tiles(r0, diag_cap(h2)).front());
         // About 2 GB of vector traffic per timed sample (at least 9 steps, at most 255): small

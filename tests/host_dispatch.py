@@ -127,5 +127,30 @@ def row_order_drops_captured_runs(rt):
     ctx.close()
 
 
+@check
+def tuning_is_of_its_matrix_and_width(rt):
+    """Where the autotuner finds the chained form slower, that matrix's blocks of that width leave it; other
+    matrices and widths on the context do not"""
+    import abi
+    for two_step in (100, 1):  # us of an LDS two-step launch: single steps or the two-step form win
+        ctx = abi.Ctx(0)
+        n, M = 20000, 258
+        tuned, other = ctx.mat(chain(n), fmt=1), ctx.mat(chain(n), fmt=1)
+        blk, narrow = ctx.block(block(n, 16)), ctx.block(block(n, 4))
+        for kernel, us in (("", 0), ("k_step", 4), ("k_step2_lds", two_step), ("k_chain", 1000)):
+            rt.cost(kernel, us)
+        abi.autotune_diagonal(tuned, blk)
+        run = rt.of(abi.moments_diagonal, tuned, blk, M)
+        assert not chained(run) and stepped(run)
+        assert bool(run["k_step2_lds"]) == (two_step == 1)
+        for mat, b in ((tuned, narrow), (other, blk), (other, narrow)):
+            run = rt.of(abi.moments_diagonal, mat, b, M)
+            assert chained(run) and not stepped(run), run
+        rt.cost("k_chain", 1)
+        abi.autotune_diagonal(tuned, blk)  # the next tuning decides anew
+        assert chained(rt.of(abi.moments_diagonal, tuned, blk, M))
+        ctx.close()
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
