@@ -3156,13 +3156,16 @@ void reset_two_step_choice(kpmx_ctx* ctx, int scalar) {
     ctx->two_step_auto[scalar] = false;
 }
 
-// Switches the chained form off for this matrix and block width while another form is faster per
-// vector and step.
+// Switches the chained form off for this matrix and block width while another form, which takes
+// `best_per_vector` milliseconds per column of its column tiles and step, is faster on the block's
+// first starter tile.  Both run every column that they would compute in earnest: the other form its
+// padded column tiles, the chain its column groups, side by side where they fit.
 void autotune_chain(const kpmx_mat* h2, const kpmx_block* r0, double best_per_vector) {
     kpmx_ctx* ctx = h2->ctx;
     if (ctx->two_step_asked(h2->scalar) || !use_chain(h2, r0->tiles, 1 << 20)) return;
-    Tile t = r0->tiles.front();
-    t.cols = std::min<int64_t>(t.cols, chain_cols(h2, t));  // one column group
+    const Tile& t = r0->tiles.front();
+    double other = 0;  // milliseconds per step
+    for (const RunTile& rt : run_tiles({t}, diag_cap(h2))) other += best_per_vector * rt.sub.vw;
     const double step_bytes = 3.0 * (double)h2->rows * t.cols * scalar_bytes(h2->scalar);
     const int64_t steps = std::max<int64_t>(24, std::min<int64_t>(256, (int64_t)(4e9 / step_bytes)));
     double* sums = static_cast<double*>(ctx->sums.get((size_t)steps * 4 * t.vw * sizeof(double)));
@@ -3176,7 +3179,7 @@ void autotune_chain(const kpmx_mat* h2, const kpmx_block* r0, double best_per_ve
         KPMX_HIP(hipEventElapsedTime(&ms, ctx->t0, ctx->t1));
         if (rep == 1 || (rep > 1 && ms < best)) best = ms;
     }
-    if (best / ((double)steps * t.cols) > best_per_vector) {
+    if (best / (double)steps > other) {
         h2->chain_tuned_off |= 1u << log2i(t.vw);
     } else if (ctx->two_step_auto[h2->scalar]) {
         reset_two_step_choice(ctx, h2->scalar);

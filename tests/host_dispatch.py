@@ -152,5 +152,27 @@ def tuning_is_of_its_matrix_and_width(rt):
         ctx.close()
 
 
+@check
+def tuning_times_what_runs(rt):
+    """The autotuner compares whole starter tiles: all column groups of the chained form, side by side as
+    they run, and the padded columns of single steps"""
+    import abi
+    n, M = 3000, 514
+    # 32 vectors: two column tiles a step, or four groups in one launch of 12 steps; 3: a block of 4
+    for nvec, launch in ((32, 60), (3, 60)):
+        ctx = abi.Ctx(0)
+        ctx.set_autotune_two_step(False)
+        mat, blk = ctx.mat(chain(n), fmt=1), ctx.block(block(n, nvec))
+        for kernel, us in (("", 0), ("k_step", 5.5), ("k_chain", launch), ("k_chain_", 0)):
+            rt.cost(kernel, us)
+        abi.autotune_diagonal(mat, blk)
+        steps, _ = abi.diagonal_form(mat, nvec, M)
+        assert steps == 12, (nvec, steps)  # 5 us a step, against 11 and 5.5
+        rt.cost("k_chain", 12 * (12 if nvec == 32 else 6))
+        abi.autotune_diagonal(mat, blk)
+        assert abi.diagonal_form(mat, nvec, M)[0] == 1
+        ctx.close()
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
