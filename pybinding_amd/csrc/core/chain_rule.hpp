@@ -15,8 +15,9 @@ inline double single_step_us(int64_t n, int64_t vw, size_t scalar) {
 // with its buffers costs about 0.13 ms and 2 us per thousand rows up to half a millisecond; chained steps
 // save 60 % of launch-bound steps and 40 % or more of the others.  First passes measured with a plan and
 // with single steps: 15 k sites, 80 steps 0.36 and 0.40 ms; 61 k sites, 80 steps 0.48 and 0.52 ms; but
-// 180 k sites, 10 vectors, 50 steps 1.18 and 0.99 ms.  Below 0.4 ms nothing is tried.  The same call
-// always takes the same form, whatever ran before.
+// 180 k sites, 10 vectors, 50 steps 1.18 and 0.99 ms.  Below 0.4 ms nothing is tried.  What ran
+// before does not enter, so the same call takes the same form (but for calls that build no plans and use
+// one that is there, and for plans that there was no memory for).
 inline bool chain_pays(int64_t n, double single_us, int64_t steps) {
     const double plan_us = 130 + std::min(2e-3 * (double)n, 500.0);
     return single_us * (double)steps >= std::max(400.0, plan_us / (single_us <= 5.5 ? 0.6 : 0.4));

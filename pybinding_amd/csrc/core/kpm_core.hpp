@@ -235,9 +235,10 @@ public:
     idx_t size() const { return original->rows; }
 
     // `whole_system`: the calculation does without the slice map (DOS, moments, conductivity, LDOS
-    // and Green's functions whose recurrence is faster without a light cone); the GPU then prefers `locality_order` (e.g. sites along a space-filling curve) when one is set,
-    // because the moments do not depend on the site order and a compact order keeps the gathered
-    // vector rows of a sweep in L2.  Otherwise the reference's BFS reorder is used.
+    // and Green's functions whose recurrence is faster without a light cone); the GPU then prefers
+    // `locality_order` (e.g. sites along a space-filling curve) when one is set, because the moments do
+    // not depend on the site order and a compact order keeps the gathered vector rows of a sweep in L2.
+    // Otherwise the reference's BFS reorder is used.
     void optimize_for(Indices const& idx, Scale<> scale, bool whole_system = false) {
         for (auto const* list : {&idx.src, &idx.dest})
             for (auto v : *list)

@@ -84,20 +84,21 @@ public:
     // light cone of the BFS order saves work, but pays a launch per step (4.7 us); the chained recurrence
     // sweeps the whole system several steps per launch.  Up to 2^21 vector elements such a step takes
     // less than that launch (137 k sites: 0.9 us, 2.1 M sites: 4.8 us); beyond, in runs too short for a
-    // chain to pay (asked before anything is prepared for it) and where no chain fits, the cone stays.  In double precision the matrix keeps the locality
-    // order from site to site (no BFS and upload for each); in 32 bits it stays BFS-ordered, so that every
-    // row's sum rounds as under the cone, and only the chain's tiles follow the locality order.
+    // chain to pay (asked before anything is prepared for it) and where no chain fits (remembered for the
+    // block width, as plans are), the cone stays.  In double precision the matrix keeps the locality order
+    // from site to site (no BFS and upload for each); in 32 bits it stays BFS-ordered, so that every row's
+    // sum rounds as under the cone, and only the chain's tiles follow the locality order.
     AlgorithmConfig optimize_for_sites(Indices const& idx, Scale<> scale, idx_t vectors, idx_t M) {
         auto alg = cfg_.algorithm;
         idx_t vw = 1;
         while (vw < vectors && vw < 64) vw <<= 1;
-        if (!no_chain_ && !oh_.locality_order.empty() && alg.reorder() && format() == KPMX_FMT_SELL && M >= 160 &&
+        if (!(no_chain_ & vw) && !oh_.locality_order.empty() && alg.reorder() && format() == KPMX_FMT_SELL && M >= 160 &&
             oh_.size() * vectors <= idx_t(1) << 21 &&
             kpmx::chain_pays(oh_.size(), kpmx::single_step_us(oh_.size(), vw, sizeof(T)), M / 2)) {
             oh_.optimize_for(idx, scale, sizeof(real_t<T>) == 8);
             alg.optimal_size = false;
             if (compute_.several_steps(oh_, format(), std::min<idx_t>(vectors, 64), M)) return alg;
-            no_chain_ = true;
+            no_chain_ |= vw;
         }
         oh_.optimize_for(idx, scale);
         return cfg_.algorithm;
@@ -196,6 +197,7 @@ public:
     void set_locality_order(std::vector<int32_t> order) override {
         if (!order.empty() && (idx_t)order.size() != h_.rows) throw std::invalid_argument("site order has the wrong size");
         oh_.locality_order = std::move(order);
+        no_chain_ = 0;
     }
 
     // Raw access for the engine's own tools
@@ -228,7 +230,7 @@ private:
     Config cfg_;
     OptimizedHamiltonian<T> oh_;
     HipCompute<T> compute_;
-    bool no_chain_ = false;  // the locality order has no chained recurrence
+    idx_t no_chain_ = 0;  // block widths (powers of two, added) without a chained recurrence on the locality order
     int kubo_mode_ = KPMX_KUBO_FP64;
     Stats stats_;
     double min_ = 0, max_ = 0;

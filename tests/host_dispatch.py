@@ -174,5 +174,26 @@ def tuning_times_what_runs(rt):
         ctx.close()
 
 
+def flake(side=25, dtype="float64"):
+    import pybinding_amd as pb
+    from pybinding_amd.repository import graphene
+    return pb.Model(graphene.monolayer(), pb.rectangle(side, side), *([pb.force_double_precision()] if dtype == "float64" else []))
+
+
+@check
+def sites_without_a_chain_decide_for_their_width_only(rt):
+    """An LDOS of many sites for which no plan fits keeps the light cone, and that of one site still takes
+    the chained form, in either order of the calls"""
+    import pybinding_amd as pb
+    rt.growth(600, 600)  # two distances exceed a tile of 8 columns, not one of a single column
+    energy = np.linspace(-3, 3, 20)
+    for dtype in ("float64", "float32"):
+        for calls in ((1, 32, 1, 32), (32, 1, 32, 1)):
+            kpm = pb.kpm(flake(dtype=dtype), energy_range=(-9, 9), silent=True)
+            for sites in calls:
+                run = rt.of(kpm.impl.calc_ldos_indices, energy, 0.05, list(range(100, 100 + sites)))
+                assert bool(chained(run)) == (sites == 1) and bool(stepped(run)) == (sites > 1), (dtype, calls, sites, run)
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
