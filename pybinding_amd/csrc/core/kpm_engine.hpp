@@ -269,12 +269,17 @@ public:
         if (!oh.used_locality && ordered_ != oh.version) {
             std::vector<int32_t> order((size_t)oh.size());
             for (size_t s = 0; s < order.size(); ++s) order[(size_t)oh.reorder_map[s]] = oh.locality_order[s];
-            check(kpmx_mat_set_row_order(h2, order.data()));
+            const int rc = kpmx_mat_set_row_order(h2, order.data());
+            if (rc == KPMX_ENOMEM) return false;
+            check(rc);
             ordered_ = oh.version;
         }
         int steps = 0, cols = 0;
         check(kpmx_diagonal_form(h2, num_vectors, num_moments, &steps, &cols));
-        return steps > 1;
+        if (steps > 1) return true;
+        if (ordered_) check(kpmx_mat_set_row_order(h2, nullptr));  // its memory is needed no more
+        ordered_ = 0;
+        return false;
     }
 
     // The light cone of the reference's optimal_size algorithm: rows computed by every step of

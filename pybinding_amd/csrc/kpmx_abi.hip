@@ -225,7 +225,7 @@ struct kpmx_mat {
     kpmx_ctx* ctx = nullptr;
     // keys captured graphs (addresses can be reused): unique per upload and per row order, which frees the
     // plans that a captured chained run reads
-    uint64_t serial = 0;
+    mutable uint64_t serial = 0;
     int scalar = 1;
     int format = KPMX_FMT_CSR;
     int64_t rows = 0, nnz = 0;
@@ -1214,6 +1214,7 @@ const ChainPlan* chain_plan(const kpmx_mat* h2, const ChainMatrix& m, int cols, 
         if (e.code != KPMX_ENOMEM) throw;
         dev_free(H->data);
         H->data = nullptr;  // no memory for the plan: single steps
+        h2->ctx->aux2.release();
     }
     h2->chains.push_back(std::move(H));
     return h2->chains.back()->data ? &h2->chains.back()->plan : nullptr;
@@ -1445,15 +1446,11 @@ void chain_steps(const kpmx_mat* h2, const ChainPlan& P, int cols, const void* x
 bool use_tape_chain(const kpmx_mat* h2, const Tile& t, int64_t steps) {
     if (h2->row_order || !use_chain(h2, {t}, steps) || chain_plan(h2, chain_cols(h2, t))->steps < 3) return false;
     kpmx_ctx* ctx = h2->ctx;
+    // as large as the backward pass needs them: growing a buffer frees it first
     const size_t column = (size_t)h2->rows * scalar_bytes(h2->scalar);
-    try {  // as large as the backward pass needs them: growing a buffer frees it first
-        for (Workspace* w : {&ctx->work0, &ctx->work1}) w->get(column * t.vw);
-        for (Workspace* w : {&ctx->work3, &ctx->work4}) w->get(column * 4 * chain_adjoint_cols(h2->scalar, t.vw));
-        size_chain(h2, t, steps);
-    } catch (const Error& e) {
-        if (e.code != KPMX_ENOMEM) throw;
-        return false;
-    }
+    for (Workspace* w : {&ctx->work0, &ctx->work1}) w->get(column * t.vw);
+    for (Workspace* w : {&ctx->work3, &ctx->work4}) w->get(column * 4 * chain_adjoint_cols(h2->scalar, t.vw));
+    size_chain(h2, t, steps);
     return true;
 }
 void run_tape_chain(const kpmx_tape* T, const Tile& t, double* sums) {
@@ -1523,17 +1520,7 @@ const ChainPlan* backward_chain(const kpmx_tape* T) {
     if (!ctx->chain[h2->scalar] || (h2->chain_tuned_off >> log2i(T->vw) & 1) || ctx->adjoint_variant >= 0) return nullptr;
     if (T->store_all && (h2->scalar == KPMX_F32 || T->vw > chain_adjoint_cols(h2->scalar, T->vw))) return nullptr;
     if (!chain_pays(h2->rows, single_step_us(h2->rows, 2 * T->vw, scalar_bytes(h2->scalar)), T->S)) return nullptr;
-    const ChainPlan* P = adjoint_chain_plan(h2, T->vw);
-    if (!P) return nullptr;
-    try {
-        ctx->work3.get(2 * backward_pair(T));
-        ctx->work4.get(2 * backward_pair(T));
-        ctx->partials.get((size_t)h2->rows * 4 * sizeof(double));
-    } catch (const Error& e) {
-        if (e.code != KPMX_ENOMEM) throw;
-        return nullptr;
-    }
-    return P;
+    return adjoint_chain_plan(h2, T->vw);
 }
 // Leaves lambda_1 in lam1 (a block like the starters) and the steps' gradient in grad (SELL order).
 // Column groups run one after the other on packed work vectors.  Between kept pairs, v_j is rebuilt from
@@ -1595,6 +1582,37 @@ void run_backward_chain(const kpmx_tape* T, const ChainPlan& P, const std::vecto
     KPMX_HIP(hipGetLastError());
 }
 
+// An entry point that may take the chained form.  Where memory runs out while the matrix holds plans,
+// they and the workspaces are given back and the call starts again, on single steps; these widths then
+// keep single steps, unless that was not enough either.
+template <class F>
+int guarded_chain(const kpmx_mat* h2, F body) {
+    return guarded([&] {
+        try {
+            body();
+            return;
+        } catch (const Error& e) {
+            if (e.code != KPMX_ENOMEM || !h2 || h2->chains.empty()) throw;
+        }
+        kpmx_ctx* ctx = h2->ctx;
+        (void)hipStreamSynchronize(ctx->stream);  // queued launches read the plans
+        h2->serial = next_serial();               // and captured ones
+        for (auto& c : h2->chains) {
+            dev_free(c->data);
+            c->data = nullptr;
+        }
+        for (Workspace* w : {&ctx->partials, &ctx->sums, &ctx->work0, &ctx->work1, &ctx->work2, &ctx->work3, &ctx->work4,
+                             &ctx->aux0, &ctx->aux1, &ctx->aux2, &ctx->panel_l, &ctx->panel_r})
+            w->release();
+        try {
+            body();
+        } catch (...) {
+            h2->chains.clear();
+            throw;
+        }
+    });
+}
+
 // copies a sub-tile's columns into `dst` (default: work2, sized beforehand) and returns the tile
 // to run
 Tile stage_run_tile(const kpmx_mat* h2, const kpmx_block* r0, const RunTile& rt, void* dst = nullptr) {
@@ -1640,15 +1658,7 @@ void diag_run(const kpmx_mat* h2, const kpmx_block* r0c, int64_t M) {
     KPMX_REQUIRE(M >= 2 && M % 2 == 0, "num_moments must be even and >= 2");
     kpmx_ctx* ctx = h2->ctx;
     const int64_t steps = M / 2;
-    bool chain = use_chain(h2, r0->tiles, steps);
-    if (chain) {
-        try {
-            for (const Tile& t : r0->tiles) size_chain(h2, t, steps);
-        } catch (const Error& e) {
-            if (e.code != KPMX_ENOMEM) throw;
-            chain = false;  // no memory for its work vectors: single steps
-        }
-    }
+    const bool chain = use_chain(h2, r0->tiles, steps);
     const int cap = chain ? 64 : diag_cap(h2);
     r0->sums_chain = chain;
     const auto rts = run_tiles(r0, cap);
@@ -1657,6 +1667,7 @@ void diag_run(const kpmx_mat* h2, const kpmx_block* r0c, int64_t M) {
         r0->drop_graph();
         for (auto* s : r0->sums) dev_free(s);
         r0->sums.clear();
+        r0->sums_moments = 0;  // until they are there again
         for (auto& rt : rts) r0->sums.push_back(dev_alloc((size_t)steps * 4 * rt.sub.vw * sizeof(double)));
         r0->sums_moments = M;
         r0->sums_cap = cap;
@@ -2349,7 +2360,7 @@ int kpmx_diagonal_form(const kpmx_mat* h2, int64_t num_vectors, int64_t num_mome
 }
 
 int kpmx_moments_diagonal_run(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments) {
-    return guarded([&] {
+    return guarded_chain(h2, [&] {
         KPMX_REQUIRE(h2 && r0, "null matrix or starter block");
         KPMX_HIP(hipSetDevice(h2->ctx->device));
         diag_run(h2, r0, num_moments);
@@ -2365,7 +2376,7 @@ int kpmx_moments_diagonal_fetch(const kpmx_mat* h2, const kpmx_block* r0, int64_
 }
 
 int kpmx_moments_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, void* mu) {
-    return guarded([&] {
+    return guarded_chain(h2, [&] {
         KPMX_REQUIRE(h2 && r0 && mu, "null argument");
         KPMX_HIP(hipSetDevice(h2->ctx->device));
         diag_run(h2, r0, num_moments);
@@ -2476,7 +2487,7 @@ int kpmx_moments_diagonal_noalloc(const kpmx_mat* h2, const kpmx_block* r0, int6
 
 int kpmx_moments_generic(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, const void* beta, int64_t op_nnz,
                          const int32_t* op_indptr, const int32_t* op_indices, const void* op_values, void* mu) {
-    return guarded([&] {
+    return guarded_chain(h2, [&] {
         check_pair(h2, r0);
         KPMX_REQUIRE(beta && mu, "null beta or output");
         KPMX_REQUIRE(M >= 2, "num_moments must be >= 2");
@@ -2557,7 +2568,7 @@ int kpmx_moments_generic(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, co
 
 int kpmx_moments_multi_unit(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, int64_t ndest, const int32_t* dest,
                             void* mu) {
-    return guarded([&] {
+    return guarded_chain(h2, [&] {
         check_pair(h2, r0);
         KPMX_REQUIRE(mu && (ndest == 0 || dest), "null output or dest");
         KPMX_REQUIRE(M >= 2, "num_moments must be >= 2");
@@ -2709,8 +2720,7 @@ struct ChainOpHolder {
 };
 
 // The plan of panel sweeps with an operator applied in them (H.op), under the conditions of the
-// diagonal recurrence; null where the operator couples a tile to rows beyond its neighbours or memory
-// is short.
+// diagonal recurrence; null where the operator couples a tile to rows beyond its neighbours.
 const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, int64_t steps, ChainOpHolder& H) {
     kpmx_ctx* ctx = h2->ctx;
     if (!chain_allowed(h2, cols) || op->format != KPMX_FMT_SELL || h2->row_order) return nullptr;
@@ -2736,15 +2746,7 @@ const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, 
     o.rows = (int)P->tile_rows;
     const size_t cells = (size_t)P->ntiles * o.groups * o.rows;
     const size_t lidx = (cells * sizeof(ushort4) + 255) / 256 * 256, vals = (cells * 4 * sb + 255) / 256 * 256;
-    try {
-        H.data = static_cast<char*>(dev_alloc(lidx + vals + sizeof(int32_t)));
-        for (Workspace* w : {&ctx->work0, &ctx->work1, &ctx->work3, &ctx->work4}) w->get((size_t)h2->rows * cols * sb);
-    } catch (const Error& e) {
-        if (e.code != KPMX_ENOMEM) throw;
-        dev_free(H.data);
-        H.data = nullptr;
-        return nullptr;
-    }
+    H.data = static_cast<char*>(dev_alloc(lidx + vals + sizeof(int32_t)));
     o.lidx = reinterpret_cast<ushort4*>(H.data);
     o.vals = H.data + lidx;
     int32_t* missing = reinterpret_cast<int32_t*>(H.data + lidx + vals);
@@ -2767,7 +2769,7 @@ const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, 
 
 int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr, const kpmx_block* r0, int64_t M,
                       int mode, void* mu_nm) {
-    return guarded([&] {
+    return guarded_chain(h2, [&] {
         check_pair(h2, r0);
         KPMX_REQUIRE(vl && vr && mu_nm, "null argument");
         KPMX_REQUIRE(mode == KPMX_KUBO_FP64 || mode == KPMX_KUBO_FP32_SPLIT || mode == KPMX_KUBO_BF16X3,
@@ -3188,7 +3190,7 @@ void autotune_chain(const kpmx_mat* h2, const kpmx_block* r0, double best_per_ve
 }  // namespace
 
 int kpmx_autotune_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int* variant) {
-    return guarded([&] {
+    return guarded_chain(h2, [&] {
         check_pair(h2, r0);
         kpmx_ctx* ctx = h2->ctx;
         KPMX_HIP(hipSetDevice(ctx->device));
@@ -3664,10 +3666,15 @@ const ChainHolder* batch_chain(kpmx_batch* b, int64_t steps) {
         }
     } catch (const Error& e) {
         if (e.code != KPMX_ENOMEM) throw;
-        if (H) {
-            dev_free(H->data);
-            H->data = nullptr;
-        }
+        // no memory for the plan or its vectors: what there is of them is given back
+        KPMX_HIP(hipStreamSynchronize(ctx->stream));
+        b->drop_graph();
+        for (void* p : {(void*)H->data, b->w2, b->w3, (void*)b->chain_partials}) dev_free(p);
+        H->data = nullptr;
+        b->w2 = b->w3 = nullptr;
+        b->chain_partials = nullptr;
+        b->chain_partials_bytes = 0;
+        ctx->aux2.release();
         return nullptr;
     }
     return H;
@@ -3958,7 +3965,7 @@ int kpmx_batch_destroy(kpmx_batch* b) {
 
 int kpmx_adjoint_forward(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, int64_t checkpoint, void* mu,
                          kpmx_tape** out) {
-    return guarded([&] {
+    return guarded_chain(h2, [&] {
         check_pair(h2, r0);
         KPMX_REQUIRE(out, "null output");
         KPMX_REQUIRE(M >= 4 && M % 2 == 0, "num_moments must be even and >= 4");
@@ -4059,7 +4066,7 @@ int kpmx_adjoint_forward(const kpmx_mat* h2, const kpmx_block* r0, int64_t M, in
 }
 
 int kpmx_adjoint_backward(kpmx_tape* T, const double* w, double* grad) {
-    return guarded([&] {
+    return guarded_chain(T ? T->h2 : nullptr, [&] {
         KPMX_REQUIRE(T && w && grad, "null argument");
         const kpmx_mat* h2 = T->h2;
         kpmx_ctx* ctx = h2->ctx;

@@ -195,5 +195,69 @@ def sites_without_a_chain_decide_for_their_width_only(rt):
                 assert bool(chained(run)) == (sites == 1) and bool(stepped(run)) == (sites > 1), (dtype, calls, sites, run)
 
 
+@check
+def memory_for_single_steps_is_enough(rt):
+    """Under every limit on device memory with which a call succeeds on single steps (a pinned tile width, the
+    light cone) it succeeds where the chained form is the default: plans and their vectors are given up"""
+    import abi
+    import pybinding_amd as pb
+    n, M = 30000, 258
+    h = chain(n)
+    w = np.ones(M)
+
+    def on_context(call):
+        def run(single):
+            ctx = abi.Ctx(0)
+            try:
+                if single:
+                    ctx.set_tile_width(np.float64, 16)
+                mats = [ctx.mat(h, fmt=1) for _ in range(3)]
+                blocks = {v: ctx.block(block(n, v)) for v in (1, 4, 16)}
+                call(ctx, mats, blocks)
+            finally:
+                ctx.close()
+        return run
+
+    def ldos(single):
+        kpm = pb.kpm(model, energy_range=(-9, 9), silent=True, **(dict(site_order="bfs") if single else {}))
+        kpm.impl.calc_ldos_indices(np.linspace(-3, 3, 20), 0.05, [100])
+        kpm.impl.calc_greens_vector(5, [6, 7], np.linspace(-3, 3, 20), 0.05)
+
+    model = flake(20, "float32")
+    calls = {
+        "diagonal": on_context(lambda c, m, b: abi.moments_diagonal(m[0], b[16], M)),
+        "generic": on_context(lambda c, m, b: abi.moments_generic(m[0], b[4], M, np.ones(n))),
+        "generic after diagonal": on_context(lambda c, m, b: (abi.moments_diagonal(m[0], b[1], M),
+                                                              abi.moments_generic(m[0], b[4], M, np.ones(n)))),
+        "multi_unit": on_context(lambda c, m, b: abi.moments_multi_unit(m[0], b[1], M, [1, 2, 3])),
+        "kubo": on_context(lambda c, m, b: abi.kubo_moments(m[0], m[1], m[2], b[1], 100)),
+        "gradient": on_context(lambda c, m, b: abi.adjoint_diagonal(m[0], b[16], M, w, 64)),
+        "autotune": on_context(lambda c, m, b: abi.autotune_diagonal(m[0], b[4])),
+        "ldos": ldos,
+    }
+
+    def fits(call, single, limit):
+        rt.lib.host_runtime_limit(ctypes.c_size_t(limit))
+        try:
+            rt.launches()
+            call(single)
+            return True
+        except RuntimeError as e:
+            assert "hipMalloc" in str(e) or "do not fit" in str(e), e
+            return False
+
+    for name, call in calls.items():
+        rt.lib.host_runtime_limit(ctypes.c_size_t(8 << 30))
+        assert fits(call, True, 8 << 30) and not chained(rt.launches()), name
+        assert fits(call, False, 8 << 30) and chained(rt.launches()), name
+        low, high = 0, 8 << 30  # the least memory for single steps
+        while high - low > 4096:
+            mid = (low + high) // 2
+            low, high = (low, mid) if fits(call, True, mid) else (mid, high)
+        for extra in [0] + [int(2e5 * 1.35 ** k) for k in range(14)]:
+            if fits(call, True, high + extra):
+                assert fits(call, False, high + extra), (name, high, extra)
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
