@@ -2719,6 +2719,26 @@ struct ChainOpHolder {
     ~ChainOpHolder() { dev_free(data); }
 };
 
+// Columns of the chained sweeps that write the panels of a group of g vectors (0: single steps, which
+// advance all g in one launch).  Panels exist for the widest rows and for single columns, one after
+// another.  Single columns: one or two pay everywhere (160 moments, 20 k to 524 k sites: 1.07 to 3.8 times as
+// fast); four do on small systems, where both are launches (20 k sites, before and now: fp64 2.53 and 1.90 ms,
+// complex64 3.07 and 2.73 ms; 60 k sites 2.60 and 2.60, 4.61 and 4.85 ms), and in fp64 again once the single
+// steps are bound by memory (361 k sites 9.9 and 8.0 ms); fp32 groups of eight are slower (2.4 and 3.8 ms on
+// 20 k sites, 9.0 and 10.3 ms on 137 k).  Widest rows: up to three groups pay everywhere, more where their
+// vectors are large enough (complex128 on 20 k sites: 32 vectors 8.6 and 11.0 ms; on 60 k sites 24.5 and 24.2;
+// fp64, 64 vectors: 5 k sites 5.0 and 5.5 ms, 20 k sites 12.0 and 8.7 ms).
+int panel_columns(int scalar, int64_t n, int g) {
+    const int widest = chain_max_cols(scalar);
+    if (g < widest) {
+        const bool four = n <= (is_complex(scalar) ? 20000 : 32768) || (scalar == KPMX_F64 && n >= 320000);
+        return g <= 2 || (g == 4 && four) ? 1 : 0;
+    }
+    static const double least[4] = {0, 4e6, 8e6, 24e6};  // bytes of a group's vectors
+    const bool many = g / widest >= (scalar == KPMX_F64 ? 8 : 4);
+    return many && (double)n * g * scalar_bytes(scalar) < least[scalar] ? 0 : widest;
+}
+
 // The plan of panel sweeps with an operator applied in them (H.op), under the conditions of the
 // diagonal recurrence; null where the operator couples a tile to rows beyond its neighbours.
 const ChainPlan* chain_panels(const kpmx_mat* h2, const kpmx_mat* op, int cols, int64_t steps, ChainOpHolder& H) {
@@ -2815,9 +2835,8 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
             if (split) g = std::min(g, 4);
             for (int64_t c0 = 0; c0 < full.cols; c0 += g) {
                 const int64_t cols = std::min<int64_t>(g, full.cols - c0);
-                // panels from the chained sweeps, in groups of its widest rows or single columns
-                const int pcols = g >= chain_max_cols(sc) ? chain_max_cols(sc) : 1;
-                const ChainPlan* chain = split ? nullptr : chain_panels(h2, vr, pcols, M - 1, vop);
+                const int pcols = split ? 0 : panel_columns(sc, n, g);
+                const ChainPlan* chain = pcols ? chain_panels(h2, vr, pcols, M - 1, vop) : nullptr;
                 // this group's starters r (n x g), and vl r (n x g)
                 void* Pr = ctx->aux0.get((size_t)n * g * sb);
                 if (g == full.vw) {

@@ -259,5 +259,28 @@ def memory_for_single_steps_is_enough(rt):
                 assert fits(call, False, high + extra), (name, high, extra)
 
 
+@check
+def kubo_panels_take_the_chain_where_it_pays(rt):
+    """Panels of the chain's widest rows where not many groups of small vectors run one after another, and
+    of single columns for up to two vectors, for four on small systems and in fp64 on large ones; other
+    groups advance all their vectors in single steps"""
+    import abi
+    M = 160
+    for dtype, n, forms in ((np.float32, 20000, {1: 1, 2: 1, 3: 1, 8: 0, 16: 1, 64: 1}), (np.float32, 40000, {2: 1, 4: 0}),
+                            (np.float64, 20000, {4: 1, 8: 1, 64: 1}), (np.float64, 5000, {64: 0}),
+                            (np.float64, 60000, {2: 1, 4: 0}), (np.float64, 400000, {4: 1}),
+                            (np.complex64, 40000, {2: 1, 4: 0, 8: 1}), (np.complex64, 5000, {4: 1, 32: 0}),
+                            (np.complex64, 400000, {4: 0}), (np.complex128, 20000, {1: 1, 2: 1, 4: 1, 8: 1, 16: 0, 32: 0}),
+                            (np.complex128, 120000, {16: 1})):
+        h = chain(n, dtype)
+        ctx = abi.Ctx(0)
+        mat, v = ctx.mat(h, fmt=1), ctx.mat(h, fmt=1)
+        for nvec, form in forms.items():
+            run = rt.of(abi.kubo_moments, mat, v, v, ctx.block(block(n, nvec, dtype)), M)
+            # single launches beside the chain: the left operator, and the right one on a group's last vector
+            assert bool(chained(run)) == bool(form) and (stepped(run) < M) == bool(form), (dtype, n, nvec, run)
+        ctx.close()
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
