@@ -383,10 +383,7 @@ struct kpmx_batch {
     const ChainHolder* graph_chain = nullptr;
     int64_t graph_nvec = 0, graph_tile_cols = 0;
     std::vector<std::unique_ptr<ChainHolder>> chains;
-    void* w2 = nullptr;              // with w0 and w1 its four work vectors
-    void* w3 = nullptr;
-    double* chain_partials = nullptr;
-    size_t chain_partials_bytes = 0;
+    Workspace chain_work;            // two work vectors beside w0 and w1, then partial sums
     double* sums = nullptr;
     int64_t sums_steps = 0;
     hipGraph_t graph = nullptr;
@@ -403,7 +400,7 @@ struct kpmx_batch {
         drop_graph();
         for (void* p : {(void*)slice_ptr, (void*)slice_width, (void*)slice_sys, (void*)sidx, svals, (void*)tile_begin,
                         (void*)slot_begin, (void*)slot_index, (void*)slot_first, r0, w0, w1, (void*)partials, (void*)partials2,
-                        (void*)barrier, w2, w3, (void*)chain_partials, (void*)sums, (void*)cslice_ptr, (void*)cslice_width, (void*)cidx, (void*)ccodes,
+                        (void*)barrier, (void*)sums, (void*)cslice_ptr, (void*)cslice_width, (void*)cidx, (void*)ccodes,
                         cdiag, ctable, (void*)ctab_off})
             dev_free(p);
     }
@@ -1070,7 +1067,17 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     if (heights.empty()) return;
     constexpr int ST = CHAIN_MAX_STEPS + 1;
     std::vector<int32_t> ring(heights.size() * CHAIN_SAMPLES * ST);
-    int32_t* d = static_cast<int32_t*>(ctx->aux2.get(ring.size() * sizeof(int32_t)));
+    auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
+    // first rows, ring counts and halo rows of `tiles` tiles of at most `h` rows
+    auto scratch_bytes = [&](double tiles, int h) {
+        return pad((size_t)(tiles + 1) * sizeof(int32_t)) + pad((size_t)tiles * ST * sizeof(int32_t)) +
+               (size_t)tiles * std::min(CHAIN_MAX_HALO, cap - h) * sizeof(int32_t);
+    };
+    // scratch of the samples and, in the same allocation (growing it later took 0.2 ms on 1 M rows), of any
+    // choice of tiles, most of whose halvings add half as many again
+    size_t scratch_size = ring.size() * sizeof(int32_t);
+    for (int h : heights) scratch_size = std::max(scratch_size, scratch_bytes(1.4 * ((double)cut(h).size() + 1), h));
+    int32_t* d = static_cast<int32_t*>(ctx->aux2.get(scratch_size));
     KPMX_REQUIRE(chain_sample(m, heights.data(), (int)heights.size(), cap, d, ctx->stream) == 0, "no LDS for a chain plan");
     KPMX_HIP(hipGetLastError());
     KPMX_HIP(hipMemcpyAsync(ring.data(), d, ring.size() * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -1103,13 +1110,11 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     P.tile_rows = rows;
     P.ext_stride = std::min(CHAIN_MAX_HALO, cap - rows);
     std::vector<int32_t> begin = cut(rows);
-    auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
     std::vector<int> most(ST, 0);
     for (int pass = 0;; ++pass) {
         P.ntiles = (int64_t)begin.size() - 1;
         const size_t ring_size = (size_t)P.ntiles * ST;
-        char* w = static_cast<char*>(ctx->aux2.get(pad(begin.size() * sizeof(int32_t)) + pad(ring_size * sizeof(int32_t)) +
-                                                   (size_t)P.ntiles * P.ext_stride * sizeof(int32_t)));
+        char* w = static_cast<char*>(ctx->aux2.get(scratch_bytes((double)P.ntiles, rows)));
         P.tile_begin = reinterpret_cast<int32_t*>(w);
         P.ring = reinterpret_cast<int32_t*>(w + pad(begin.size() * sizeof(int32_t)));
         P.ext = reinterpret_cast<int32_t*>(w + pad(begin.size() * sizeof(int32_t)) + pad(ring_size * sizeof(int32_t)));
@@ -3488,10 +3493,9 @@ int kpmx_batch_starters(kpmx_batch* b, int64_t num_vectors, const void* r0) {
             dev_free(b->r0);
             dev_free(b->w0);
             dev_free(b->w1);
-            dev_free(b->w2);
-            dev_free(b->w3);
+            b->chain_work.release();
             dev_free(b->sums);
-            b->r0 = b->w0 = b->w1 = b->w2 = b->w3 = nullptr;
+            b->r0 = b->w0 = b->w1 = nullptr;
             b->sums = nullptr;
             b->sums_steps = 0;
             b->drop_graph();
@@ -3592,6 +3596,10 @@ void batch_enqueue(kpmx_batch* b, int64_t steps, int64_t t = 0) {
 }  // namespace
 
 namespace {
+size_t batch_block_bytes(const kpmx_batch* b) {
+    return ((size_t)b->n_pad * b->vw * scalar_bytes(b->scalar) + 255) / 256 * 256;
+}
+
 int batch_chain_cols(const kpmx_batch* b) { return std::min(pick_vw(b->tile_cols), chain_max_cols(b->scalar)); }
 
 ChainMatrix batch_chain_matrix(const kpmx_batch* b) {
@@ -3620,14 +3628,14 @@ ChainMatrix batch_chain_matrix(const kpmx_batch* b) {
 }
 
 // The plan of the batch's chained form with its work vectors and partial sums, or null: short runs
-// (as for one matrix), pinned partitions, halos that do not fit and memory that is not there keep the
+// (batch_chain_pays), pinned partitions, halos that do not fit and memory that is not there keep the
 // walkers.  A tile lies in one system, so its sums belong to that system.
 const ChainHolder* batch_chain(kpmx_batch* b, int64_t steps) {
     kpmx_ctx* ctx = b->ctx;
     const size_t sb = scalar_bytes(b->scalar);
     const double sweep = 3.0 * (double)b->n_pad * b->vw * sb / 5.6e6;
-    if (!b->chain_on || std::max(10.0, sweep) * steps * b->ntiles < 400) return nullptr;
     const int cols = batch_chain_cols(b);
+    if (!b->chain_on || !batch_chain_pays(b->n_pad, cols, std::max(10.0, sweep), steps * b->ntiles)) return nullptr;
     ChainHolder* H = nullptr;
     for (auto& c : b->chains)
         if (c->cols == cols && c->coded == b->use_coded) H = c.get();
@@ -3669,30 +3677,22 @@ const ChainHolder* batch_chain(kpmx_batch* b, int64_t steps) {
             }
         }
         if (!H->data) return nullptr;
-        const size_t blk = (size_t)b->n_pad * b->vw * sb;
-        if (!b->w2) b->w2 = dev_alloc(blk);
-        if (!b->w3) b->w3 = dev_alloc(blk);
         const size_t step_bytes = (size_t)H->plan.ntiles * chain_partial_width(b->scalar, cols) * sizeof(double);
-        const size_t need = std::min(std::max(CHAIN_PARTIALS, H->plan.steps * step_bytes), (steps + H->plan.steps) * step_bytes);
-        if (need > b->chain_partials_bytes) {
+        const size_t need = 2 * batch_block_bytes(b) +
+                            std::min(std::max(CHAIN_PARTIALS, H->plan.steps * step_bytes), (steps + H->plan.steps) * step_bytes);
+        if (need > b->chain_work.bytes) {
             KPMX_HIP(hipStreamSynchronize(ctx->stream));
             b->drop_graph();
-            dev_free(b->chain_partials);
-            b->chain_partials = nullptr;
-            b->chain_partials_bytes = 0;
-            b->chain_partials = static_cast<double*>(dev_alloc(need));
-            b->chain_partials_bytes = need;
+            b->chain_work.get(need);
         }
     } catch (const Error& e) {
         if (e.code != KPMX_ENOMEM) throw;
         // no memory for the plan or its vectors: what there is of them is given back
         KPMX_HIP(hipStreamSynchronize(ctx->stream));
         b->drop_graph();
-        for (void* p : {(void*)H->data, b->w2, b->w3, (void*)b->chain_partials}) dev_free(p);
+        dev_free(H->data);
         H->data = nullptr;
-        b->w2 = b->w3 = nullptr;
-        b->chain_partials = nullptr;
-        b->chain_partials_bytes = 0;
+        b->chain_work.release();
         ctx->aux2.release();
         return nullptr;
     }
@@ -3705,7 +3705,10 @@ void batch_enqueue_chain(kpmx_batch* b, const ChainHolder& H, int64_t steps, int
     const size_t sb = scalar_bytes(b->scalar);
     const char* r0 = static_cast<const char*>(b->r0) + (size_t)t * b->n_pad * b->vw * sb;
     double* sums = b->sums + (size_t)t * steps * b->num_sys * 4 * b->vw;
-    const ChainBuffers B{{{b->w0, b->w1}, {b->w2, b->w3}}, b->chain_partials, b->chain_partials_bytes};
+    const size_t blk = batch_block_bytes(b);
+    char* work = static_cast<char*>(b->chain_work.ptr);
+    const ChainBuffers B{{{b->w0, b->w1}, {work, work + blk}}, reinterpret_cast<double*>(work + 2 * blk),
+                         b->chain_work.bytes - 2 * blk};
     run_chain(ctx, batch_chain_matrix(b), H.plan, H.cols, r0, b->vw, std::min<int64_t>(b->tile_cols, b->nvec - t * b->tile_cols),
               steps, H.systems, b->num_sys, sums, B);
 }

@@ -282,5 +282,19 @@ def kubo_panels_take_the_chain_where_it_pays(rt):
         ctx.close()
 
 
+@check
+def short_batch_runs_keep_the_walkers(rt):
+    """A batch builds a plan for runs long enough to pay for it in their first pass, by its rows and vectors"""
+    import abi
+    for systems, size, nvec, forms in ((2, 500000, 8, {40: 0, 60: 1}), (2, 500000, 4, {60: 0, 100: 1}), (10, 2000, 4, {60: 0, 80: 1})):
+        ctx = abi.Ctx(0)
+        b = abi.Batch(ctx, [chain(size)] * systems)
+        b.starters(block(size * systems, nvec))
+        for M, form in forms.items():
+            run = rt.of(b.run, M, False)
+            assert bool(chained(run)) == bool(form), (size, nvec, M, run)
+        ctx.close()
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
