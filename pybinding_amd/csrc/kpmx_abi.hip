@@ -1518,14 +1518,26 @@ size_t backward_pair(const kpmx_tape* T) {  // bytes of two work vectors of a co
 // chose; long rows; small runs, as in use_chain; tapes that keep every vector, in fp32, where a rebuilt
 // vector would differ in the last bits from the kept one, or of several column groups, which would each
 // fetch the whole rows of the kept blocks in every launch: 1 M sites, 16 fp64 vectors, 1024 moments
-// 107 ms against 101 ms with single steps).
+// 107 ms against 101 ms with single steps; checkpoints so close that launches, which end at them, are
+// too short).  The launches between two checkpoints do C steps, the first of them one: on average they
+// have to do 1.5 steps for one column group and 2 for two, since a launch loads and stores its tiles
+// whatever it does in between; for more, 3.1 where a block exceeds 2^25 bytes and 3.9 below, where a single
+// step is bound by its launch (129 steps, single and chained, in ms: 305 k sites, 16 fp64 vectors, C = 2
+// 6.3 and 14.5, C = 5 7.0 and 7.9, C = 16 7.5 and 6.3; 61 k sites C = 6 1.7 and 2.2, C = 16 1.71 and 1.71, C = 64 1.7
+// and 1.5; 305 k sites, 16 fp32 vectors, C = 3 5.4 and 5.5, C = 4 5.5 and 4.8; 61 k sites, one fp64 vector,
+// C = 2 1.0 and 1.1, C = 3 1.1 and 0.9).
 const ChainPlan* backward_chain(const kpmx_tape* T) {
     const kpmx_mat* h2 = T->h2;
     kpmx_ctx* ctx = h2->ctx;
     if (!ctx->chain[h2->scalar] || (h2->chain_tuned_off >> log2i(T->vw) & 1) || ctx->adjoint_variant >= 0) return nullptr;
     if (T->store_all && (h2->scalar == KPMX_F32 || T->vw > chain_adjoint_cols(h2->scalar, T->vw))) return nullptr;
     if (!chain_pays(h2->rows, single_step_us(h2->rows, 2 * T->vw, scalar_bytes(h2->scalar)), T->S)) return nullptr;
-    return adjoint_chain_plan(h2, T->vw);
+    const ChainPlan* P = adjoint_chain_plan(h2, T->vw);
+    if (!P || T->store_all) return P;
+    const int groups = T->vw / chain_adjoint_cols(h2->scalar, T->vw);
+    const double launches = 1.0 + std::ceil((double)(T->C - 1) / P->steps);  // from one checkpoint to the next
+    const double least = groups == 1 ? 1.5 : groups == 2 ? 2.0 : T->blk > (size_t)1 << 25 ? 3.1 : 3.9;
+    return (double)T->C < least * launches ? nullptr : P;
 }
 // Leaves lambda_1 in lam1 (a block like the starters) and the steps' gradient in grad (SELL order).
 // Column groups run one after the other on packed work vectors.  Between kept pairs, v_j is rebuilt from

@@ -296,5 +296,23 @@ def short_batch_runs_keep_the_walkers(rt):
         ctx.close()
 
 
+@check
+def close_checkpoints_keep_single_reverse_steps(rt):
+    """The backward pass leaves the chained form where its launches end at checkpoints after too few steps"""
+    import abi
+    n, M = 20000, 258
+    for dtype, nvec, forms in ((np.float64, 16, {2: 0, 4: 0, 6: 0, 16: 1, 64: 1}), (np.float32, 16, {2: 0, 3: 0, 4: 1, 64: 1}),
+                               (np.float64, 1, {2: 0, 3: 1, 64: 1}), (np.float32, 3, {2: 0, 3: 1, 64: 1})):
+        ctx = abi.Ctx(0)
+        mat, blk = ctx.mat(chain(n, dtype), fmt=1), ctx.block(block(n, nvec, dtype))
+        for interval, form in forms.items():
+            tape = abi.Tape(mat, blk, M, interval)
+            run = rt.of(tape.backward, np.ones(M))
+            single = sum(c for k, c in run.items() if k.startswith("k_adjoint") and "chain" not in k)
+            assert bool(run["k_chain_adjoint"]) == bool(form) and (single < 5) == bool(form), (dtype, nvec, interval, run)
+            tape.close()
+        ctx.close()
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))
