@@ -1150,7 +1150,13 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     while (steps > 1 && most[steps] < 0) --steps;
     if (steps < 2) return;
     int halo = 0;
-    for (int64_t t = 0; t < P.ntiles; ++t) halo = std::max(halo, ring[t * ST + steps] - ring[t * ST]);
+    double mean[ST] = {};
+    for (int64_t t = 0; t < P.ntiles; ++t) {
+        halo = std::max(halo, ring[t * ST + steps] - ring[t * ST]);
+        for (int j = 0; j <= steps; ++j) mean[j] += (double)ring[t * ST + j] / (double)P.ntiles;
+    }
+    // with the halos of all tiles, the halved ones and the steps that fit them
+    if (chain_cost(m, (double)n / (double)P.ntiles, mean, steps, row_bytes, ctx->num_cu) > single_us) return;
     const size_t ring_bytes = (size_t)P.ntiles * ST * sizeof(int32_t), begin_bytes = (size_t)(P.ntiles + 1) * sizeof(int32_t);
     P.steps = steps;
     P.width = m.width();

@@ -314,5 +314,22 @@ def close_checkpoints_keep_single_reverse_steps(rt):
         ctx.close()
 
 
+@check
+def plans_are_weighed_as_they_come_out(rt):
+    """A plan whose tiles were halved and left with fewer steps per launch than its samples promised is
+    taken only if it still promises to be faster than single steps (here: halos that grow by `growth` rows
+    a step in a fifth of the system, between the samples)"""
+    import abi
+    n, M = 1000000, 1026
+    h = chain(n)
+    for growth, steps in ((30, 12), (300, 4), (500, 1)):
+        rt.growth(30, 30)
+        rt.lib.host_runtime_region(n // 5, growth)
+        ctx = abi.Ctx(0)
+        form = abi.diagonal_form(ctx.mat(h, fmt=1), 1, M)
+        assert form[0] == steps, (growth, form)
+        ctx.close()
+
+
 if __name__ == "__main__":
     CHECKS[sys.argv[2]](Runtime(sys.argv[1]))

@@ -4,8 +4,8 @@
 // settable time.  Loaded with global symbols before libkpmx.so, whose HIP calls it then takes.
 //
 // Two kernels leave something, so that plans of the chained recurrence can be built: the rings of a tile
-// of r rows get r + growth * j local rows up to distance j (growths of sampled and of all tiles apart),
-// as far as these fit.
+// of r rows get r + growth * j local rows up to distance j (growths of sampled, of all and of the first
+// tiles apart), as far as these fit.
 #include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
 
@@ -24,7 +24,7 @@ size_t g_used = 0, g_limit = (size_t)8 << 30;
 std::vector<std::string> g_log, g_captured;
 std::vector<std::vector<std::string>> g_graphs;
 bool g_capturing = false;
-int g_captures = 0, g_sample_growth = 16, g_growth = 16;
+int g_captures = 0, g_sample_growth = 16, g_growth = 16, g_region = 0, g_region_growth = 0;
 double g_clock = 0;  // us
 std::map<std::string, double> g_cost;
 std::string g_text;
@@ -52,6 +52,11 @@ size_t host_runtime_used() { return g_used; }
 void host_runtime_growth(int sampled, int all) {
     g_sample_growth = sampled;
     g_growth = all;
+}
+// tiles that begin before `rows` have another growth among all tiles
+void host_runtime_region(int rows, int growth) {
+    g_region = rows;
+    g_region_growth = growth;
 }
 void host_runtime_cost(const char* kernel_prefix, double us) { g_cost[kernel_prefix] = us; }
 int host_runtime_captures() { return g_captures; }
@@ -114,7 +119,8 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, 
         const auto* begin = *static_cast<const int32_t* const*>(args[1]);
         auto* out = *static_cast<int32_t**>(args[4]);
         const int64_t halo = *static_cast<const int64_t*>(args[6]);
-        for (unsigned t = 0; t < grid.x; ++t) ring(out + t * RINGS, begin[t + 1] - begin[t], g_growth, (int)halo);
+        for (unsigned t = 0; t < grid.x; ++t)
+            ring(out + t * RINGS, begin[t + 1] - begin[t], begin[t] < g_region ? g_region_growth : g_growth, (int)halo);
     }
     return hipSuccess;
 }
