@@ -2032,14 +2032,16 @@ void build_coded_sell(kpmx_mat* m, const int32_t* indptr, const int32_t* indices
     std::vector<std::string> table;
     std::map<std::string, int> code_of;
     const std::string zero(sb, '\0');
+    int last = -1;  // of the value before: most entries repeat it
     auto code = [&](const char* p) -> int {
+        if (last >= 0 && std::memcmp(table[(size_t)last].data(), p, sb) == 0) return last;
         const std::string key(p, sb);
         auto it = code_of.find(key);
-        if (it != code_of.end()) return it->second;
+        if (it != code_of.end()) return last = it->second;
         if (table.size() >= 256) return -1;
         code_of[key] = (int)table.size();
         table.push_back(key);
-        return (int)table.size() - 1;
+        return last = (int)table.size() - 1;
     };
     const int zcode = code(zero.data());
     std::vector<char> diag((size_t)rows * sb, 0);
