@@ -415,28 +415,32 @@ def kubo_contraction(n1=724, n2=724, M=512, R=16):
 
 def ldos_light_cone(reps=3):
     """LDOS at the centre of a 1 M-site graphene flake (161.8 x 161.8 nm, fp64) through
-    kpm(model).calc_ldos at 0.05 eV broadening: with the reference's optimal_size light cone (each
-    step computes only the BFS slices reached so far) and with full sweeps.  Best of `reps`."""
+    kpm(model).calc_ldos at 0.05 eV broadening: in the default form (chained sweeps of the whole system
+    on the locality order), with the reference's optimal_size light cone on the BFS order (each step
+    computes only the BFS slices reached so far) and with full sweeps in single steps.  Best of `reps`."""
     import pybinding_amd as pb
     from pybinding_amd.repository import graphene
     model = pb.Model(graphene.monolayer(), pb.rectangle(161.8, 161.8), pb.force_double_precision())
     n = model.hamiltonian.shape[0]
     energy = np.linspace(-1, 1, 200)
     out = {"sites": n, "broadening": 0.05}
-    for opt in (True, False):
-        kpm = pb.kpm(model, energy_range=(-9, 9), silent=True, optimal_size=opt, interleaved=False)
-        kpm.calc_ldos(energy, broadening=0.05, position=[0, 0])   # BFS reorder and upload
+    for form, options in (("chained", {}), ("cone", {"site_order": "bfs"}),
+                          ("full", {"site_order": "bfs", "optimal_size": False, "interleaved": False})):
+        kpm = pb.kpm(model, energy_range=(-9, 9), silent=True, **options)
+        kpm.calc_ldos(energy, broadening=0.05, position=[0, 0])   # reorder and upload
         best = float("inf")
         for _ in range(reps):
             t0 = time.perf_counter()
             kpm.calc_ldos(energy, broadening=0.05, position=[0, 0])
             best = min(best, time.perf_counter() - t0)
         st = kpm.stats
-        out["cone_ms" if opt else "full_ms"] = best * 1000
-        out["cone_fraction_of_rows" if opt else "moments"] = (st.opt_vec / st.vec) if opt else st.num_moments
+        out[form + "_ms"] = best * 1000
+        out["moments"] = st.num_moments
+        if form == "cone":
+            out["cone_fraction_of_rows"] = st.opt_vec / st.vec
     out["speedup"] = out["full_ms"] / out["cone_ms"]
-    log("LDOS light cone: %d sites, %d moments: %.1f ms with the cone (%.2f of the rows), %.1f ms full sweeps"
-        % (n, out["moments"], out["cone_ms"], out["cone_fraction_of_rows"], out["full_ms"]))
+    log("LDOS: %d sites, %d moments: %.1f ms in the default form, %.1f ms with the cone (%.2f of the rows), %.1f ms "
+        "full sweeps" % (n, out["moments"], out["chained_ms"], out["cone_ms"], out["cone_fraction_of_rows"], out["full_ms"]))
     return out
 
 
