@@ -274,8 +274,9 @@ int kpmx_kubo_moments(const kpmx_mat* h2, const kpmx_mat* vl, const kpmx_mat* vr
  * vector pairs, the vectors in between recomputed by running the recurrence backwards
  * (v_{j-1} = H2 v_j - v_{j+1}) inside the adjoint steps, restarting from every stored pair; <= 0
  * keeps every vector (no recomputation).  Runs long enough for a plan use the chained form: launches of
- * several steps forward (checkpointed) and backward (rows of at most four entries; without checkpoints
- * only fp64 and at most four vectors), under the conditions of kpmx_moments_diagonal.
+ * several steps forward (checkpointed) and backward (rows of at most four entries, checkpoints far enough
+ * apart for them; without checkpoints only fp64 and at most four vectors), under the conditions of
+ * kpmx_moments_diagonal.
  * Real H2 (KPMX_F32 / KPMX_F64) uploaded with KPMX_FMT_SELL; at most 64 vectors.
  * mu (optional): host, num_vectors x num_moments, the forward moments. */
 int kpmx_adjoint_diagonal(const kpmx_mat* h2, const kpmx_block* r0, int64_t num_moments, const double* w,
@@ -300,12 +301,13 @@ int kpmx_tape_destroy(kpmx_tape* tape);
  *             to them).
  *   starters: num_vectors (1..64) starters per system, host, vector-major num_vectors x N.
  *   run:      all num_moments / 2 steps, in modes 0 and 1 in launches of several steps (the chained
- *             form of kpmx_moments_diagonal) unless a partition was set or the autotuner found single
- *             steps faster.  use_graph (the run mode): 0 one launch per step or chain of steps (and
- *             per-system reduction), 1 the whole step sequence captured in one HIP graph on the
- *             first run for this num_moments and replayed afterwards, 2 one persistent kernel
- *             launch for all steps (grid barriers between steps; the partition's workgroups must
- *             fit the resident grid, else KPMX_EINVAL; returns after the run has finished).
+ *             form of kpmx_moments_diagonal) where the run is long enough for its plan, unless a
+ *             partition was set or the autotuner found single steps faster.  use_graph (the run
+ *             mode): 0 one launch per step or chain of steps (and per-system reduction), 1 the whole
+ *             step sequence captured in one HIP graph on the first run for this num_moments and
+ *             these vectors and replayed afterwards, 2 one persistent kernel launch for all steps
+ *             (grid barriers between steps; the partition's workgroups must fit the resident grid,
+ *             else KPMX_EINVAL; returns after the run has finished).
  *   fetch:    mu: host, num_systems x num_vectors x num_moments (mu_0 halved). */
 int kpmx_batch_upload(kpmx_ctx* ctx, int scalar, int64_t num_systems, const int64_t* row_offsets, int64_t nnz,
                       const int32_t* indptr, const int32_t* indices, const void* values, kpmx_batch** out);

@@ -237,7 +237,6 @@ __device__ __forceinline__ P& at(P* p, unsigned i) {
     return *reinterpret_cast<P*>(reinterpret_cast<byte*>(p) + (size_t)(i * (unsigned)sizeof(P)));
 }
 
-// v plus v of another lane of the same row of 16 (DPP)
 // the sums of <w| on one element: conj(w) x (real, imaginary part), then conj(w) y
 template <class T>
 __device__ __forceinline__ void add_dots(T w, T y, T x, double* s) {
@@ -258,6 +257,7 @@ __device__ __forceinline__ double column_of(const dpair& e, int i) { return i ? 
 __device__ __forceinline__ float column_of(const fquad& e, int i) { return e.v[i]; }
 __device__ __forceinline__ cf32 column_of(const cpair& e, int i) { return e.v[i]; }
 
+// v plus v of another lane of the same row of 16 (DPP)
 template <int CTRL>
 __device__ __forceinline__ double dpp_add(double v) {
     union { double d; int i[2]; } a, b;
