@@ -1067,17 +1067,7 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     if (heights.empty()) return;
     constexpr int ST = CHAIN_MAX_STEPS + 1;
     std::vector<int32_t> ring(heights.size() * CHAIN_SAMPLES * ST);
-    auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
-    // first rows, ring counts and halo rows of `tiles` tiles of at most `h` rows
-    auto scratch_bytes = [&](double tiles, int h) {
-        return pad((size_t)(tiles + 1) * sizeof(int32_t)) + pad((size_t)tiles * ST * sizeof(int32_t)) +
-               (size_t)tiles * std::min(CHAIN_MAX_HALO, cap - h) * sizeof(int32_t);
-    };
-    // scratch of the samples and, in the same allocation (growing it later took 0.2 ms on 1 M rows), of any
-    // choice of tiles, most of whose halvings add half as many again
-    size_t scratch_size = ring.size() * sizeof(int32_t);
-    for (int h : heights) scratch_size = std::max(scratch_size, scratch_bytes(1.4 * ((double)cut(h).size() + 1), h));
-    int32_t* d = static_cast<int32_t*>(ctx->aux2.get(scratch_size));
+    int32_t* d = static_cast<int32_t*>(ctx->aux2.get(ring.size() * sizeof(int32_t)));
     KPMX_REQUIRE(chain_sample(m, heights.data(), (int)heights.size(), cap, d, ctx->stream) == 0, "no LDS for a chain plan");
     KPMX_HIP(hipGetLastError());
     KPMX_HIP(hipMemcpyAsync(ring.data(), d, ring.size() * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -1110,11 +1100,17 @@ void build_chain(kpmx_ctx* ctx, const ChainMatrix& m, int cols, double single_us
     P.tile_rows = rows;
     P.ext_stride = std::min(CHAIN_MAX_HALO, cap - rows);
     std::vector<int32_t> begin = cut(rows);
+    auto pad = [](size_t b) { return (b + 255) / 256 * 256; };
+    // first rows, ring counts and halo rows of `tiles` tiles
+    auto scratch_bytes = [&](size_t tiles) {
+        return pad((tiles + 1) * sizeof(int32_t)) + pad(tiles * ST * sizeof(int32_t)) + tiles * P.ext_stride * sizeof(int32_t);
+    };
+    ctx->aux2.get(scratch_bytes(2 * begin.size()));  // room for halved tiles (growing it took 0.1 ms on 1 M rows)
     std::vector<int> most(ST, 0);
     for (int pass = 0;; ++pass) {
         P.ntiles = (int64_t)begin.size() - 1;
         const size_t ring_size = (size_t)P.ntiles * ST;
-        char* w = static_cast<char*>(ctx->aux2.get(scratch_bytes((double)P.ntiles, rows)));
+        char* w = static_cast<char*>(ctx->aux2.get(scratch_bytes((size_t)P.ntiles)));
         P.tile_begin = reinterpret_cast<int32_t*>(w);
         P.ring = reinterpret_cast<int32_t*>(w + pad(begin.size() * sizeof(int32_t)));
         P.ext = reinterpret_cast<int32_t*>(w + pad(begin.size() * sizeof(int32_t)) + pad(ring_size * sizeof(int32_t)));
