@@ -262,8 +262,10 @@ public:
     }
 
     // Whether diagonal recurrences of `num_vectors` vectors without a light cone run several steps per
-    // launch on `oh`; a BFS-ordered matrix gets the locality order for its tiles.
-    bool several_steps(OptimizedHamiltonian<T> const& oh, int format, idx_t num_vectors, idx_t num_moments) {
+    // launch on `oh`; a BFS-ordered matrix gets the locality order for its tiles.  Out of line: inlined
+    // into its callers it shifts the starters' and curves' loops of the module (stochastic DOS, 32 k sites,
+    // 16 vectors: 1.77 ms against 1.71 ms, the same instructions on other addresses).
+    [[gnu::noinline]] bool several_steps(OptimizedHamiltonian<T> const& oh, int format, idx_t num_vectors, idx_t num_moments) {
         kpmx_mat* h2 = matrix(oh, format);
         set_cone(h2, {});
         if (!oh.used_locality && ordered_ != oh.version) {
